@@ -289,11 +289,13 @@ def run_search(vs, NN, workload, args, ctx, full=False):
     roof = roofline("mfma", 2.0 * nq * n * d, scan_s, ctx["peaks"], "scan", nscan, traffic, tsrc,
                     peak_div=1 if bf16 else 3,
                     extra={"scan_kinds": {f: idx.prof_get(f)[0] for f in
-                                          ("shared", "gemm", "streamed")
+                                          ("shared", "gemm", "streamed", "direct")
                                           if idx.prof_get(f)[0]},
                            "merge_avg_ms": round(merge_s * 1e3, 4),
                            "prepass_ms_per_step": round(pre_ms / args.steps, 4) if npre else None,
-                           "exact_fallback_queries": idx.prof_get("exact_fallback")[0]})
+                           # (a direct search's queries are counted with the fallback's)
+                           "exact_fallback_queries": idx.prof_get("exact_fallback")[0]
+                           - nq * idx.prof_get("direct")[0]})
     out = {"metric": METRIC, "value": round(nq * args.steps / wall, 1), "unit": "queries/s",
            "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
            "ms_per_step": round(wall / args.steps * 1e3, 3), "higher_is_better": True,

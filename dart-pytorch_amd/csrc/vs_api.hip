@@ -163,6 +163,8 @@ int64_t next_pow2(int64_t v) {
     return p;
 }
 
+constexpr size_t kCtlBytes = 256;  // control words at the head of an index's pinned block
+
 int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
 }  // namespace
@@ -193,6 +195,8 @@ struct VsOptions {
     int merge_g = 0;       // merge: workgroups per query (0: by batch size; 1: one; 2..64: split)
     int guess_div_log2 = 0;  // large batches: the estimate's sample is 1/2^this of the rows (0: 5)
     int kmin_init = 1;       // k-means: start the assign scan's running minima from the last step
+    int direct = -1;         // searches straight on the exact keys: -1 rule, 0 off, 1 wherever the
+                             // keys fit
     int assign_order = 1;    // k-means: the assign scan walks the points grouped by the last
                              // step's clusters
 };
@@ -223,6 +227,10 @@ struct vs_index {
     // k-means: pinned copies of the distances, assignments and new centroids
     HostBuf km_hbest, km_hassign, km_hcen, km_hfb;
     HostBuf rstage;  // reconstruct: pinned staging of stored rows
+    DevBuf ex_qd, ex_keys, ex_part;  // exact keys: fp64 queries, keys, segments' best
+    // pinned: control words (kCtlBytes), then a small host search's queries and
+    // results
+    HostBuf hio;
     hipStream_t st_copy = nullptr;  // k-means: reads results back beside the update
     // k-means: km_order holds the last step's points grouped by cluster, for
     // these rows (version) and this many points
@@ -911,6 +919,12 @@ int take_lists(vs_index *x, Arena &A, size_t elems, size_t lists, ListBufs *L) {
 // A plan warms up badly when it makes many lists per query over many rows.
 // Rows per sampled row of the small-batch threshold pre-pass.
 constexpr int kPrepassDiv = 1024;
+// Largest nq * n * d of a search on the exact keys.  They take about 40 us
+// plus 1 us per 8.5e6 products, the selection 110 to 160 us on such inputs
+// before its scan grows (fp32 rows, k = 10: 10k x 384, 100 queries: 139 us
+// against 88; 50k x 384, 32 queries, 6e8 products: 179 against 144; 50k x 768,
+// 32 queries, 1.2e9: 204 against 220).
+constexpr double kDirectMacs = 5e8;
 
 bool needs_seed(const vs_index *x, const vs::ScanPlan &plan) {
     return plan.kind == 0 && plan.nsplit * plan.lw >= 512 && x->ntotal >= (1 << 18);
@@ -1088,70 +1102,132 @@ void topk_error_model(const vs_index *x, int planes, vs::TopkCheck *chk) {
 int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t nq, int64_t k,
                   float *D, int32_t *I, bool safe = false, size_t list_budget = 0);
 
-// Exact top-k of nq fp32 query rows (device, [nq][d]) without the MFMA
-// selection: per-(query, split) lists of the kk best exact keys, then the
-// merge (k <= kMaxFusedK), or a per-query sort of every row's key (larger
-// k; not in a fixed arena).
+// Exact top-k of nq query rows (device or pinned host memory, `stride`
+// elements apart) from a matrix of exact keys (vs_exact.hip), in chunks of
+// queries whose keys take at most 256 MiB (a kept buffer; over more than
+// 2^25 rows a call-local one of up to 1 GiB).  hflags (host-visible, or null:
+// the queries are known to be finite) receives the queries' flags; the call
+// must then be one chunk (direct_search's rule sees to it), and D and I stay
+// as they are if any query is not finite.
+int exact_topk(vs_index *x, Arena &A, const void *q, int q_dtype, int64_t stride, int64_t nq,
+               int64_t k, float *D, int32_t *I, uint32_t *hflags) {
+    const int64_t n = x->ntotal, ldd = vs::exact_ldd(x->d);
+    const bool select = vs::select_keys_cap(k) > 0 &&
+                        (size_t)vs::select_keys_cap(k) * 8 + 8192 + 1024 <= x->lds_max;
+    const int64_t most = n > (1 << 25) ? (int64_t)1 << 27 : (int64_t)1 << 25;  // keys at a time
+    const int64_t qc = std::min<int64_t>({nq, std::max<int64_t>(1, most / n),
+                                          std::max<int64_t>(1, ((int64_t)1 << 24) / ldd)});
+    if (hflags && qc < nq) return set_err(VS_ERR_HIP, "internal: direct search in chunks");
+    const int nseg = select ? vs::select_keys_segments(qc, n, k, x->num_cu) : 1;
+    size_t tmp_bytes = 0;
+    if (!select)
+        VS_HIP(vs::sort_topk_keys(nullptr, n, k, x->metric, nullptr, nullptr, nullptr, nullptr,
+                                  tmp_bytes, x->st),
+               "sort size");
+    const size_t kbytes = (size_t)(select ? qc : qc + 1) * n * 8;
+    void *p_qd, *p_keys, *p_part = nullptr, *p_rf = nullptr, *p_tmp = nullptr;
+    VS_TAKE(A.get(x->ex_qd, (size_t)qc * ldd * 8, &p_qd, "query rows"));
+    if (kbytes <= (size_t)1 << 28) VS_TAKE(A.get(x->ex_keys, kbytes, &p_keys, "keys"));
+    else VS_TAKE(A.tmp(kbytes, &p_keys, "keys"));
+    if (nseg > 1) VS_TAKE(A.get(x->ex_part, (size_t)qc * nseg * k * 8, &p_part, "segment keys"));
+    if (hflags) VS_TAKE(A.get(x->flags, (size_t)nq * 4, &p_rf, "query flags"));
+    if (!select) VS_TAKE(A.tmp(tmp_bytes + 256, &p_tmp, "sort scratch"));
+    double *qd = (double *)p_qd;
+    uint64_t *keys = (uint64_t *)p_keys;
+    const int64_t es = q_dtype == VS_DTYPE_BF16 ? 2 : 4;
+    for (int64_t q0 = 0; q0 < nq; q0 += qc) {
+        const int64_t m = std::min(qc, nq - q0);
+        VS_HIP(vs::launch_exact_queries((const char *)q + q0 * stride * es, q_dtype, stride, m,
+                                        x->d, qd, (uint32_t *)p_rf, x->st),
+               "query rows");
+        {
+            ProfScope ps(x, "scan");
+            VS_HIP(vs::launch_exact_tile(x->xb, x->storage, x->ld, x->d, x->metric, qd, m, n, keys,
+                                         n, x->st),
+                   "exact keys");
+        }
+        ProfScope ps(x, "merge");
+        if (select) {
+            VS_HIP(vs::launch_select_keys(keys, m, n, n, k, x->metric, nseg, (uint64_t *)p_part,
+                                          D + q0 * k, I + q0 * k, (const uint32_t *)p_rf, nq,
+                                          hflags, x->st),
+                   "key selection");
+            continue;
+        }
+        for (int64_t qi = 0; qi < m; ++qi)
+            VS_HIP(vs::sort_topk_keys(keys + qi * n, n, k, x->metric, D + (q0 + qi) * k,
+                                      I + (q0 + qi) * k, keys + qc * n, p_tmp, tmp_bytes, x->st),
+                   "exact sort");
+    }
+    return VS_OK;
+}
+
+// Whether a search goes straight to the exact keys: no selection to prove, no
+// thresholds to seed, three launches.
+bool direct_search(const vs_index *x, int64_t nq, int64_t k) {
+    const VsOptions &o = x->opt;
+    const int64_t n = x->ntotal;
+    if (o.direct == 0 || n < 1 || nq > ((int64_t)1 << 22) / vs::exact_ldd(x->d)) return false;
+    if (nq > ((int64_t)1 << 25) / n || !vs::select_keys_cap(k) ||
+        (size_t)vs::select_keys_cap(k) * 8 + 8192 + 1024 > x->lds_max)
+        return false;
+    if (o.direct > 0) return true;
+    // an option that forces a scan leaves small inputs to that scan
+    if (o.gemm >= 0 || o.share >= 0 || o.gemm_min_nq || o.gemm_wq || o.gemm_qb || o.gemm_kc ||
+        o.gemm4 || o.scan_kkw || o.scan_nw8)
+        return false;
+    if (k > 409) return true;  // (the fused selection's lists do not hold k)
+    return n < (1 << 18) && (double)nq * (double)n * (double)x->d <= kDirectMacs;
+}
+
+// Exact top-k of nq finite fp32 query rows (device, [nq][d]) without the MFMA
+// selection.  In a fixed arena, whose scratch does not hold a key matrix:
+// per-(query, split) lists of the best exact keys, then the merge (k <= 409).
 int exact_search(vs_index *x, Arena &A, const float *qf, int64_t nq, int64_t k, float *D,
                  int32_t *I) {
     if (nq <= 0) return VS_OK;
-    const int64_t kk = std::max<int64_t>(8, next_pow2(k + std::max<int64_t>(4, k / 4)));
-    if (kk <= 512) {
-        // splits: a few workgroups per CU over all queries, >= 1024 rows each
-        const int64_t target = (int64_t)x->num_cu * 4;
-        int64_t ns = std::max<int64_t>(1, (target + nq - 1) / nq);
-        ns = std::min<int64_t>(ns, std::max<int64_t>(1, x->ntotal / 1024));
-        if (A.fixed())  // the lists stay within 16 MiB
-            ns = std::max<int64_t>(1, std::min<int64_t>(ns, (int64_t)(16 << 20) / (nq * kk * 8)));
-        const int64_t rps = round_up((x->ntotal + ns - 1) / ns, 256);
-        ns = (x->ntotal + rps - 1) / rps;
-        void *pv, *pi;
-        VS_TAKE(A.tmp((size_t)nq * ns * kk * 4, &pv, "exact lists"));
-        VS_TAKE(A.tmp((size_t)nq * ns * kk * 4, &pi, "exact lists"));
-        VS_HIP(vs::launch_exact_lists(x->xb, x->storage, x->ld, x->d, x->metric, qf, nq, x->ntotal,
-                                      (int)kk, ns, rps, (float *)pv, (int32_t *)pi, x->st),
-               "exact lists");
-        vs::PreparedQueries pq;
-        pq.qf = (float *)qf;
-        pq.nq = nq;
-        pq.nq_pad = nq;
-        vs::ScanPlan plan;
-        plan.kind = 0;
-        plan.bn = 1;
-        plan.lw = 1;
-        plan.kk = (int)kk;
-        plan.kk_final = (int)kk;
-        plan.cap = (int)kk;
-        plan.nqblk = nq;
-        plan.nsplit = ns;
-        void *pf;
-        VS_TAKE(A.get(x->flags, sizeof(uint32_t), &pf, "flags buffer"));
-        VS_HIP(vs::launch_fill32(pf, 1, 0u, x->st), "clearing flags");
-        VS_HIP(vs::launch_merge_refine(x->xb, x->storage, x->ld, x->d, x->metric, pq, plan,
-                                       (float *)pv, (int32_t *)pi, nullptr, nullptr, nullptr,
-                                       nullptr, k, D, I, x->ntotal, (uint32_t *)pf, 0, nullptr,
-                                       nullptr, x->st),
-               "exact merge");
+    if (!A.fixed()) {
         if (!x->prof_fixed) x->prof["exact_queries"].launches += nq;
-        return VS_OK;
+        return exact_topk(x, A, qf, VS_DTYPE_F32, x->d, nq, k, D, I, nullptr);
     }
-    if (A.fixed())
+    const int64_t kk = std::max<int64_t>(8, next_pow2(k + std::max<int64_t>(4, k / 4)));
+    if (kk > 512)
         return set_err(VS_ERR_UNSUPPORTED, "k=%lld needs the sorting path, which allocates",
                        (long long)k);
-    // one query chunk of keys within 1 GiB, plus the sort's output and scratch
-    const int64_t n = x->ntotal;
-    const int64_t qchunk = std::max<int64_t>(1, std::min<int64_t>(nq, (int64_t)(1 << 27) / n));
-    size_t tmp_bytes = 0;
-    VS_HIP(vs::exact_sort_topk(x->xb, x->storage, x->ld, x->d, x->metric, qf, nq, n, k, D, I,
-                               nullptr, qchunk, nullptr, tmp_bytes, x->st),
-           "sort size");
-    void *keys, *tmp;
-    VS_TAKE(A.tmp((size_t)(qchunk + 1) * n * 8, &keys, "sort keys"));
-    VS_TAKE(A.tmp(tmp_bytes + 256, &tmp, "sort scratch"));
-    VS_HIP(vs::exact_sort_topk(x->xb, x->storage, x->ld, x->d, x->metric, qf, nq, n, k, D, I,
-                               (uint64_t *)keys, qchunk, tmp, tmp_bytes, x->st),
-           "exact sort");
-    if (!x->prof_fixed) x->prof["exact_sort_queries"].launches += nq;
+    // splits: a few workgroups per CU over all queries, >= 1024 rows each,
+    // lists within 16 MiB
+    const int64_t target = (int64_t)x->num_cu * 4;
+    int64_t ns = std::max<int64_t>(1, (target + nq - 1) / nq);
+    ns = std::min<int64_t>(ns, std::max<int64_t>(1, x->ntotal / 1024));
+    ns = std::max<int64_t>(1, std::min<int64_t>(ns, (int64_t)(16 << 20) / (nq * kk * 8)));
+    const int64_t rps = round_up((x->ntotal + ns - 1) / ns, 256);
+    ns = (x->ntotal + rps - 1) / rps;
+    void *pv, *pi;
+    VS_TAKE(A.tmp((size_t)nq * ns * kk * 4, &pv, "exact lists"));
+    VS_TAKE(A.tmp((size_t)nq * ns * kk * 4, &pi, "exact lists"));
+    VS_HIP(vs::launch_exact_lists(x->xb, x->storage, x->ld, x->d, x->metric, qf, nq, x->ntotal,
+                                  (int)kk, ns, rps, (float *)pv, (int32_t *)pi, x->st),
+           "exact lists");
+    vs::PreparedQueries pq;
+    pq.qf = (float *)qf;
+    pq.nq = nq;
+    pq.nq_pad = nq;
+    vs::ScanPlan plan;
+    plan.kind = 0;
+    plan.bn = 1;
+    plan.lw = 1;
+    plan.kk = (int)kk;
+    plan.kk_final = (int)kk;
+    plan.cap = (int)kk;
+    plan.nqblk = nq;
+    plan.nsplit = ns;
+    void *pf;
+    VS_TAKE(A.get(x->flags, sizeof(uint32_t), &pf, "flags buffer"));
+    VS_HIP(vs::launch_fill32(pf, 1, 0u, x->st), "clearing flags");
+    VS_HIP(vs::launch_merge_refine(x->xb, x->storage, x->ld, x->d, x->metric, pq, plan,
+                                   (float *)pv, (int32_t *)pi, nullptr, nullptr, nullptr, nullptr,
+                                   k, D, I, x->ntotal, (uint32_t *)pf, 0, nullptr, nullptr, x->st),
+           "exact merge");
     return VS_OK;
 }
 
@@ -1189,6 +1265,7 @@ int research_listed(vs_index *x, Arena &A, const vs::PreparedQueries &pq, const 
 // the candidate lists (the streaming scan's split count adapts).
 int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t nq, int64_t k,
                   float *D, int32_t *I, bool safe, size_t list_budget) {
+    int rc0 = VS_OK;
     if (nq < 0 || k < 0) return set_err(VS_ERR_INVALID, "nq and k must be >= 0");
     if (nq == 0) return VS_OK;
     if (k == 0) {
@@ -1202,6 +1279,19 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
             D, I, m, x->metric == 0 ? __builtin_huge_valf() : -__builtin_huge_valf());
         VS_HIP(hipGetLastError(), "filling sentinels");
         VS_HIP(hipStreamSynchronize(x->st), "search");
+        return VS_OK;
+    }
+    if (!safe && !A.fixed() && direct_search(x, nq, k)) {
+        VS_HIP(x->hio.ensure(kCtlBytes), "control words");
+        uint32_t *hf = x->hio.as<uint32_t>();
+        *hf = 0;
+        if ((rc0 = exact_topk(x, A, q_dev, q_dtype, x->d, nq, k, D, I, hf))) return rc0;
+        // counted with the queries that the selection sent to the exact path
+        x->prof["exact_fallback"].launches += nq;
+        x->prof["direct"].launches++;
+        VS_HIP(hipStreamSynchronize(x->st), "search");
+        if (*(volatile uint32_t *)hf & vs::kFlagNonFinite)
+            return set_err(VS_ERR_NONFINITE, "queries contain NaN or infinity");
         return VS_OK;
     }
     const int64_t kk = std::max<int64_t>(8, next_pow2(k + std::max<int64_t>(4, k / 4)));
@@ -1283,9 +1373,14 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
                    "merge kernel");
         }
         if (!x->prof_fixed && plan.merge_g > 1) x->prof["split_merges"].launches++;
-        int32_t hc[4] = {0, 0, 0, 0};
-        VS_HIP(hipMemcpyAsync(hc, ctl, sizeof hc, hipMemcpyDeviceToHost, x->st), "merge flags");
+        int32_t hc[4] = {0, 0, 0, 0}, *ph = hc;
+        if (!A.fixed()) {  // (a fixed arena's call allocates no pinned memory either)
+            VS_HIP(x->hio.ensure(kCtlBytes), "control words");
+            ph = x->hio.as<int32_t>();
+        }
+        VS_HIP(hipMemcpyAsync(ph, ctl, sizeof hc, hipMemcpyDeviceToHost, x->st), "merge flags");
         VS_HIP(hipStreamSynchronize(x->st), "search");
+        if (ph != hc) memcpy(hc, ph, sizeof hc);
         if (attempt == 0 && spec && ((uint32_t)hc[3] & vs::kFlagNotBf16) &&
             !((uint32_t)hc[3] & vs::kFlagNonFinite)) {
             pq.planes = 2;  // (both planes were prepared)
@@ -1581,13 +1676,14 @@ void vs_index_destroy(vs_index *x) {
                       &x->km_offsets, &x->km_out, &x->km_iota, &x->lcnt,   &x->km_qp,
                       &x->km_qf,   &x->km_qnorm,  &x->km_cen16, &x->km_c16n, &x->xb16,
                       &x->xb16n,   &x->vx,        &x->ctl,      &x->km_shift, &x->km_init,
-                      &x->km_pkeys, &x->km_part};
+                      &x->km_pkeys, &x->km_part, &x->ex_qd,   &x->ex_keys, &x->ex_part};
     for (DevBuf *b : bufs) b->release();
     x->km_hbest.release();
     x->km_hassign.release();
     x->km_hcen.release();
     x->km_hfb.release();
     x->rstage.release();
+    x->hio.release();
     if (x->st_copy) {
         (void)hipStreamSynchronize(x->st_copy);
         (void)hipStreamDestroy(x->st_copy);
@@ -1819,20 +1915,44 @@ int vs_index_search(vs_index *x, const void *q, int q_dtype, int64_t nq, int64_t
     if (nq == 0) return VS_OK;
     if (k > 0 && (!q || !D || !I)) return set_err(VS_ERR_INVALID, "null query or output buffer");
     DeviceGuard g(x->device);
-    const size_t qbytes = (size_t)nq * x->d * (q_dtype == 1 ? 2 : 4);
-    VS_HIP(x->stage.ensure(qbytes), "query staging");
-    VS_HIP(hipMemcpyAsync(x->stage.p, q, qbytes, hipMemcpyHostToDevice, x->st), "uploading queries");
     Arena A;
-    if (k == 0) return search_device(x, A, x->stage.p, q_dtype, nq, k, nullptr, nullptr);
-    VS_HIP(x->outD.ensure((size_t)nq * k * 4), "result buffer");
-    VS_HIP(x->outI.ensure((size_t)nq * k * 4), "result buffer");
-    int rc = search_device(x, A, x->stage.p, q_dtype, nq, k, x->outD.as<float>(),
-                           x->outI.as<int32_t>());
+    if (k == 0) return search_device(x, A, q, q_dtype, nq, k, nullptr, nullptr);
+    // up to 1 MiB, queries and results go through pinned memory, which the
+    // copies need not stage and the last kernel writes by itself (a pageable
+    // copy costs about 10 us however small); a direct search's first kernel
+    // reads the queries from there too
+    constexpr size_t kPinned = (size_t)1 << 20;
+    const size_t qbytes = (size_t)nq * x->d * (q_dtype == 1 ? 2 : 4);
+    const size_t rbytes = (size_t)nq * k * 4;
+    const void *src = q;
+    const size_t hq = qbytes <= kPinned ? (size_t)round_up((int64_t)qbytes, 256) : 0;
+    const size_t hr = 2 * rbytes <= kPinned ? 2 * rbytes : 0;
+    VS_HIP(x->hio.ensure(kCtlBytes + hq + hr), "pinned queries and results");
+    if (hq) {
+        src = x->hio.as<char>() + kCtlBytes;
+        memcpy((void *)src, q, qbytes);
+    }
+    if (src == q || x->ntotal == 0 || !direct_search(x, nq, k)) {
+        VS_HIP(x->stage.ensure(qbytes), "query staging");
+        VS_HIP(hipMemcpyAsync(x->stage.p, src, qbytes, hipMemcpyHostToDevice, x->st),
+               "uploading queries");
+        src = x->stage.p;
+    }
+    if (hr) {
+        float *hD = (float *)(x->hio.as<char>() + kCtlBytes + hq);
+        int32_t *hI = (int32_t *)((char *)hD + rbytes);
+        if (int rc = search_device(x, A, src, q_dtype, nq, k, hD, hI)) return rc;
+        memcpy(D, hD, rbytes);
+        memcpy(I, hI, rbytes);
+        return VS_OK;
+    }
+    VS_HIP(x->outD.ensure(rbytes), "result buffer");
+    VS_HIP(x->outI.ensure(rbytes), "result buffer");
+    int rc = search_device(x, A, src, q_dtype, nq, k, x->outD.as<float>(), x->outI.as<int32_t>());
     if (rc) return rc;
-    VS_HIP(hipMemcpyAsync(D, x->outD.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, x->st),
+    VS_HIP(hipMemcpyAsync(D, x->outD.p, rbytes, hipMemcpyDeviceToHost, x->st),
            "reading distances");
-    VS_HIP(hipMemcpyAsync(I, x->outI.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, x->st),
-           "reading ids");
+    VS_HIP(hipMemcpyAsync(I, x->outI.p, rbytes, hipMemcpyDeviceToHost, x->st), "reading ids");
     VS_HIP(hipStreamSynchronize(x->st), "search");
     return VS_OK;
 }
@@ -2901,6 +3021,7 @@ int vs_index_set_option(vs_index *x, const char *name, int64_t value) {
         {"guess_div_log2", &VsOptions::guess_div_log2, 0, 10},
         {"kmin_init", &VsOptions::kmin_init, 0, 1},
         {"assign_order", &VsOptions::assign_order, 0, 1},
+        {"direct", &VsOptions::direct, -1, 1},
     };
     if (strcmp(name, "fail_alloc") == 0) {  // not a planner option: this thread's countdown
         if (value < 0) return set_err(VS_ERR_INVALID, "option fail_alloc: value %lld < 0", (long long)value);

@@ -195,15 +195,36 @@ hipError_t launch_scatter_rows(const void *src, const int32_t *list, int64_t m, 
                                void *dst, hipStream_t st);
 hipError_t launch_fill32(void *p, int64_t n, uint32_t v, hipStream_t st);
 
-// Exact top-k by sorting (any k): for nq queries (fp32 rows qf [nq][d]) the
-// fp64 score of every row, as keys (fp32 key code, id), sorted per query;
-// D / I [nq][k] receive the k first, sentinel-filled past n.  keys holds
-// qchunk * n + n words of 64 bits, tmp tmp_bytes (query with tmp == nullptr).
-hipError_t exact_sort_topk(const void *xb, int storage, int64_t ld, int64_t d, int metric,
-                           const float *qf, int64_t nq, int64_t n, int64_t k, float *D, int32_t *I,
-                           uint64_t *keys, int64_t qchunk, void *tmp, size_t &tmp_bytes,
-                           hipStream_t st);
-// The same for one query (fp32 row qf [d]) over the rows ids[0 .. m) (ids in
+// Exact top-k without the MFMA selection (vs_exact.hip).
+// Queries as fp64 rows qd [nq][exact_ldd(d)], zero past d; rowflags [nq]
+// (or null) receives kFlagNonFinite per query (such a row becomes zero).
+int64_t exact_ldd(int64_t d);
+hipError_t launch_exact_queries(const void *src, int src_dtype, int64_t stride, int64_t nq,
+                                int64_t d, double *qd, uint32_t *rowflags, hipStream_t st);
+// keys [nq][kstride]: per query and row r < n the 64-bit key (order-preserving
+// code of the fp32 score (L2) or its negative (IP), then r) of the fp64 score.
+hipError_t launch_exact_tile(const void *xb, int storage, int64_t ld, int64_t d, int metric,
+                             const double *qd, int64_t nq, int64_t n, uint64_t *keys,
+                             int64_t kstride, hipStream_t st);
+// D / I [nq][k] from the k smallest of each query's n keys (sentinels past n;
+// k <= kSelectMaxK).  nseg > 1 cuts a query's keys into segments, whose best
+// go through part [nq][nseg][k] (select_keys_segments gives the count).  With
+// rowflags (nflags words: every query of the call), nothing is written to D
+// and I if one is set; *hflags (host-visible) receives their union.
+constexpr int64_t kSelectMaxK = 8192;
+int select_keys_cap(int64_t k);  // LDS keys of a workgroup; 0: k is too large
+int select_keys_segments(int64_t nq, int64_t n, int64_t k, int num_cu);
+hipError_t launch_select_keys(const uint64_t *keys, int64_t nq, int64_t n, int64_t kstride,
+                              int64_t k, int metric, int nseg, uint64_t *part, float *D, int32_t *I,
+                              const uint32_t *rowflags, int64_t nflags, uint32_t *hflags,
+                              hipStream_t st);
+
+// D / I [k] of one query by sorting its n keys (k beyond kSelectMaxK), into
+// out [n]; sentinel-filled past n.  tmp_bytes of scratch (query with tmp ==
+// nullptr).
+hipError_t sort_topk_keys(const uint64_t *keys, int64_t n, int64_t k, int metric, float *D,
+                          int32_t *I, uint64_t *out, void *tmp, size_t &tmp_bytes, hipStream_t st);
+// The same for one fp32 query row qf [d] over the rows ids[0 .. m) (ids in
 // [0, ntotal), checked by the caller): keys holds 2 m words of 64 bits, tmp
 // tmp_bytes (query with tmp == nullptr); D / I [k], sentinel-filled past m.
 hipError_t exact_sort_topk_ids(const void *xb, int storage, int64_t ld, int64_t d, int metric,
