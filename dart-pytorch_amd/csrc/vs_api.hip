@@ -2,6 +2,7 @@
 // include/vs_hip.h): index lifecycle, planning, host<->device staging,
 // error reporting.  All device work of a handle runs on its own stream.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -64,13 +65,21 @@ struct DeviceGuard {
 // Per thread, like the error text.
 thread_local int64_t g_fail_alloc = 0;
 
-// Every device allocation of an index goes through here.
+bool release_idle_copies();  // below: frees row copies on the current device
+
+// Every device allocation of an index goes through here.  A full device
+// takes the row copies of indexes that no call is using back first.
 hipError_t dev_malloc(void **p, size_t bytes) {
     if (g_fail_alloc > 0 && --g_fail_alloc == 0) {
         *p = nullptr;
         return hipErrorOutOfMemory;
     }
-    return hipMalloc(p, bytes);
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && release_idle_copies()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
 }
 
 // Every pinned host allocation of an index goes through here.
@@ -245,10 +254,18 @@ struct vs_index {
     vs::PreparedQueries km_pq;
     uint32_t km_pflags = 0;
     uint64_t km_prep_version = ~0ull;
-    // bf16 copy of fp32 rows for the GEMM-tiled one-pass selection (range,
-    // self-join), kept while the rows are unchanged
-    DevBuf xb16, xb16n;
-    uint64_t xb16_version = ~0ull;
+    // bf16 copy of fp32 rows for the one-pass selection (search, range,
+    // self-join): rows [0, copy_n) of stride copy_ld, zero rows after them
+    DevBuf xb16;
+    int64_t copy_ld = 0, copy_n = 0, copy_cap = 0;
+    float copy_res = 0.f;  // largest |row - copied row| (an upper bound)
+    std::atomic_flag copy_busy = ATOMIC_FLAG_INIT;  // held by a call that reads the copy
+    // the rows that the current call's scans and planning read
+    struct {
+        const void *rows = nullptr;
+        int storage = 0;
+        int64_t ld = 0;
+    } sel;
     int64_t km_iota_n = -1;  // km_iota holds 0 .. km_iota_n - 1
     bool prof_on = false;
     bool prof_fixed = false;  // inside an allocation-free call: no profiling bookkeeping
@@ -256,11 +273,54 @@ struct vs_index {
     // largest stored row norm, for the version of the rows it was taken at
     float xmax_cache = 0.f;
     uint64_t xmax_version = ~0ull;
+    DevBuf fbl;   // top-k: list of the queries searched again
+    DevBuf qres;  // top-k: residual norms of the queries' first planes
     DevBuf vx, ctl;  // top-k: exact-path query list, control words
     std::vector<PendingEvent> pending;
 };
 
 namespace {
+
+// Indexes that hold a row copy.  A copy belongs to its handle's thread while
+// copy_busy is set (every call that reads it holds it until its GPU work is
+// done); otherwise any thread short of memory may free it under this lock.
+std::mutex g_copies_mu;
+std::vector<vs_index *> g_copies;
+
+void drop_copy(vs_index *x) {  // the caller holds g_copies_mu
+    x->xb16.release();
+    x->copy_n = x->copy_cap = 0;
+    g_copies.erase(std::remove(g_copies.begin(), g_copies.end(), x), g_copies.end());
+}
+
+bool release_idle_copies() {
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lk(g_copies_mu);
+    bool any = false;
+    const std::vector<vs_index *> all = g_copies;
+    for (vs_index *y : all) {
+        if (y->device != dev || y->copy_busy.test_and_set(std::memory_order_acquire)) continue;
+        drop_copy(y);
+        y->copy_busy.clear(std::memory_order_release);
+        any = true;
+    }
+    return any;
+}
+
+// Holds an index's row copy for one call.
+struct CopyHold {
+    vs_index *x;
+    bool mine;
+    explicit CopyHold(vs_index *x_) : x(x_) {
+        // (only a thread that frees copies can hold it meanwhile, briefly)
+        std::lock_guard<std::mutex> lk(g_copies_mu);
+        mine = !x->copy_busy.test_and_set(std::memory_order_acquire);
+    }
+    ~CopyHold() {
+        if (mine) x->copy_busy.clear(std::memory_order_release);
+    }
+};
 
 int64_t elem_size(int storage) { return storage == 1 ? 2 : 4; }
 
@@ -411,6 +471,7 @@ int widen_storage(vs_index *x) {
     x->cap = nc;
     x->ld = new_ld;
     x->storage = 0;
+    x->copy_n = 0;
     ++x->version;
     return VS_OK;
 }
@@ -491,10 +552,10 @@ bool plan_share(const vs_index *x, int64_t nq, int64_t nrows, int planes, int st
                 vs::ScanPlan *p, int64_t max_split, int lane = -1) {
     const int mode = x->opt.share;
     if (mode == 0 || (storage != 1 && storage != vs::kSelectCoarse) || planes != 1) return false;
-    if (!(x->ld == 128 || (x->ld == 256 && (mode > 0 || storage == vs::kSelectCoarse))))
+    if (!(x->sel.ld == 128 || (x->sel.ld == 256 && (mode > 0 || storage == vs::kSelectCoarse))))
         return false;
     if (nq < 256) return false;
-    const int nks = (int)(x->ld / 32), nqb = nks == 4 ? 4 : 2;
+    const int nks = (int)(x->sel.ld / 32), nqb = nks == 4 ? 4 : 2;
     // fp32 tiles: half the rows, the same staging registers
     const int rt = storage == 1 ? (nks == 4 ? 8 : 4) : 2;
     vs::ScanPlan sp = *p;
@@ -513,7 +574,7 @@ bool plan_share(const vs_index *x, int64_t nq, int64_t nrows, int planes, int st
     // Splits: the whole grid resident at once (or whole rounds of it), so the
     // query blocks of a split -- dealt to one XCD back to back -- walk its
     // rows together through that XCD's L2, and no round is left half empty.
-    const int bpc = std::max(1, vs::share_blocks_per_cu(storage, nks, p->bn, rt, x->ld, lds, 0));
+    const int bpc = std::max(1, vs::share_blocks_per_cu(storage, nks, p->bn, rt, x->sel.ld, lds, 0));
     const int64_t resident = (int64_t)std::max(1, x->num_cu) * bpc;
     const int64_t target = resident * 4;
     int64_t nsplit = std::max<int64_t>(1, target / p->nqblk);
@@ -535,7 +596,7 @@ bool plan_gemm(const vs_index *x, int64_t nq, int64_t nrows, int planes, int sto
     const VsOptions &o = x->opt;
     const int mode = o.gemm;
     if (mode == 0) return false;
-    if (mode < 0 && x->ld < 256) return false;
+    if (mode < 0 && x->sel.ld < 256) return false;
     if (nq < (o.gemm_min_nq > 0 ? o.gemm_min_nq : mode < 0 ? 512 : 256)) return false;
     struct Shape {
         int st, pb, wr, wq, rb, qb, kc;
@@ -551,7 +612,7 @@ bool plan_gemm(const vs_index *x, int64_t nq, int64_t nrows, int planes, int sto
     // groups of four 32-element K-chunks, one query plane
     static const Shape pipe4 = {1, 1, 2, 2, 4, 4, 32};
     p->g_pipe = 0;
-    if (o.gemm4 && storage == 1 && planes == 1 && x->ld % 128 == 0 && (!fwq || fwq == 2) &&
+    if (o.gemm4 && storage == 1 && planes == 1 && x->sel.ld % 128 == 0 && (!fwq || fwq == 2) &&
         (!fqb || fqb == 4) && (!fkc || fkc == 32)) {
         kk = p->kk;
         if (!kk_forced && kk < p->kk_final) kk = std::max(kk, p->kk_final / pipe4.wr);
@@ -568,7 +629,7 @@ bool plan_gemm(const vs_index *x, int64_t nq, int64_t nrows, int planes, int sto
         if (fwq && sh.wq != fwq) continue;
         if (fqb && sh.qb != fqb) continue;
         if (fkc && sh.kc != fkc) continue;
-        if (x->ld % sh.kc) continue;
+        if (x->sel.ld % sh.kc) continue;
         kk = p->kk;
         if (!kk_forced && kk < p->kk_final) kk = std::max(kk, p->kk_final / sh.wr);
         // a wave may append up to 32 * rb entries per query and row tile
@@ -597,7 +658,7 @@ bool plan_gemm(const vs_index *x, int64_t nq, int64_t nrows, int planes, int sto
     // query planes take <= 1.5 MiB, so that they stay in the XCD's 4 MiB L2
     // beside the rows; a chunk of the grid (group x split run, about one
     // XCD's resident workgroups) covers 32 / group splits
-    const int64_t qbytes = (int64_t)p->bn * x->ld * 2 * planes;
+    const int64_t qbytes = (int64_t)p->bn * x->sel.ld * 2 * planes;
     int64_t qg = 1;
     while (qg < 32 && 2 * qg * qbytes <= (int64_t)3 << 19) qg *= 2;
     p->tile_group = std::max<int64_t>(1, std::min<int64_t>(p->nqblk, qg));
@@ -661,10 +722,11 @@ int plan_scan_core(const vs_index *x, int64_t nq, int64_t nrows, int planes, int
     if (safe) kk = kk_final;
     p->kk_final = (int)kk_final;
     p->kk = (int)kk;
-    p->cap = (int)next_pow2(kk + 48);
+    // range: the cap is that of the waves' pair buffers
+    p->cap = range ? 256 : (int)next_pow2(kk + 48);
     // 16-row blocks per wave tile: one for short rows (d <= 128: measured
     // faster on 1M x 128, the epilogue dominates), two otherwise
-    p->tm = x->ld <= 128 && storage == 1 ? 1 : 2;
+    p->tm = x->sel.ld <= 128 && storage == 1 ? 1 : 2;
     p->kind = 0;
     if (!range && kkw <= 0 && !list_budget &&
         plan_share(x, nq, nrows, planes, storage, p, max_lists))
@@ -672,7 +734,7 @@ int plan_scan_core(const vs_index *x, int64_t nq, int64_t nrows, int planes, int
     // (a list limit shapes the split count of the row-shared and streaming
     // scans; the GEMM-tiled scan makes few lists per query anyway)
     if (!list_budget && plan_gemm(x, nq, nrows, planes, storage, kkw > 0 || safe, p)) return VS_OK;
-    const int nks = (int)(x->ld / 32);
+    const int nks = (int)(x->sel.ld / 32);
     const int cands[3] = {64, 32, 16};
     p->bn = 0;
     p->nks = 0;
@@ -680,7 +742,7 @@ int plan_scan_core(const vs_index *x, int64_t nq, int64_t nrows, int planes, int
         if (bn > 16 && round_up(nq, 16) < bn) continue;
         const bool qreg = storage == 1 && planes == 1 && (nks == 4 || nks == 8) &&
                           nks * (bn / 16) <= 16;
-        if (vs::scan_lds_bytes(bn, qreg ? 0 : planes, x->ld, p->cap, 4) <= x->lds_max) {
+        if (vs::scan_lds_bytes(bn, qreg ? 0 : planes, x->sel.ld, p->cap, 4) <= x->lds_max) {
             p->bn = bn;
             p->nks = qreg ? nks : 0;
             break;
@@ -696,10 +758,10 @@ int plan_scan_core(const vs_index *x, int64_t nq, int64_t nrows, int planes, int
     // 20M x 768 bf16, so off by default)
     p->lw = 4;
     if (storage == 1 && !p->nks && p->tm == 2 && x->opt.scan_nw8 &&
-        2 * vs::scan_lds_bytes(p->bn, planes, x->ld, p->cap, 4) > x->lds_max &&
-        vs::scan_lds_bytes(p->bn, planes, x->ld, p->cap, 8) <= x->lds_max)
+        2 * vs::scan_lds_bytes(p->bn, planes, x->sel.ld, p->cap, 4) > x->lds_max &&
+        vs::scan_lds_bytes(p->bn, planes, x->sel.ld, p->cap, 8) <= x->lds_max)
         p->lw = 8;
-    p->lds_bytes = vs::scan_lds_bytes(p->bn, p->nks ? 0 : planes, x->ld, p->cap, p->lw);
+    p->lds_bytes = vs::scan_lds_bytes(p->bn, p->nks ? 0 : planes, x->sel.ld, p->cap, p->lw);
     p->nqblk = (nq + p->bn - 1) / p->bn;
     const int64_t tile_rows = 16 * p->lw * p->tm;  // rows per block per round
     const int64_t target = (int64_t)x->num_cu * 4;
@@ -835,22 +897,29 @@ int scan_fits(const vs::ScanPlan &plan, const vs::PreparedQueries &pq) {
 // as the unit vector e_0, so that the search runs on finite values).  With
 // spec_one_plane, fp32 queries take the same path with one plane on trust
 // (both planes are written): the caller reads the flags with its results and
-// searches again with two planes if any query was not bf16-exact.
+// searches again with two planes if any query was not bf16-exact, or proves
+// its results with the queries' residuals (want_res).
+// The planes' stride is that of the rows the scans will read (x->sel).
 int prepare_queries(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t stride,
                     int64_t nq, vs::PreparedQueries *pq, uint32_t *flags_out, DevBuf &qp,
                     DevBuf &qf, DevBuf &qnorm, uint32_t *defer_flags = nullptr,
-                    bool spec_one_plane = false) {
+                    bool spec_one_plane = false, bool want_res = false) {
     pq->nq = nq;
     pq->nq_pad = query_pad(nq);
     void *p_qp, *p_qf, *p_qn, *p_fl;
-    VS_TAKE(A.get(qp, (size_t)pq->nq_pad * 2 * x->ld * 2, &p_qp, "query planes"));
+    VS_TAKE(A.get(qp, (size_t)pq->nq_pad * 2 * x->sel.ld * 2, &p_qp, "query planes"));
     VS_TAKE(A.get(qf, (size_t)std::max<int64_t>(nq, 1) * x->d * 4, &p_qf, "query copy"));
     VS_TAKE(A.get(qnorm, (size_t)pq->nq_pad * 4, &p_qn, "query norms"));
     pq->qp = (uint16_t *)p_qp;
     pq->qf = (float *)p_qf;
     pq->qnorm = (float *)p_qn;
+    if (want_res) {
+        void *p_qr;
+        VS_TAKE(A.get(x->qres, (size_t)pq->nq_pad * 4, &p_qr, "query residuals"));
+        pq->qres = (float *)p_qr;
+    }
     if (defer_flags && (q_dtype == VS_DTYPE_BF16 || spec_one_plane)) {
-        VS_HIP(vs::launch_prepare_queries(q_dev, q_dtype, stride, nq, x->d, x->ld, x->metric, *pq,
+        VS_HIP(vs::launch_prepare_queries(q_dev, q_dtype, stride, nq, x->d, x->sel.ld, x->metric, *pq,
                                           defer_flags, x->st),
                "preparing queries");
         pq->planes = 1;
@@ -859,7 +928,7 @@ int prepare_queries(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64
     }
     VS_TAKE(A.get(x->flags, sizeof(uint32_t), &p_fl, "flags buffer"));
     VS_HIP(vs::launch_fill32(p_fl, 1, 0u, x->st), "clearing flags");
-    VS_HIP(vs::launch_prepare_queries(q_dev, q_dtype, stride, nq, x->d, x->ld, x->metric, *pq,
+    VS_HIP(vs::launch_prepare_queries(q_dev, q_dtype, stride, nq, x->d, x->sel.ld, x->metric, *pq,
                                       (uint32_t *)p_fl, x->st),
            "preparing queries");
     uint32_t f = 0;
@@ -873,9 +942,10 @@ int prepare_queries(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64
 
 int prepare_queries(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t stride,
                     int64_t nq, vs::PreparedQueries *pq, uint32_t *flags_out,
-                    uint32_t *defer_flags = nullptr, bool spec_one_plane = false) {
+                    uint32_t *defer_flags = nullptr, bool spec_one_plane = false,
+                    bool want_res = false) {
     return prepare_queries(x, A, q_dev, q_dtype, stride, nq, pq, flags_out, x->qp, x->qf,
-                           x->qnorm, defer_flags, spec_one_plane);
+                           x->qnorm, defer_flags, spec_one_plane, want_res);
 }
 
 __global__ void fill_sentinels_kernel(float *D, int32_t *I, int64_t m, float v) {
@@ -899,7 +969,8 @@ struct ListBufs {
 size_t list_count(const vs::ScanPlan &p) { return (size_t)p.nqblk * p.nsplit * p.lw * p.bn; }
 // the lists, then the split merge's partial area
 size_t list_elems(const vs::ScanPlan &p) {
-    const size_t part = p.merge_g > 1 ? (size_t)p.nqblk * p.bn * p.merge_g * p.kk_final : 0;
+    const size_t part =
+        p.merge_g > 1 ? (size_t)p.nqblk * p.bn * p.merge_g * std::max(p.keep, p.kk_final) : 0;
     return list_count(p) * p.cap + part;
 }
 
@@ -951,7 +1022,7 @@ int seed_thresholds(vs_index *x, const vs::PreparedQueries &pq, int64_t S, int64
     S = std::min<int64_t>(S, x->ntotal);
     vs::ScanPlan pp;
     if (max_lists < 0) max_lists = 0;
-    int rc = plan_scan(x, pq.nq, S, pq.planes, kk_final, x->storage, &pp, false, max_lists, false,
+    int rc = plan_scan(x, pq.nq, S, pq.planes, kk_final, x->sel.storage, &pp, false, max_lists, false,
                        2, list_budget);
     if (rc) return rc;
     // an estimate needs only the values of the sample's seed_rank smallest:
@@ -960,7 +1031,7 @@ int seed_thresholds(vs_index *x, const vs::PreparedQueries &pq, int64_t S, int64
     // the estimate is larger, never smaller)
     if (pp.kind == 3 && seed_rank > 0 && seed_rank <= 4 * vs::share_topm_est()) {
         vs::ScanPlan tp = pp;
-        if (plan_share(x, pq.nq, S, pq.planes, x->storage, &tp, max_lists, 0)) {
+        if (plan_share(x, pq.nq, S, pq.planes, x->sel.storage, &tp, max_lists, 0)) {
             pp = tp;
             pp.share_topm = vs::share_topm_est();
             plan_merge(x, pq.nq, &pp);
@@ -1004,7 +1075,7 @@ int seed_thresholds(vs_index *x, const vs::PreparedQueries &pq, int64_t S, int64
     VS_HIP(vs::launch_fill32(L->cnt + list_count(pp), 1, 0u, x->st), "list counts");
     {
         ProfScope ps(x, "prepass");
-        VS_HIP(vs::launch_scan_topk(x->xb, x->storage, x->ld, x->xn, S, x->metric, pq, pp, L->v,
+        VS_HIP(vs::launch_scan_topk(x->sel.rows, x->sel.storage, x->sel.ld, x->xn, S, x->metric, pq, pp, L->v,
                                     L->i, gthr, nullptr, L->cnt, x->st),
                "seeding scan");
     }
@@ -1026,9 +1097,13 @@ int seed_thresholds(vs_index *x, const vs::PreparedQueries &pq, int64_t S, int64
 // chosen four standard deviations and four rows above that mean (below 1e-5
 // per query for every kk_final this build allows).  Queries whose estimate
 // was too tight are found by the merge and searched again exactly.
+// Without a threshold the lists' bookkeeping outweighs the scan long before
+// 2^18 rows (200,000 x 768, 3,000 queries: 4.2 ms of scan for 0.8 ms of
+// products); small batches over more rows than that start from a bound
+// instead (needs_seed).
 bool needs_guess(const vs_index *x, const vs::ScanPlan &plan, int64_t nq) {
-    return x->opt.guess && nq >= 256 &&
-           x->ntotal >= (1 << 18) && plan.nsplit * plan.lw * plan.kk >= 4 * plan.kk_final;
+    return x->opt.guess && x->opt.scan_kkw == 0 && nq >= (x->ntotal >= (1 << 18) ? 256 : 16) &&
+           x->ntotal >= (1 << 14) && plan.nsplit * plan.lw * plan.kk >= 4 * plan.kk_final;
 }
 
 // The sample is 1/2^div_log2 of the rows (option guess_div_log2, 1/32 by
@@ -1045,12 +1120,15 @@ int guess_div_log2(const vs_index *x) {
 int guess_thresholds(vs_index *x, const vs::PreparedQueries &pq, int64_t kk_final, int div_log2,
                      uint32_t *gthr, ListBufs *L, size_t *need_elems, size_t *need_lists) {
     const int64_t S =
-        std::min<int64_t>(x->ntotal, std::max<int64_t>(4096, x->ntotal >> div_log2));
+        std::min<int64_t>(x->ntotal, std::max<int64_t>(1024, x->ntotal >> div_log2));
     const double lam = (double)kk_final * (double)S / (double)x->ntotal;
     const int j = (int)std::ceil(lam + 4.0 * std::sqrt(lam) + 4.0);
     const int64_t kkp = std::max<int64_t>(8, next_pow2(j));
     if (L && !x->prof_fixed) x->prof["guess_scans"].launches++;
-    return seed_thresholds(x, pq, S, kkp, gthr, L, need_elems, need_lists, j, 12);
+    // few lists per query warm up soonest; small batches need more to fill the
+    // chip (100 queries, 6,250 rows of 768: 604 us on 8 workgroups)
+    const int64_t lists = std::max<int64_t>(12, 12 * 1024 / pq.nq);
+    return seed_thresholds(x, pq, S, kkp, gthr, L, need_elems, need_lists, j, lists);
 }
 
 // The largest stored row norm (times 1 + 1e-6), cached per row version.
@@ -1073,6 +1151,72 @@ int xnorm_max(vs_index *x, Arena &A, float *out) {
     return VS_OK;
 }
 
+// Brings the bf16 copy of fp32 rows up to date (rows added since the last
+// call are appended); false if there is none: the copy is optional, and taken
+// only where it leaves three quarters of the free memory to others.  The
+// caller holds it (CopyHold).  One wait, when rows were copied.
+bool ensure_copy16(vs_index *x) {
+    if (x->storage != 0 || x->ntotal == 0) return false;
+    const int64_t ld16 = vs::storage_ld(x->d, 1);
+    if (x->copy_n == x->ntotal && x->copy_cap >= x->ntotal) return std::isfinite(x->copy_res);
+    const size_t rb = (size_t)ld16 * 2;
+    auto fail = [&] {
+        (void)hipGetLastError();
+        std::lock_guard<std::mutex> lk(g_copies_mu);
+        drop_copy(x);
+        return false;
+    };
+    if (x->copy_cap < x->ntotal) {
+        size_t freeb = 0, total = 0;
+        const size_t bytes = (size_t)(x->cap + kRowSlack) * rb;
+        {
+            std::lock_guard<std::mutex> lk(g_copies_mu);
+            drop_copy(x);
+        }
+        if (hipMemGetInfo(&freeb, &total) != hipSuccess || bytes > freeb / 4) return fail();
+        // (not dev_malloc: the copy is optional and evicts no other; its last
+        // 256 bytes hold the residual's maximum)
+        if (hipMalloc(&x->xb16.p, bytes + 256) != hipSuccess) {
+            x->xb16.p = nullptr;
+            return fail();
+        }
+        x->xb16.bytes = bytes;
+        x->copy_ld = ld16;
+        x->copy_cap = x->cap;
+        std::lock_guard<std::mutex> lk(g_copies_mu);
+        g_copies.push_back(x);
+    }
+    float *res_dev = (float *)(x->xb16.as<char>() + x->xb16.bytes);
+    if (x->copy_n == 0) x->copy_res = 0.f;
+    char *dst = x->xb16.as<char>() + (size_t)x->copy_n * rb;
+    const char *src = (const char *)x->xb + (size_t)x->copy_n * row_bytes(x);
+    const int64_t m = x->ntotal - x->copy_n;
+    float res = 0.f;
+    // (the tile past the last row is read whole: zero rows after it)
+    if (vs::launch_copy_rows16(src, x->ld, m, ld16, dst, res_dev, x->st) != hipSuccess ||
+        hipMemsetAsync(dst + (size_t)m * rb, 0, (size_t)kRowSlack * rb, x->st) != hipSuccess ||
+        hipMemcpyAsync(&res, res_dev, sizeof res, hipMemcpyDeviceToHost, x->st) != hipSuccess ||
+        hipStreamSynchronize(x->st) != hipSuccess)
+        return fail();
+    x->copy_res = std::max(x->copy_res, res);
+    x->copy_n = x->ntotal;
+    return std::isfinite(x->copy_res);
+}
+
+// The scans of this call read the stored rows.
+void select_rows(vs_index *x) {
+    x->sel.rows = x->xb;
+    x->sel.storage = x->storage;
+    x->sel.ld = x->ld;
+}
+
+// The scans of this call read the bf16 copy of the rows.
+void select_copy(vs_index *x) {
+    x->sel.rows = x->xb16.p;
+    x->sel.storage = 1;
+    x->sel.ld = x->copy_ld;
+}
+
 // Accumulator error model of a top-k scan of these rows with these queries
 // (relative error of one product of MFMA operands; the accumulation factor
 // covers up to three passes of d products and the fp32 row norms):
@@ -1092,8 +1236,8 @@ double accum_gamma(int64_t d, int npass) {
 }
 
 void topk_error_model(const vs_index *x, int planes, vs::TopkCheck *chk) {
-    chk->err_g = (float)accum_gamma(x->d, x->storage == 1 ? planes : 1 + planes);
-    if (x->storage == 1)
+    chk->err_g = (float)accum_gamma(x->d, x->sel.storage == 1 ? planes : 1 + planes);
+    if (x->sel.storage == 1)
         chk->err_r = planes == 1 ? 0.f : (float)(1.0 / 65536.0);
     else
         chk->err_r = planes == 1 ? (float)(1.0 / 65536.0) : (float)(1.0 / 32768.0);
@@ -1232,21 +1376,22 @@ int exact_search(vs_index *x, Arena &A, const float *qf, int64_t nq, int64_t k, 
 }
 
 // Re-search of the queries listed in list_dev (device, m entries) of the
-// prepared queries pq: their rows are gathered, searched by `how` (0: the
-// MFMA selection again with full-length lists and no estimates; 1: the
-// exact path), and their k results scattered back into D / I.
-int research_listed(vs_index *x, Arena &A, const vs::PreparedQueries &pq, const int32_t *list_dev,
-                    int64_t m, int64_t k, float *D, int32_t *I, int how) {
+// query rows qf (gathered: row i is query list[i] already): searched by `how`
+// (0: the MFMA selection again with full-length lists and no estimates; 1:
+// the exact path), and their k results scattered back into D / I.
+int research_listed(vs_index *x, Arena &A, const float *qf, const int32_t *list_dev, int64_t m,
+                    int64_t k, float *D, int32_t *I, int how, bool gathered = false) {
     if (m <= 0) return VS_OK;
-    void *lst, *fq, *fD, *fI;
+    void *lst, *fq = (void *)qf, *fD, *fI;
     VS_TAKE(A.tmp((size_t)m * 4, &lst, "fallback list"));
-    VS_TAKE(A.tmp((size_t)m * x->d * 4, &fq, "fallback queries"));
+    if (!gathered) VS_TAKE(A.tmp((size_t)m * x->d * 4, &fq, "fallback queries"));
     VS_TAKE(A.tmp((size_t)m * k * 4, &fD, "fallback results"));
     VS_TAKE(A.tmp((size_t)m * k * 4, &fI, "fallback results"));
     VS_HIP(hipMemcpyAsync(lst, list_dev, (size_t)m * 4, hipMemcpyDeviceToDevice, x->st),
            "fallback list");
-    VS_HIP(vs::launch_gather_rows(pq.qf, (const int32_t *)lst, m, x->d, fq, x->st),
-           "fallback gather");
+    if (!gathered)
+        VS_HIP(vs::launch_gather_rows(qf, (const int32_t *)lst, m, x->d, fq, x->st),
+               "fallback gather");
     const size_t mk = A.mark();
     int rc = how == 0 ? search_device(x, A, fq, VS_DTYPE_F32, m, k, (float *)fD, (int32_t *)fI,
                                       true, A.fixed() ? (size_t)(48 << 20) : 0)
@@ -1259,9 +1404,129 @@ int research_listed(vs_index *x, Arena &A, const vs::PreparedQueries &pq, const 
     return VS_OK;
 }
 
+// fp32 rows, queries of any values: the scan multiplies their bf16 roundings
+// once (one MFMA pass over half the bytes, instead of three passes over hi
+// and lo planes), the merge re-ranks its candidates in fp64 from the fp32
+// rows, and its proof allows for the rounding: an accumulator lies within
+// s (r_q (x_max + r_x) + |q| r_x) of that of the unrounded operands, r_q the
+// norm of the query's rounding residual and r_x the largest of a row's (both
+// measured, about 0.0016 of the norms).  The merge keeps twice the
+// candidates; queries it cannot prove go to bounded_research.
+bool coarse_search(const vs_index *x, int64_t k) {
+    const VsOptions &o = x->opt;
+    if (x->storage != 0 || !o.coarse || !o.copy16 || k > 200) return false;
+    // an option that forces a scan is about that scan on these rows
+    return o.gemm < 0 && o.share < 0 && !o.gemm_min_nq && !o.gemm_wq && !o.gemm_qb && !o.gemm_kc &&
+           !o.gemm4 && !o.scan_kkw && !o.scan_nw8;
+}
+
+// Exact top-k of the m queries listed in list_dev (device) whose selection the
+// merge could not prove, given k results each (any k rows: the k-th exact
+// score e_k among them bounds the true one).  A row of the true top-k has an
+// accumulator at or below e_k's plus the error bound, so a range scan of the
+// same rows (x->sel) under that bound finds them all; the candidates are
+// scored exactly and the k best selected.  One more scan, whatever the data:
+// rows in clusters tighter than the error leave hundreds of candidates per
+// query, not thousands of products with every row.  Past 2^27 candidates, the
+// exact path.
+int bounded_research(vs_index *x, Arena &A, const vs::PreparedQueries &pq, int planes,
+                     const vs::TopkCheck &chk, const int32_t *list_dev, int64_t m, int64_t k,
+                     float *D, int32_t *I) {
+    if (m <= 0) return VS_OK;
+    void *lst, *fq, *fD, *fI;
+    VS_TAKE(A.get(x->fbl, (size_t)m * 4, &lst, "re-search list"));
+    VS_TAKE(A.get(x->fbq, (size_t)m * x->d * 4, &fq, "re-search queries"));
+    VS_TAKE(A.get(x->fbD, (size_t)m * k * 4, &fD, "re-search results"));
+    VS_TAKE(A.get(x->fbI, (size_t)m * k * 4, &fI, "re-search results"));
+    VS_HIP(hipMemcpyAsync(lst, list_dev, (size_t)m * 4, hipMemcpyDeviceToDevice, x->st),
+           "re-search list");
+    VS_HIP(vs::launch_gather_rows(pq.qf, (const int32_t *)lst, m, x->d, fq, x->st),
+           "re-search gather");
+    x->prof["exact_fallback"].launches += m;
+    vs::PreparedQueries rq;
+    VS_HIP(x->flags.ensure(8), "flags buffer");
+    uint32_t *fl = x->flags.as<uint32_t>();  // [0] query flags, [1] the kernels' errors
+    VS_HIP(vs::launch_fill32(fl, 2, 0u, x->st), "clearing flags");
+    int rc = prepare_queries(x, A, fq, VS_DTYPE_F32, x->d, m, &rq, nullptr, fl, true,
+                             chk.qres != nullptr);
+    if (rc) return rc;
+    rq.planes = planes;  // (both planes are written)
+    vs::ScanPlan plan;
+    rc = plan_scan(x, m, x->ntotal, planes, 8, x->sel.storage, &plan, false, 0, true);
+    if (rc) return rc;
+    if ((rc = scan_fits(plan, rq))) return rc;
+    VS_HIP(x->athr.ensure((size_t)m * 4), "re-search bounds");
+    VS_HIP(vs::launch_bounded_thresholds(rq, x->d, x->metric, chk, D, (const int32_t *)lst, k,
+                                         x->athr.as<float>(), x->st),
+           "re-search bounds");
+    // counters: the candidates found; per query its count, then its fill
+    VS_HIP(x->rcount.ensure(16 + (size_t)(3 * m + 1) * 4), "re-search counters");
+    unsigned long long *count = x->rcount.as<unsigned long long>();
+    int32_t *qcnt = (int32_t *)(count + 2), *qfill = qcnt + m, *qoff = qfill + m;
+    int64_t cap = std::min<int64_t>((int64_t)1 << 24, std::max<int64_t>((int64_t)1 << 18, m * 512));
+    VS_HIP(x->hio.ensure(kCtlBytes), "control words");
+    volatile unsigned long long *hfound = (unsigned long long *)(x->hio.as<char>() + 64);
+    void *cq = nullptr, *ci = nullptr;
+    int64_t found = 0;
+    for (int attempt = 0;; ++attempt) {
+        if (attempt == 0) {
+            VS_TAKE(A.get(x->rq, (size_t)cap * 4, &cq, "re-search candidates"));
+            VS_TAKE(A.get(x->ri, (size_t)cap * 4, &ci, "re-search candidates"));
+        } else {
+            VS_TAKE(A.tmp((size_t)cap * 4, &cq, "re-search candidates"));
+            VS_TAKE(A.tmp((size_t)cap * 4, &ci, "re-search candidates"));
+        }
+        VS_HIP(vs::launch_fill32(count, 4 + 2 * m, 0u, x->st), "re-search counters");
+        {
+            ProfScope ps(x, "rescan");
+            VS_HIP(vs::launch_scan_range(x->sel.rows, x->sel.storage, x->sel.ld, x->xn, x->ntotal,
+                                         rq, plan, x->athr.as<float>(), 0, x->metric,
+                                         (int32_t *)cq, (int32_t *)ci, count, cap, x->st),
+                   "re-search scan");
+        }
+        VS_HIP(hipMemcpyAsync((void *)hfound, count, 8, hipMemcpyDeviceToHost, x->st),
+               "re-search count");
+        VS_HIP(hipStreamSynchronize(x->st), "re-search scan");
+        found = (int64_t)*hfound;
+        if (found <= cap || found > ((int64_t)1 << 27)) break;
+        cap = found;
+    }
+    bool ok = found <= cap;
+    if (ok) {
+        void *keys;
+        const size_t kb = (size_t)std::max<int64_t>(found, 1) * 8;
+        if (kb <= (size_t)1 << 28) VS_TAKE(A.get(x->ex_keys, kb, &keys, "re-search keys"));
+        else VS_TAKE(A.tmp(kb, &keys, "re-search keys"));
+        VS_HIP(vs::launch_count_pairs((const int32_t *)cq, found, m, qcnt, x->st),
+               "re-search counts");
+        VS_HIP(vs::launch_exclusive_scan_i32(qcnt, m, qoff, x->st), "re-search offsets");
+        VS_HIP(vs::launch_exact_pair_keys(x->xb, x->storage, x->ld, x->d, x->metric, rq.qf,
+                                          (const int32_t *)cq, (const int32_t *)ci, found, m,
+                                          x->ntotal, qoff, qfill, (uint64_t *)keys, fl + 1, x->st),
+               "re-search scores");
+        VS_HIP(vs::launch_select_groups((const uint64_t *)keys, qoff, qcnt, m, k, x->metric,
+                                        (float *)fD, (int32_t *)fI, fl + 1, x->st),
+               "re-search selection");
+        volatile uint32_t *herr = (uint32_t *)(x->hio.as<char>() + 72);
+        VS_HIP(hipMemcpyAsync((void *)herr, fl + 1, 4, hipMemcpyDeviceToHost, x->st),
+               "re-search flags");
+        VS_HIP(hipStreamSynchronize(x->st), "re-search");
+        if (*herr & vs::kFlagBadId)
+            return set_err(VS_ERR_HIP, "internal error: a re-search candidate outside the index");
+        ok = !(*herr & vs::kFlagShort);
+    }
+    if (!ok) {  // too many candidates, or fewer than k (accumulators past fp32)
+        rc = exact_search(x, A, (const float *)fq, m, k, (float *)fD, (int32_t *)fI);
+        if (rc) return rc;
+    }
+    VS_HIP(vs::launch_scatter_rows(fD, (const int32_t *)lst, m, k, D, x->st), "re-search scatter");
+    VS_HIP(vs::launch_scatter_rows(fI, (const int32_t *)lst, m, k, I, x->st), "re-search scatter");
+    return VS_OK;
+}
+
 // Top-k search of nq device query rows into device D / I [nq][k].  safe:
 // full-length lists and no threshold estimates (the re-search of queries
-// the merge could not prove exact).  list_budget > 0 bounds the bytes of
+// the merge could not prove exact), on every plane of fp32 rows.  list_budget > 0 bounds the bytes of
 // the candidate lists (the streaming scan's split count adapts).
 int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t nq, int64_t k,
                   float *D, int32_t *I, bool safe, size_t list_budget) {
@@ -1294,7 +1559,12 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
             return set_err(VS_ERR_NONFINITE, "queries contain NaN or infinity");
         return VS_OK;
     }
-    const int64_t kk = std::max<int64_t>(8, next_pow2(k + std::max<int64_t>(4, k / 4)));
+    int64_t kk = std::max<int64_t>(8, next_pow2(k + std::max<int64_t>(4, k / 4)));
+    select_rows(x);
+    CopyHold hold(x);
+    const bool coarse = !safe && !A.fixed() && hold.mine && coarse_search(x, k) &&
+                        ensure_copy16(x);
+    if (coarse) select_copy(x);
     // control words: merge flags, the counts of the two lists, then the
     // query flags of bf16 queries (read with the results)
     void *p_ctl;
@@ -1306,9 +1576,9 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
     // the query flags, which are read with the results); the rare batch with
     // a query that bf16 does not hold is searched again with two planes (not
     // in a fixed arena, whose scratch holds one search)
-    const bool spec = kk <= 512 && q_dtype != VS_DTYPE_BF16 && x->storage == 1 && !A.fixed();
+    const bool spec = kk <= 512 && q_dtype != VS_DTYPE_BF16 && x->sel.storage == 1 && !A.fixed();
     int rc = prepare_queries(x, A, q_dev, q_dtype, x->d, nq, &pq, nullptr,
-                             kk <= 512 ? (uint32_t *)(ctl + 3) : nullptr, spec);
+                             kk <= 512 ? (uint32_t *)(ctl + 3) : nullptr, spec, coarse);
     if (rc) return rc;
     if (kk > 512) {  // beyond the fused selection: the sorting path
         rc = exact_search(x, A, pq.qf, nq, k, D, I);
@@ -1316,14 +1586,27 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
         VS_HIP(hipStreamSynchronize(x->st), "search");
         return VS_OK;
     }
+    bool coarse_wide = false;
     for (int attempt = 0;; ++attempt) {
         vs::ScanPlan plan;
-        rc = plan_scan(x, nq, x->ntotal, pq.planes, kk, x->storage, &plan, safe, 0, false, 8,
+        rc = plan_scan(x, nq, x->ntotal, pq.planes, kk, x->sel.storage, &plan, safe, 0, false, 8,
                        list_budget);
         if (rc) return rc;
         if ((rc = scan_fits(plan, pq))) return rc;
+        bool guess = !safe && needs_guess(x, plan, nq);
+        if (coarse && guess) {
+            // the estimate leaves about four times kk candidates in the lists:
+            // the merge keeps more of them than the scan's thresholds promise
+            plan.keep = (int)std::min<int64_t>(512, 2 * kk);
+            plan_merge(x, nq, &plan);
+        } else if (coarse && kk <= 256 && !coarse_wide) {
+            // thresholds tighten to the kk-th value: ask for more candidates
+            coarse_wide = true;
+            kk = std::max<int64_t>(nq <= 64 ? 64 : 32, 2 * kk);
+            --attempt;
+            continue;
+        }
         const bool verify = plan.kk < plan.kk_final;
-        const bool guess = !safe && needs_guess(x, plan, nq);
         const bool seed = !guess && !safe && needs_seed(x, plan) && x->opt.prepass;
         const int64_t seed_S =
             std::max<int64_t>((int64_t)1 << x->opt.prepass_log2, x->ntotal / kPrepassDiv);
@@ -1355,13 +1638,20 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
         VS_HIP(vs::launch_fill32(L.cnt + list_count(plan), 1, 0u, x->st), "list counts");
         {
             ProfScope ps(x, "scan");
-            VS_HIP(vs::launch_scan_topk(x->xb, x->storage, x->ld, x->xn, x->ntotal, x->metric, pq, plan,
-                                        L.v, L.i, gthr, (float *)p_lb, L.cnt, x->st),
+            VS_HIP(vs::launch_scan_topk(x->sel.rows, x->sel.storage, x->sel.ld, x->xn, x->ntotal,
+                                        x->metric, pq, plan, L.v, L.i, gthr, (float *)p_lb, L.cnt, x->st),
                    "scan kernel");
         }
         vs::TopkCheck chk;
         VS_TAKE(xnorm_max(x, A, &chk.xmax));
         topk_error_model(x, pq.planes, &chk);
+        if (coarse) {
+            chk.qres = pq.qres;
+            chk.xres = x->copy_res;
+            // non-finite queries leave the caller's results alone, as where
+            // they are found before the scan
+            chk.qflags = (const uint32_t *)(ctl + 3);
+        }
         chk.vx_count = ctl + 2;
         chk.vx_list = (int32_t *)p_vx;
         {
@@ -1381,7 +1671,7 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
         VS_HIP(hipMemcpyAsync(ph, ctl, sizeof hc, hipMemcpyDeviceToHost, x->st), "merge flags");
         VS_HIP(hipStreamSynchronize(x->st), "search");
         if (ph != hc) memcpy(hc, ph, sizeof hc);
-        if (attempt == 0 && spec && ((uint32_t)hc[3] & vs::kFlagNotBf16) &&
+        if (attempt == 0 && spec && !coarse && ((uint32_t)hc[3] & vs::kFlagNotBf16) &&
             !((uint32_t)hc[3] & vs::kFlagNonFinite)) {
             pq.planes = 2;  // (both planes were prepared)
             VS_HIP(vs::launch_fill32(ctl, 3, 0u, x->st), "control words");
@@ -1392,15 +1682,30 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
         if ((uint32_t)hc[0] & vs::kFlagBadId)
             return set_err(VS_ERR_HIP, "internal error: a candidate id outside the index reached the merge");
         // queries whose shortened lists may have dropped a winner, or whose
-        // estimated threshold left fewer than kk_final candidates, are searched
-        // again with full-length lists and no estimate; queries whose selection
-        // the accumulator's error could have changed go to the exact path
-        // (both rare for unordered data)
-        // (the exact path first: the re-search prepares its queries into the
-        // index's query buffers, which both gathers read)
-        rc = research_listed(x, A, pq, (const int32_t *)p_vx, hc[2], k, D, I, 1);
+        // estimated threshold left fewer than kk_final candidates (on the
+        // one-pass selection: fewer than k), are searched again with
+        // full-length lists and no estimate; queries whose selection the
+        // accumulator's error could have changed are searched again within
+        // that error (both rare for unordered data), or, in a fixed arena, by
+        // the exact path.  (The list of the former is read last: both
+        // gathers read the query buffers, which the re-searches prepare
+        // theirs into, so it gathers first.)
+        void *vfq = nullptr, *vfl = nullptr;
+        if (hc[1] > 0 && hc[2] > 0 && !A.fixed()) {
+            VS_TAKE(A.tmp((size_t)hc[1] * x->d * 4, &vfq, "fallback queries"));
+            VS_TAKE(A.tmp((size_t)hc[1] * 4, &vfl, "fallback list"));
+            VS_HIP(hipMemcpyAsync(vfl, p_vf, (size_t)hc[1] * 4, hipMemcpyDeviceToDevice, x->st),
+                   "fallback list");
+            VS_HIP(vs::launch_gather_rows(pq.qf, (const int32_t *)vfl, hc[1], x->d, vfq, x->st),
+                   "fallback gather");
+        }
+        rc = A.fixed() ? research_listed(x, A, pq.qf, (const int32_t *)p_vx, hc[2], k, D, I, 1)
+                       : bounded_research(x, A, pq, pq.planes, chk, (const int32_t *)p_vx, hc[2], k,
+                                          D, I);
         if (rc) return rc;
-        rc = research_listed(x, A, pq, (const int32_t *)p_vf, hc[1], k, D, I, 0);
+        rc = research_listed(x, A, vfq ? (const float *)vfq : pq.qf,
+                             vfq ? (const int32_t *)vfl : (const int32_t *)p_vf, hc[1], k, D, I, 0,
+                             vfq != nullptr);
         if (rc) return rc;
         VS_HIP(hipStreamSynchronize(x->st), "search");
         return VS_OK;
@@ -1412,71 +1717,49 @@ struct RangeHits {
     std::vector<float> s;
 };
 
-// Candidate scan + exact re-test; hits sorted by (query, id).
-int range_core(vs_index *x, const vs::PreparedQueries &pq, double radius, int self_join,
-               uint32_t qflags, RangeHits *out) {
+// Candidate scan + exact re-test of nq query rows (device, `stride` elements
+// apart); hits sorted by (query, id).
+int range_core(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int64_t nq,
+               double radius, int self_join, RangeHits *out) {
     out->q.clear();
     out->id.clear();
     out->s.clear();
-    if (pq.nq == 0 || x->ntotal == 0) return VS_OK;
-    // one-pass selection of fp32 rows where the GEMM-tiled scan runs it: the
-    // acceptance bounds widen to its error and every hit is re-tested exactly
+    if (nq == 0 || x->ntotal == 0) return VS_OK;
+    select_rows(x);
+    // One-pass selection of fp32 rows: the acceptance bounds widen to the
+    // operands' rounding to bf16 and every hit is re-tested exactly.  It
+    // multiplies the bf16 copy of the rows (with the fp32 rows' norms), or,
+    // without one, rounds them in the GEMM-tiled scan where that applies.
+    CopyHold hold(x);
+    const bool copy = x->storage == 0 && x->opt.coarse && x->opt.copy16 && hold.mine &&
+                      ensure_copy16(x);
+    if (copy) select_copy(x);
+    Arena A;
+    vs::PreparedQueries pq;
+    uint32_t qflags = 0;
+    int rc = prepare_queries(x, A, q_dev, q_dtype, stride, nq, &pq, &qflags, nullptr, false, copy);
+    if (rc) return rc;
+    if (copy) pq.planes = 1;
     vs::ScanPlan plan;
-    int rc = VS_OK;
-    bool coarse = x->storage == 0 && x->opt.coarse;
+    bool coarse = !copy && x->storage == 0 && x->opt.coarse;
     if (coarse)
-        coarse = plan_scan(x, pq.nq, x->ntotal, 1, 8, vs::kSelectCoarse, &plan, false, 0, true) ==
+        coarse = plan_scan(x, nq, x->ntotal, 1, 8, vs::kSelectCoarse, &plan, false, 0, true) ==
                      VS_OK &&
                  plan.kind == 2;
     if (!coarse) {
         plan = vs::ScanPlan();
-        rc = plan_scan(x, pq.nq, x->ntotal, pq.planes, 8, x->storage, &plan, false, 0, true);
+        rc = plan_scan(x, nq, x->ntotal, pq.planes, 8, x->sel.storage, &plan, false, 0, true);
         if (rc) return rc;
     }
     if ((rc = scan_fits(plan, pq))) return rc;
-    // the one-pass selection multiplies the rows' bf16 rounding: it reads a
-    // bf16 copy of them (half the bytes, no conversion in the kernel) with
-    // the fp32 rows' norms, when the copy fits in memory
-    const void *scan_rows = x->xb;
-    int scan_storage = x->storage;
-    if (coarse && plan.tile_st == vs::kSelectCoarse && x->opt.copy16) {
-        const size_t bytes = (size_t)(x->ntotal + kRowSlack) * x->ld * 2;
-        if (x->xb16_version != x->version) {
-            x->xb16_version = ~0ull;
-            if (x->xb16.ensure(bytes) == hipSuccess &&
-                x->xb16n.ensure((size_t)(x->ntotal + kRowSlack) * 4) == hipSuccess) {
-                VS_HIP(hipMemsetAsync(x->xb16.p, 0, bytes, x->st), "row copy");
-                VS_HIP(x->flags.ensure(4), "flags");
-                VS_HIP(vs::launch_store_rows(x->xb, 0, x->ld, x->ntotal, x->ld, x->xb16.p, 1, x->ld,
-                                             x->xb16n.as<float>(), x->flags.as<uint32_t>(), x->st),
-                       "row copy");
-                x->xb16_version = x->version;
-            } else {
-                (void)hipGetLastError();
-                x->xb16.release();
-                x->xb16n.release();
-            }
-        }
-        if (x->xb16_version == x->version) {
-            // the copy holds bf16 rows: their own plan (the four-wave
-            // pipelined kernel applies to them)
-            vs::ScanPlan p16;
-            if (plan_scan(x, pq.nq, x->ntotal, 1, 8, 1, &p16, false, 0, true) == VS_OK &&
-                p16.kind == 2 && p16.bn <= 256 && p16.nqblk * p16.bn <= pq.nq_pad)
-                plan = p16;
-            plan.tile_st = 1;
-            scan_rows = x->xb16.p;
-            scan_storage = 1;
-        }
-    }
-    Arena A;
     float xmax = 0.f;
     VS_TAKE(xnorm_max(x, A, &xmax));
     VS_HIP(x->athr.ensure((size_t)pq.nq * 4), "range bounds");
-    const int exact_q = (qflags & vs::kFlagNotBf16) ? 0 : 1;
-    const int exact_x = x->storage == 1 ? 1 : 0;
+    // (on the copy, the residual norms stand for both operands' rounding)
+    const int exact_q = copy || !(qflags & vs::kFlagNotBf16) ? 1 : 0;
+    const int exact_x = x->sel.storage == 1 ? 1 : 0;
     VS_HIP(vs::launch_range_bounds(pq, x->d, x->metric, radius, xmax, exact_q, exact_x, coarse,
-                                   x->athr.as<float>(), x->st),
+                                   copy ? x->copy_res : 0.f, x->athr.as<float>(), x->st),
            "range bounds");
     VS_HIP(x->rcount.ensure(sizeof(unsigned long long)), "range counter");
     int64_t cap = std::max<int64_t>(1 << 20, pq.nq * 4);
@@ -1488,8 +1771,8 @@ int range_core(vs_index *x, const vs::PreparedQueries &pq, double radius, int se
         note_scan_kind(x, plan);
         {
             ProfScope ps(x, self_join ? "join" : "range");
-            VS_HIP(vs::launch_scan_range(scan_rows, scan_storage, x->ld, x->xn, x->ntotal, pq, plan,
-                                         x->athr.as<float>(), self_join, x->metric,
+            VS_HIP(vs::launch_scan_range(x->sel.rows, x->sel.storage, x->sel.ld, x->xn, x->ntotal,
+                                         pq, plan, x->athr.as<float>(), self_join, x->metric,
                                          x->rq.as<int32_t>(), x->ri.as<int32_t>(),
                                          x->rcount.as<unsigned long long>(), cap, x->st),
                    "range scan");
@@ -1661,6 +1944,10 @@ void vs_index_destroy(vs_index *x) {
     if (!x) return;
     DeviceGuard g(x->device);
     if (x->st) (void)hipStreamSynchronize(x->st);
+    {
+        std::lock_guard<std::mutex> lk(g_copies_mu);
+        drop_copy(x);
+    }
     for (auto &p : x->pending) {
         (void)hipEventDestroy(p.a);
         (void)hipEventDestroy(p.b);
@@ -1674,8 +1961,8 @@ void vs_index_destroy(vs_index *x) {
                       &x->misc,    &x->km_cen,    &x->km_cxn,   &x->km_assign, &x->km_best,
                       &x->km_fb,   &x->km_keys,   &x->km_order, &x->km_tmp,   &x->km_counts,
                       &x->km_offsets, &x->km_out, &x->km_iota, &x->lcnt,   &x->km_qp,
-                      &x->km_qf,   &x->km_qnorm,  &x->km_cen16, &x->km_c16n, &x->xb16,
-                      &x->xb16n,   &x->vx,        &x->ctl,      &x->km_shift, &x->km_init,
+                      &x->km_qf,   &x->km_qnorm,  &x->km_cen16, &x->km_c16n, &x->qres, &x->fbl,
+                      &x->vx,        &x->ctl,      &x->km_shift, &x->km_init,
                       &x->km_pkeys, &x->km_part, &x->ex_qd,   &x->ex_keys, &x->ex_part};
     for (DevBuf *b : bufs) b->release();
     x->km_hbest.release();
@@ -1710,6 +1997,7 @@ int vs_index_reset(vs_index *x) {
         VS_HIP(hipStreamSynchronize(x->st), "reset");
     }
     x->ntotal = 0;
+    x->copy_n = 0;
     ++x->version;
     return VS_OK;
 }
@@ -1856,6 +2144,7 @@ int vs_index_remove_ids(vs_index *x, const int64_t *ids, int64_t n, int64_t *nre
     x->xb = nxb;
     x->xn = nxn;
     x->ntotal = w;
+    x->copy_n = 0;
     ++x->version;
     if (nremoved) *nremoved = removed;
     return VS_OK;
@@ -1973,12 +2262,7 @@ int vs_index_range_search(vs_index *x, const void *q, int q_dtype, int64_t nq, d
         VS_HIP(x->stage.ensure(qbytes), "query staging");
         VS_HIP(hipMemcpyAsync(x->stage.p, q, qbytes, hipMemcpyHostToDevice, x->st),
                "uploading queries");
-        vs::PreparedQueries pq;
-        uint32_t f = 0;
-        Arena A;
-        int rc = prepare_queries(x, A, x->stage.p, q_dtype, x->d, nq, &pq, &f);
-        if (rc) return rc;
-        rc = range_core(x, pq, radius, 0, f, &hits);
+        int rc = range_core(x, x->stage.p, q_dtype, x->d, nq, radius, 0, &hits);
         if (rc) return rc;
     }
     vs_range_result *r = (vs_range_result *)calloc(1, sizeof(vs_range_result));
@@ -2111,6 +2395,7 @@ int vs_index_search_subsets(vs_index *x, const void *q, int q_dtype, int64_t nq,
     VS_HIP(x->stage.ensure(qbytes), "query staging");
     VS_HIP(hipMemcpyAsync(x->stage.p, q, qbytes, hipMemcpyHostToDevice, x->st), "uploading queries");
     vs::PreparedQueries pq;
+    select_rows(x);
     if (int rc = prepare_queries(x, A, x->stage.p, q_dtype, x->d, nq, &pq, nullptr)) return rc;
     if (kk > 512) return search_subsets_sorted(x, A, pq, k, ids, seg_off, seg_len, nseg, D, I);
     const int64_t ns = std::max<int64_t>(1, nseg);
@@ -2179,12 +2464,7 @@ int vs_index_self_join(vs_index *x, double threshold, vs_pairs **out) {
     DeviceGuard g(x->device);
     RangeHits hits;
     if (x->ntotal > 1) {
-        vs::PreparedQueries pq;
-        uint32_t f = 0;
-        Arena A;
-        int rc = prepare_queries(x, A, x->xb, x->storage, x->ld, x->ntotal, &pq, &f);
-        if (rc) return rc;
-        rc = range_core(x, pq, threshold, 1, f, &hits);
+        int rc = range_core(x, x->xb, x->storage, x->ld, x->ntotal, threshold, 1, &hits);
         if (rc) return rc;
     }
     vs_pairs *p = (vs_pairs *)calloc(1, sizeof(vs_pairs));
@@ -2278,6 +2558,7 @@ int vs_kmeans_step(vs_index *x, const float *centroids_in, int64_t K, int64_t mi
     // points as prepared queries against the centroid "database" (kept
     // across iterations while the stored rows are unchanged)
     if (x->km_prep_version != x->version) {
+        select_rows(x);
         x->km_prep_version = ~0ull;
         int rc0 = prepare_queries(x, A, x->xb, 0, ld, n, &x->km_pq, &x->km_pflags, x->km_qp,
                                   x->km_qf, x->km_qnorm);
@@ -2288,7 +2569,7 @@ int vs_kmeans_step(vs_index *x, const float *centroids_in, int64_t K, int64_t mi
     int rc = VS_OK;
     // the distance kernels index the centroid rows with the points' ld
     vs_index cview;
-    cview.ld = ld;
+    cview.ld = cview.sel.ld = ld;
     cview.d = d;
     cview.lds_max = x->lds_max;
     cview.num_cu = x->num_cu;

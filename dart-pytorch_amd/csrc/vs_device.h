@@ -231,6 +231,74 @@ __device__ __forceinline__ void cut_lists_lanes(float *cv, int32_t *ci, int *cnt
     wave_sync();
 }
 
+// Range scans' (query, row) pairs.  A wave gathers its hits in LDS (bq / bi
+// [cap], *fill of them) and reserves room for a whole buffer with one atomic
+// on the scan's counter: reserved per tile, millions of hits serialise on
+// that word at about 10 ns each (300,000 x 256 rows, 500 queries, 147,000
+// hits one by one: 1.7 ms of a 0.2 ms scan).
+__device__ __forceinline__ void flush_pairs(const ScanKArgs &a, int *fill, const int *bq,
+                                            const int *bi, int lane) {
+    lds_wave_sync();
+    const int f = __builtin_amdgcn_readfirstlane(*fill);
+    if (f > 0) {
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(a.count, (unsigned long long)f);
+        base = __shfl(base, 0);
+        for (int t = lane; t < f; t += 64) {
+            if (base + t < (unsigned long long)a.out_cap) {
+                a.out_q[base + t] = bq[t];
+                a.out_i[base + t] = bi[t];
+            }
+        }
+    }
+    lds_wave_sync();
+    if (lane == 0) *fill = 0;
+    lds_wave_sync();
+}
+
+// Adds c pairs of each lane: emit(put) calls put(query, row) for each of
+// them.  More than the buffer takes at once go to memory directly.
+template <typename Emit>
+__device__ __forceinline__ void sink_pairs(const ScanKArgs &a, int c, int *fill, int *bq, int *bi,
+                                           int cap, int lane, Emit &&emit) {
+    int inc = c;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o);
+        if (lane >= o) inc += y;
+    }
+    const int total = __builtin_amdgcn_readlane(inc, 63);
+    if (!total) return;
+    int f = __builtin_amdgcn_readfirstlane(*fill);
+    if (f > 0 && total > cap - f) {
+        flush_pairs(a, fill, bq, bi, lane);
+        f = 0;
+    }
+    int *dq = bq + f, *di = bi + f;
+    long long room = cap;
+    const bool direct = total > cap;
+    if (direct) {
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(a.count, (unsigned long long)total);
+        base = __shfl(base, 0);
+        dq = a.out_q + base;
+        di = a.out_i + base;
+        room = (long long)a.out_cap - (long long)base;
+    }
+    int pos = inc - c;
+    emit([&](int q, int row) {
+        if (pos < room) {
+            dq[pos] = q;
+            di[pos] = row;
+        }
+        ++pos;
+    });
+    if (!direct) {
+        lds_wave_sync();
+        if (lane == 0) *fill = f + total;
+        lds_wave_sync();
+    }
+}
+
 // Word 3 of a raw buffer resource (gfx9: 32-bit data format, no swizzle).
 constexpr int kBufRsrcWord3 = 0x00020000;
 

@@ -259,6 +259,11 @@ struct SelectKeysArgs {
     const uint32_t *rowflags;
     int64_t nflags;
     uint32_t *hflags;
+    // groups instead of equal rows of keys (off non-null): query q's keys are
+    // keys[off[q] .. + cnt[q]); kFlagShort goes to *short_flag for one of
+    // fewer than k
+    const int32_t *off, *cnt;
+    uint32_t *short_flag;
 };
 
 __device__ __forceinline__ void sort_keys_block(uint64_t *b, int n) {
@@ -291,8 +296,9 @@ __global__ __launch_bounds__(kSelThreads) void select_keys_kernel(SelectKeysArgs
     const int64_t q = blockIdx.x / a.nseg;
     const int seg = (int)(blockIdx.x % a.nseg);
     const int64_t k0 = (int64_t)seg * a.seglen;
-    const int m = (int)max((int64_t)0, min(a.seglen, a.n - k0));
-    const uint64_t *kp = a.keys + q * a.kstride + k0;
+    const int m = a.off ? a.cnt[q] : (int)max((int64_t)0, min(a.seglen, a.n - k0));
+    const uint64_t *kp = a.keys + (a.off ? (int64_t)a.off[q] : q * a.kstride + k0);
+    if (a.off && tid == 0 && m < a.k) atomicOr(a.short_flag, kFlagShort);
 
     uint32_t flag = 0;
     if (a.rowflags) {
@@ -434,7 +440,7 @@ int select_keys_cap(int64_t k) {
 }
 
 static hipError_t launch_select_pass(const SelectKeysArgs &a, int64_t blocks, hipStream_t st) {
-    void (*fn)(SelectKeysArgs) = a.seglen <= kSelRegKeys * kSelThreads ? select_keys_kernel<true>
+    void (*fn)(SelectKeysArgs) = !a.off && a.seglen <= kSelRegKeys * kSelThreads ? select_keys_kernel<true>
                                                                        : select_keys_kernel<false>;
     const size_t lds = (size_t)a.cap * 8 + kSelBins * 4;
     if (lds > 64 * 1024) {
@@ -489,6 +495,169 @@ hipError_t launch_select_keys(const uint64_t *keys, int64_t nq, int64_t n, int64
     a.nflags = nflags;
     a.hflags = hflags;
     return launch_select_pass(a, nq, st);
+}
+
+hipError_t launch_select_groups(const uint64_t *keys, const int32_t *off, const int32_t *cnt,
+                                int64_t nq, int64_t k, int metric, float *D, int32_t *I,
+                                uint32_t *flags, hipStream_t st) {
+    if (nq <= 0) return hipSuccess;
+    const int cap = select_keys_cap(k);
+    if (!cap || k < 1 || nq > INT32_MAX || !off || !cnt || !flags) return hipErrorInvalidValue;
+    SelectKeysArgs a{};
+    a.keys = keys;
+    a.k = k;
+    a.cap = cap;
+    a.metric = metric;
+    a.nseg = 1;
+    a.off = off;
+    a.cnt = cnt;
+    a.short_flag = flags;
+    a.D = D;
+    a.I = I;
+    return launch_select_pass(a, nq, st);
+}
+
+__global__ __launch_bounds__(256) void count_pairs_kernel(const int32_t *__restrict__ cq, int64_t m,
+                                                          int64_t nq, int32_t *__restrict__ cnt) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= m) return;
+    const int32_t q = cq[t];
+    if (q >= 0 && q < nq) atomicAdd(&cnt[q], 1);
+}
+
+hipError_t launch_count_pairs(const int32_t *cq, int64_t m, int64_t nq, int32_t *cnt,
+                              hipStream_t st) {
+    if (m <= 0) return hipSuccess;
+    count_pairs_kernel<<<dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st>>>(cq, m, nq, cnt);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Exact scores of (query, row) pairs in any order.  A lane sums one pair in
+// dimension order; a wave's 64 rows and 64 query rows come through LDS in
+// 32-element chunks, eight lanes reading 128 contiguous bytes of each, with
+// the next chunk's loads in flight while one is summed.  (A lane reading its
+// own row touches 64 cache lines per load.)  One wave per workgroup: waves
+// share nothing, and 18 KB of LDS leave eight on a CU.
+// ---------------------------------------------------------------------------
+constexpr int kPairK = 32, kPairLd = kPairK + 4;
+
+template <int ST, int METRIC, typename Done>
+__device__ __forceinline__ void exact_pairs_wave(const void *xb, int64_t ld, int64_t d,
+                                                 const float *qf, const int32_t *cq,
+                                                 const int32_t *ci, int64_t m, int64_t nq,
+                                                 int64_t n, uint32_t *flags, Done &&done) {
+    __shared__ __align__(16) float xs[64][kPairLd];
+    __shared__ __align__(16) float qs[64][kPairLd];
+    __shared__ int s_q[64], s_id[64];
+    const int lane = threadIdx.x;
+    const int64_t t = (int64_t)blockIdx.x * 64 + lane;
+    bool ok = t < m;
+    int32_t q = ok ? cq[t] : 0, id = ok ? ci[t] : 0;
+    if (ok && (q < 0 || q >= nq || id < 0 || id >= n)) {
+        atomicOr(flags, kFlagBadId);
+        ok = false;
+        q = id = 0;
+    }
+    s_q[lane] = q;
+    s_id[lane] = id;
+    __syncthreads();
+    // rows: pieces of 16 bytes; queries: rows of d floats without alignment,
+    // so element by element where d is not a multiple of four
+    constexpr int PE = ST == 1 ? 8 : 4, TPR = kPairK / PE, NPR = 64 * TPR / 64;
+    u32x4_t xr[NPR];
+    float4 qr[8];
+    const bool q4 = (d & 3) == 0;
+    auto load = [&](int64_t k0) {
+#pragma unroll
+        for (int i = 0; i < NPR; ++i) {
+            const int r = i * (64 / TPR) + lane / TPR, c = (lane % TPR) * PE;
+            const int64_t e = (int64_t)s_id[r] * ld + k0 + c;
+            xr[i] = *(const u32x4_t *)((const char *)xb + e * (ST == 1 ? 2 : 4));
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int r = i * 8 + lane / 8;
+            const int64_t j = k0 + (lane % 8) * 4;
+            const float *p = qf + (int64_t)s_q[r] * d + j;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (q4) {
+                if (j < d) v = *(const float4 *)p;
+            } else {
+                if (j < d) v.x = p[0];
+                if (j + 1 < d) v.y = p[1];
+                if (j + 2 < d) v.z = p[2];
+                if (j + 3 < d) v.w = p[3];
+            }
+            qr[i] = v;
+        }
+    };
+    double s = 0.0;
+    load(0);
+    for (int64_t k0 = 0; k0 < d; k0 += kPairK) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NPR; ++i) {
+            const int r = i * (64 / TPR) + lane / TPR, c = (lane % TPR) * PE;
+            const u32x4_t p = xr[i];
+            if constexpr (ST == 1) {
+                const u32x4_t lo = {p.x << 16, p.x & 0xFFFF0000u, p.y << 16, p.y & 0xFFFF0000u};
+                const u32x4_t hi = {p.z << 16, p.z & 0xFFFF0000u, p.w << 16, p.w & 0xFFFF0000u};
+                *(u32x4_t *)&xs[r][c] = lo;
+                *(u32x4_t *)&xs[r][c + 4] = hi;
+            } else {
+                *(u32x4_t *)&xs[r][c] = p;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *(float4 *)&qs[i * 8 + lane / 8][(lane % 8) * 4] = qr[i];
+        __syncthreads();
+        if (k0 + kPairK < d) load(k0 + kPairK);
+        // (elements past d are zero on both sides: their terms add +0)
+#pragma unroll
+        for (int j = 0; j < kPairK; j += 4) {
+            const float4 xv = *(const float4 *)&xs[lane][j], qv = *(const float4 *)&qs[lane][j];
+            const float xa[4] = {xv.x, xv.y, xv.z, xv.w}, qa[4] = {qv.x, qv.y, qv.z, qv.w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if constexpr (METRIC == 0) {
+                    const double diff = (double)qa[c] - (double)xa[c];
+                    s = s + diff * diff;
+                } else {
+                    s = __builtin_fma((double)qa[c], (double)xa[c], s);
+                }
+            }
+        }
+    }
+    if (t < m) done(t, q, id, ok, s);
+}
+
+template <int ST, int METRIC>
+__global__ __launch_bounds__(64) void exact_pair_keys_kernel(
+    const void *xb, int64_t ld, int64_t d, const float *qf, const int32_t *cq, const int32_t *ci,
+    int64_t m, int64_t nq, int64_t n, const int32_t *off, int32_t *fill, uint64_t *keys,
+    uint32_t *flags) {
+    exact_pairs_wave<ST, METRIC>(
+        xb, ld, d, qf, cq, ci, m, nq, n, flags,
+        [&](int64_t, int32_t q, int32_t id, bool ok, double s) {
+            if (!ok) return;
+            const float key = METRIC == 0 ? (float)s : -(float)s;
+            keys[(int64_t)off[q] + atomicAdd(&fill[q], 1)] =
+                ((uint64_t)enc_order(key) << 32) | (uint32_t)id;
+        });
+}
+
+hipError_t launch_exact_pair_keys(const void *xb, int storage, int64_t ld, int64_t d, int metric,
+                                  const float *qf, const int32_t *cq, const int32_t *ci, int64_t m,
+                                  int64_t nq, int64_t n, const int32_t *off, int32_t *fill,
+                                  uint64_t *keys, uint32_t *flags, hipStream_t st) {
+    if (m <= 0) return hipSuccess;
+    if ((m + 63) / 64 > INT32_MAX) return hipErrorInvalidValue;
+    auto fn = storage == 1 ? (metric == 0 ? exact_pair_keys_kernel<1, 0> : exact_pair_keys_kernel<1, 1>)
+                           : (metric == 0 ? exact_pair_keys_kernel<0, 0> : exact_pair_keys_kernel<0, 1>);
+    hipLaunchKernelGGL(fn, dim3((unsigned)((m + 63) / 64)), dim3(64), 0, st, xb, ld, d, qf, cq, ci,
+                       m, nq, n, off, fill, keys, flags);
+    return hipGetLastError();
 }
 
 }  // namespace vs

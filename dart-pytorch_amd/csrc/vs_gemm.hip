@@ -274,8 +274,7 @@ __device__ __forceinline__ void gemm_epilogue(f32x16_t (&acc)[QB][RB], const Sca
             // reported: below lim, and above the query (self-join)
             const int omin =
                 a.self_join ? (int)max((int64_t)0, min((int64_t)(32 * RB), qg - wr0 + 1)) : 0;
-            // one reservation per lane for all of its hits, found as bit
-            // masks in VGPRs (no lane mask per value stays live)
+            // the lane's hits, found as bit masks in VGPRs (no lane mask per value stays live)
             uint32_t mk[RB];
             int c = 0;
 #pragma unroll
@@ -285,8 +284,19 @@ __device__ __forceinline__ void gemm_epilogue(f32x16_t (&acc)[QB][RB], const Sca
                           ~rows_below_mask(omin - rb * 32 - 4 * h);
                 c += __builtin_popcount(mk[rb]);
             }
+            // one reservation per wave (buffering the pairs in LDS as the
+            // streaming scan does spilled registers of the main loop: a
+            // 200,000 x 512 self-join went from 19.0 to 20.6 ms)
+            int inc = c;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(inc, o);
+                if (lane >= o) inc += y;
+            }
+            unsigned long long base = 0;
+            if (lane == 63 && inc > 0) base = atomicAdd(a.count, (unsigned long long)inc);
+            base = __shfl(base, 63);
             if (c > 0) {
-                unsigned long long pos = atomicAdd(a.count, (unsigned long long)c);
+                unsigned long long pos = base + (unsigned long long)(inc - c);
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
 #pragma unroll

@@ -51,6 +51,7 @@ struct PreparedQueries {
     uint16_t *qp = nullptr;  // [nq_pad][planes][ld] bf16
     float *qf = nullptr;     // [nq][d] fp32 copy of the queries as given
     float *qnorm = nullptr;  // [nq] sqrt of the fp64 sum of squares
+    float *qres = nullptr;   // [nq] |q - plane 0 / s| (an upper bound), or null
     int planes = 1;
     int64_t nq = 0, nq_pad = 0;
 };
@@ -58,7 +59,8 @@ struct PreparedQueries {
 // Status flags written by the query-preparation kernel.
 // kFlagBadId: a kernel met a candidate id outside the rows it indexes (an
 // internal error, reported instead of reading past the rows).
-enum : uint32_t { kFlagNonFinite = 1u, kFlagNotBf16 = 2u, kFlagBadId = 4u };
+// kFlagShort: a re-search found fewer than k candidates.
+enum : uint32_t { kFlagNonFinite = 1u, kFlagNotBf16 = 2u, kFlagBadId = 4u, kFlagShort = 8u };
 
 // order-preserving code of +inf (see enc_order in vs_kernels.hip)
 constexpr uint32_t kGthrInit = 0xFF800000u;
@@ -74,6 +76,12 @@ hipError_t launch_store_rows(const void *src, int src_dtype, int64_t src_stride,
                              int64_t d, void *dst, int dst_dtype, int64_t ld, float *xn,
                              uint32_t *flags, hipStream_t st);
 
+// n fp32 rows (stride ld, a multiple of 64, zero past their elements) rounded
+// to bf16 rows of stride ld16 >= ld; *res receives an upper bound on the
+// largest |row - rounded row|.
+hipError_t launch_copy_rows16(const void *src, int64_t ld, int64_t n, int64_t ld16, void *dst,
+                              float *res, hipStream_t st);
+
 // Build PreparedQueries from n query rows (src dtype / stride).
 hipError_t launch_prepare_queries(const void *src, int src_dtype, int64_t src_stride, int64_t nq,
                                   int64_t d, int64_t ld, int metric, const PreparedQueries &pq,
@@ -85,6 +93,8 @@ struct ScanPlan {
     int kk = 16;          // per-list kept candidates (power of two)
     int kk_final = 16;    // candidates kept per query by the merge (power of two, >= kk)
     int cap = 64;         // per-list buffer capacity (power of two)
+    int keep = 0;         // >0: the merge of a one-pass selection keeps this many candidates
+                          // (power of two, kk_final <= keep <= 512) of what the lists hold
     int nks = 0;          // >0: queries held in registers for this many K-steps
     int lw = 4;           // candidate lists per (workgroup, query): the workgroup's waves
     int kind = 0;         // 0: streaming scan (vs_kernels.hip);
@@ -151,7 +161,20 @@ struct TopkCheck {
     float err_g = 0.f;
     int32_t *vx_count = nullptr;
     int32_t *vx_list = nullptr;
+    // one-pass selection of fp32 rows (qres non-null): the norms of the
+    // queries' rounding residuals and the largest of a row's
+    const float *qres = nullptr;
+    float xres = 0.f;
+    // the queries' flags (or null): with kFlagNonFinite set, D and I are left
+    // alone
+    const uint32_t *qflags = nullptr;
 };
+
+// Bounds (accumulator space, as launch_range_bounds') of a re-search: athr[i]
+// = the k-th score D[list[i] k + k - 1] of prepared query i plus chk's error.
+hipError_t launch_bounded_thresholds(const PreparedQueries &pq, int64_t d, int metric,
+                                     const TopkCheck &chk, const float *D, const int32_t *list,
+                                     int64_t k, float *athr, hipStream_t st);
 
 // Merge the per-wave lists of each query, re-rank the kk survivors with the
 // exact fp64 distance and write the k best (sentinel-filled) to D / I.
@@ -219,6 +242,22 @@ hipError_t launch_select_keys(const uint64_t *keys, int64_t nq, int64_t n, int64
                               const uint32_t *rowflags, int64_t nflags, uint32_t *hflags,
                               hipStream_t st);
 
+// The same over one group of keys per query: keys[off[q] .. + cnt[q]), any
+// number; kFlagShort is set in *flags for a query with fewer than k.
+hipError_t launch_select_groups(const uint64_t *keys, const int32_t *off, const int32_t *cnt,
+                                int64_t nq, int64_t k, int metric, float *D, int32_t *I,
+                                uint32_t *flags, hipStream_t st);
+// cnt[q] += the number of pairs of query q.
+hipError_t launch_count_pairs(const int32_t *cq, int64_t m, int64_t nq, int32_t *cnt,
+                              hipStream_t st);
+// Exact keys of (query, row) pairs, grouped by query: the key of pair t goes
+// to keys[off[cq[t]] + fill[cq[t]]++].  A pair outside [0, nq) x [0, n) sets
+// kFlagBadId.
+hipError_t launch_exact_pair_keys(const void *xb, int storage, int64_t ld, int64_t d, int metric,
+                                  const float *qf, const int32_t *cq, const int32_t *ci, int64_t m,
+                                  int64_t nq, int64_t n, const int32_t *off, int32_t *fill,
+                                  uint64_t *keys, uint32_t *flags, hipStream_t st);
+
 // D / I [k] of one query by sorting its n keys (k beyond kSelectMaxK), into
 // out [n]; sentinel-filled past n.  tmp_bytes of scratch (query with tmp ==
 // nullptr).
@@ -258,10 +297,12 @@ hipError_t launch_range_refine(const void *xb, int storage, int64_t ld, int64_t 
                                double radius, float *out_s, uint8_t *keep, int64_t nrows,
                                int64_t nq, uint32_t *flags, hipStream_t st);
 
-// Per-query acceptance bounds for the range scan (accumulator space).
+// Per-query acceptance bounds for the range scan (accumulator space).  With
+// pq.qres, the operands are rounded to one bf16 plane each: xres is the
+// largest norm of a row's rounding residual.
 hipError_t launch_range_bounds(const PreparedQueries &pq, int64_t d, int metric, double radius,
-                               float xnorm_max, int exact_q, int exact_x, int coarse, float *athr,
-                               hipStream_t st);
+                               float xnorm_max, int exact_q, int exact_x, int coarse, float xres,
+                               float *athr, hipStream_t st);
 
 // Measured-peak probes: n16 16-byte loads (a read-only stream), and blocks
 // workgroups of 4 waves each running iters rounds of 8 independent

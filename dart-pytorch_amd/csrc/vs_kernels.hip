@@ -103,6 +103,57 @@ hipError_t launch_store_rows(const void *src, int src_dtype, int64_t src_stride,
 }
 
 // ---------------------------------------------------------------------------
+// bf16 copy of fp32 rows.  HBM-bound: a wave takes a row at a time, four
+// elements per lane and load, and the residuals' squares are summed beside it
+// (one atomic per workgroup on the largest).
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void copy_rows16_kernel(const float *__restrict__ src, int64_t ld,
+                                                          int64_t n, int64_t ld16,
+                                                          uint16_t *__restrict__ dst, float *res) {
+    __shared__ float wm[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float worst = 0.0f;
+    for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < n; row += (int64_t)gridDim.x * 4) {
+        float rr = 0.0f;  // (non-negative terms: off by less than ld 2^-24, covered below)
+        for (int64_t j = 4 * lane; j < ld16; j += 256) {
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (j < ld) v = *(const float4 *)(src + row * ld + j);
+            const float x[4] = {v.x, v.y, v.z, v.w};
+            uint16_t h[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                h[u] = f32_to_bf16_rne(x[u]);
+                const float e = x[u] - bf16_to_f32(h[u]);  // exact
+                rr += e * e;
+            }
+            *(u32x2_t *)(dst + row * ld16 + j) =
+                u32x2_t{(uint32_t)h[0] | (uint32_t)h[1] << 16, (uint32_t)h[2] | (uint32_t)h[3] << 16};
+        }
+        for (int o = 32; o > 0; o >>= 1) rr += __shfl_xor(rr, o);
+        worst = fmaxf(worst, rr);
+    }
+    if (lane == 0) wm[wave] = worst;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const float m = fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]));
+        // residuals whose squares leave fp32's normal range: 1e-19 at most each
+        const float r = sqrtf(m) * (1.0f + 1e-3f) + 1e-18f * (float)ld;
+        atomicMax((unsigned int *)res, __float_as_uint(r));
+    }
+}
+
+hipError_t launch_copy_rows16(const void *src, int64_t ld, int64_t n, int64_t ld16, void *dst,
+                              float *res, hipStream_t st) {
+    if (ld % 64 || ld16 % 64 || ld16 < ld) return hipErrorInvalidValue;
+    hipError_t e = launch_fill32(res, 1, 0u, st);
+    if (e != hipSuccess || n <= 0) return e;
+    const int64_t blocks = std::min<int64_t>(8192, (n + 3) / 4);
+    copy_rows16_kernel<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(
+        (const float *)src, ld, n, ld16, (uint16_t *)dst, res);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // Query preparation.  One wave per (padded) query row.
 // ---------------------------------------------------------------------------
 template <typename TS>
@@ -112,12 +163,13 @@ __global__ __launch_bounds__(256) void prep_queries_kernel(const TS *__restrict_
                                                            float scale, uint16_t *__restrict__ qp,
                                                            float *__restrict__ qf,
                                                            float *__restrict__ qnorm,
+                                                           float *__restrict__ qres,
                                                            uint32_t *flags) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= nq_pad) return;
     const bool valid = row < nq;
-    double ss = 0.0;
+    double ss = 0.0, rr = 0.0;
     uint32_t f = 0;
     for (int64_t j = lane; j < ld; j += 64) {
         const bool in = valid && j < d;
@@ -129,13 +181,16 @@ __global__ __launch_bounds__(256) void prep_queries_kernel(const TS *__restrict_
         ss += (double)v * (double)v;
         const float s = v * scale;  // scale is -1 or -2: exact
         const uint16_t h0 = f32_to_bf16_rne(s);
-        const uint16_t h1 = f32_to_bf16_rne(s - bf16_to_f32(h0));
+        const float e = s - bf16_to_f32(h0);  // exact
+        rr += (double)e * (double)e;
+        const uint16_t h1 = f32_to_bf16_rne(e);
         if (h1 & 0x7FFFu) f |= kFlagNotBf16;
         qp[(row * 2 + 0) * ld + j] = h0;
         qp[(row * 2 + 1) * ld + j] = h1;
     }
     for (int o = 32; o > 0; o >>= 1) {
         ss += __shfl_xor(ss, o);
+        rr += __shfl_xor(rr, o);
         f |= __shfl_xor(f, o);
     }
     if (f & kFlagNonFinite) {
@@ -148,9 +203,11 @@ __global__ __launch_bounds__(256) void prep_queries_kernel(const TS *__restrict_
             qp[(row * 2 + 1) * ld + j] = 0;
         }
         ss = 1.0;
+        rr = 0.0;
     }
     if (lane == 0) {
         if (valid) qnorm[row] = (float)sqrt(ss);
+        if (valid && qres) qres[row] = (float)(sqrt(rr) / -scale * (1.0 + 1e-6)) + 1e-36f;
         // one atomic per new bit: rows of the same data set the same bits, and
         // millions of atomics on one word would serialise
         if (f && (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & f) != f)
@@ -167,11 +224,11 @@ hipError_t launch_prepare_queries(const void *src, int src_dtype, int64_t src_st
     if (src_dtype == 0)
         prep_queries_kernel<float><<<grid, block, 0, st>>>((const float *)src, src_stride, nq,
                                                            pq.nq_pad, d, ld, scale, pq.qp, pq.qf,
-                                                           pq.qnorm, flags);
+                                                           pq.qnorm, pq.qres, flags);
     else
         prep_queries_kernel<uint16_t><<<grid, block, 0, st>>>((const uint16_t *)src, src_stride,
                                                               nq, pq.nq_pad, d, ld, scale, pq.qp,
-                                                              pq.qf, pq.qnorm, flags);
+                                                              pq.qf, pq.qnorm, pq.qres, flags);
     return hipGetLastError();
 }
 
@@ -522,30 +579,30 @@ __global__ __launch_bounds__(64 * NW) void scan_kernel(ScanKArgs a) {
             }
             lds_wave_sync();
         } else {
+            int c = 0;
+            auto hits = [&](auto &&f) {
 #pragma unroll
-            for (int tm = 0; tm < TM; ++tm) {
-                const int64_t rbase = t0 + tm * 16 + 4 * g;
+                for (int tm = 0; tm < TM; ++tm) {
+                    const int64_t rbase = t0 + tm * 16 + 4 * g;
 #pragma unroll
-                for (int qb = 0; qb < NQB; ++qb) {
-                    const f32x4_t v4 = acc[tm][qb];
-                    const float m4 = fminf(fminf(v4[0], v4[1]), fminf(v4[2], v4[3]));
-                    if (!__ballot(m4 <= thr_r[qb])) continue;
-                    const int64_t qg = q0 + qb * 16 + r16;
+                    for (int qb = 0; qb < NQB; ++qb) {
+                        const f32x4_t v4 = acc[tm][qb];
+                        const float m4 = fminf(fminf(v4[0], v4[1]), fminf(v4[2], v4[3]));
+                        if (!__ballot(m4 <= thr_r[qb])) continue;
+                        const int64_t qg = q0 + qb * 16 + r16;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int64_t row = rbase + i;
-                        if (v4[i] <= thr_r[qb] && (!a.self_join || row > qg)) {
-                            const unsigned long long pos = atomicAdd(a.count, 1ull);
-                            if (pos < (unsigned long long)a.out_cap) {
-                                a.out_q[pos] = (int32_t)qg;
-                                a.out_i[pos] = (int32_t)row;
-                            }
-                        }
+                        for (int i = 0; i < 4; ++i)
+                            if (v4[i] <= thr_r[qb] && (!a.self_join || rbase + i > qg))
+                                f((int)qg, (int)(rbase + i));
                     }
                 }
-            }
+            };
+            hits([&](int, int) { ++c; });
+            sink_pairs(a, c, cnt_w, (int *)sv_w, si_w, a.cap, lane, hits);
         }
     }
+
+    if constexpr (MODE == 1) flush_pairs(a, cnt_w, (const int *)sv_w, si_w, lane);
 
     if constexpr (MODE == 0) {
         if (a.list_cnt) {
@@ -688,7 +745,7 @@ hipError_t launch_scan_range(const void *xb, int storage, int64_t ld, const floa
     a.nsplit = plan.nsplit;
     a.rows_per_split = plan.rows_per_split;
     a.kk = plan.kk;
-    a.cap = plan.cap;
+    a.cap = plan.cap;  // (of the waves' pair buffers)
     a.metric = metric;
     a.kk_final = plan.kk;
     a.athr = athr;
@@ -761,8 +818,13 @@ struct MergeKArgs {
     // of the exact xn - 2 q.x (L2, s = 2, xn_max = xmax^2) or -q.x (IP,
     // s = 1, xn_max = 0).  A query whose exact k-th result does not lie
     // below (kk-th kept value - err(q)) is appended to vx_list.
+    // One-pass selection of fp32 rows (qres non-null): plus
+    // s (qres (xmax + xres) + |q| xres), the operands' rounding.
     const float *qnorm;
     float xmax, err_r, err_g;
+    const float *qres;
+    float xres;
+    const uint32_t *qflags;  // kFlagNonFinite set: D and I are left alone (or null)
     int32_t *vx_count;
     int32_t *vx_list;
     // k-means argmin mode
@@ -1031,6 +1093,7 @@ __global__ __launch_bounds__(256) void merge_refine_kernel(MergeKArgs a) {
     // candidates were still found below it.  Otherwise flag the query.
     __shared__ int s_vf;  // the query went to vf_list
     if (tid == 0) s_vf = 0;
+    __shared__ float s_lo;  // one-pass selection: the lists' lowest own threshold
     if (MODE == 0 && (a.lbound || a.guess)) {
         __shared__ float s_lmin[4];
         float lmin = VS_INF;
@@ -1049,7 +1112,10 @@ __global__ __launch_bounds__(256) void merge_refine_kernel(MergeKArgs a) {
             const float m = fminf(fminf(s_lmin[0], s_lmin[1]), fminf(s_lmin[2], s_lmin[3]));
             // (s_thr, s_thr_id): the kk-th kept pair, a sentinel if fewer were found
             const bool short_list = a.guess && s_thr_id == INT_MAX && a.nrows >= kk;
-            if (m < s_thr || short_list) {
+            s_lo = m;
+            // (the one-pass selection's proof below bounds what the lists may
+            // have dropped by their thresholds instead)
+            if (!a.qres && (m < s_thr || short_list)) {
                 a.vf_list[atomicAdd(a.vf_count, 1)] = (int32_t)qg;
                 s_vf = 1;
             }
@@ -1115,6 +1181,7 @@ __global__ __launch_bounds__(256) void merge_refine_kernel(MergeKArgs a) {
 
     if constexpr (MODE == 0) {
         bitonic_sort_block(bv, bi, kk);
+        if (a.qflags && (*a.qflags & kFlagNonFinite)) return;  // (the same for every workgroup)
         for (int64_t t = tid; t < a.k; t += 256) {
             const bool ok = t < kk && bi[t] != INT_MAX;
             a.D[qg * a.k + t] = ok ? (a.metric == 0 ? bv[t] : -bv[t])
@@ -1133,17 +1200,33 @@ __global__ __launch_bounds__(256) void merge_refine_kernel(MergeKArgs a) {
                 for (int64_t j = tid; j < a.d; j += 64) qq += (double)qsh[j] * (double)qsh[j];
                 for (int o = 32; o > 0; o >>= 1) qq += __shfl_xor(qq, o);
             }
-            if (tid == 0 && !s_vf && bi[a.k - 1] != INT_MAX && s_thr < VS_INF) {
+            // (an operand past bf16's range leaves accumulators that are not
+            // numbers, and fewer candidates than rows)
+            // One-pass selection: rows the merge does not hold lie at or above
+            // its kk-th value, the query's final shared threshold or their
+            // list's own, whichever is lowest.
+            float dropped = s_thr;
+            if (a.qres) {
+                dropped = fminf(dropped, tfinal);
+                if (a.lbound || a.guess) dropped = fminf(dropped, s_lo);
+            }
+            const bool lost = a.qres && (bi[a.k - 1] == INT_MAX ? a.nrows >= a.k
+                                                                : dropped == VS_INF && a.nrows >= kk);
+            if (tid == 0 && !s_vf && lost) {
+                a.vf_list[atomicAdd(a.vf_count, 1)] = (int32_t)qg;
+            } else if (tid == 0 && !s_vf && bi[a.k - 1] != INT_MAX && dropped < VS_INF) {
                 const double s = a.metric == 0 ? 2.0 : 1.0;
                 const double qn = a.qnorm[qg], xm = a.xmax;
-                const double err = 1.25 * ((double)a.err_r * s * qn * xm +
-                                           (double)a.err_g * ((a.metric == 0 ? xm * xm : 0.0) +
-                                                              s * qn * xm)) +
-                                   1e-30;
+                double err = 1.25 * ((double)a.err_r * s * qn * xm +
+                                     (double)a.err_g * ((a.metric == 0 ? xm * xm : 0.0) +
+                                                        s * qn * xm)) +
+                             1e-30;
+                // (1.00001: the norms are rounded to fp32)
+                if (a.qres) err += 1.00001 * s * ((double)a.qres[qg] * (xm + a.xres) + qn * a.xres);
                 const double key = bv[a.k - 1];
                 double ek = key + fabs(key) * (1.0 / 8388608.0);
                 if (a.metric == 0) ek -= qq * (1.0 - 1e-12);  // qq: fp64 sum, error < d 2^-53 qq
-                if (!(ek < (double)s_thr - err)) a.vx_list[atomicAdd(a.vx_count, 1)] = (int32_t)qg;
+                if (!(ek < (double)dropped - err)) a.vx_list[atomicAdd(a.vx_count, 1)] = (int32_t)qg;
             }
         }
     } else {
@@ -1226,11 +1309,12 @@ static hipError_t launch_merge_passes(void (*fn)(MergeKArgs), size_t lds, MergeK
         hipLaunchKernelGGL(fn, dim3((unsigned)nq), dim3(256), lds, st, a);
         return hipGetLastError();
     }
-    if (plan.kk_final % 4 || nq * g > INT32_MAX) return hipErrorInvalidValue;
+    const int keep = a.kk;
+    if (keep % 4 || nq * g > INT32_MAX) return hipErrorInvalidValue;
     const int64_t off = plan.nqblk * plan.nsplit * plan.lw * plan.bn * plan.cap;
     MergeKArgs a1 = a;
     a1.part_g = g;
-    a1.part_cap = plan.kk_final;
+    a1.part_cap = keep;
     a1.part_v = cand_v + off;
     a1.part_i = cand_i + off;
     hipLaunchKernelGGL(fn, dim3((unsigned)(nq * g)), dim3(256), lds, st, a1);
@@ -1242,8 +1326,8 @@ static hipError_t launch_merge_passes(void (*fn)(MergeKArgs), size_t lds, MergeK
     a2.bn = 1;
     a2.lw = 1;
     a2.nsplit = g;
-    a2.cap = plan.kk_final;
-    a2.kl = plan.kk_final;
+    a2.cap = keep;
+    a2.kl = keep;
     hipLaunchKernelGGL(fn, dim3((unsigned)nq), dim3(256), lds, st, a2);
     return hipGetLastError();
 }
@@ -1263,6 +1347,9 @@ hipError_t launch_merge_refine(const void *xb, int storage, int64_t ld, int64_t 
         a.xmax = chk->xmax;
         a.err_r = chk->err_r;
         a.err_g = chk->err_g;
+        a.qres = chk->qres;
+        a.xres = chk->xres;
+        a.qflags = chk->qflags;
         a.vx_count = chk->vx_count;
         a.vx_list = chk->vx_list;
     }
@@ -1279,7 +1366,7 @@ hipError_t launch_merge_refine(const void *xb, int storage, int64_t ld, int64_t 
     a.nq = pq.nq;
     a.bn = plan.bn;
     a.lw = plan.lw;
-    a.kk = plan.kk_final;
+    a.kk = plan.keep ? plan.keep : plan.kk_final;
     a.kl = a.list_cnt ? plan.cap : plan.kk;
     a.nlists_all = plan.nqblk * plan.nsplit * plan.lw * plan.bn;
 
@@ -2490,14 +2577,18 @@ hipError_t launch_exclusive_scan_i32(const int32_t *in, int64_t n, int32_t *out,
 // with |acc - exact| <= err(q) = c * |q| * max|x| (+ the norm rounding for
 // L2).  The scan keeps acc <= athr, athr = exact bound + err, and the exact
 // fp64 re-test decides.
-__global__ void range_bounds_kernel(const float *__restrict__ qnorm, int64_t nq, int metric,
-                                    double radius, float xmax, float rel, float *athr) {
+__global__ void range_bounds_kernel(const float *__restrict__ qnorm,
+                                    const float *__restrict__ qres, int64_t nq, int metric,
+                                    double radius, float xmax, float xres, float rel, float *athr) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nq) return;
     const double qn = qnorm[i];
     const double xm = xmax;
-    const double err =
+    double err =
         metric == 0 ? (double)rel * (2.0 * qn * xm + qn * qn + xm * xm) : (double)rel * qn * xm;
+    // both operands rounded to bf16 (1.00001: the norms are rounded to fp32)
+    if (qres)
+        err += 1.00001 * (metric == 0 ? 2.0 : 1.0) * ((double)qres[i] * (xm + xres) + qn * xres);
     double t;
     if (metric == 0)
         t = radius - qn * qn + err;
@@ -2507,8 +2598,8 @@ __global__ void range_bounds_kernel(const float *__restrict__ qnorm, int64_t nq,
 }
 
 hipError_t launch_range_bounds(const PreparedQueries &pq, int64_t d, int metric, double radius,
-                               float xnorm_max, int exact_q, int exact_x, int coarse, float *athr,
-                               hipStream_t st) {
+                               float xnorm_max, int exact_q, int exact_x, int coarse, float xres,
+                               float *athr, hipStream_t st) {
     if (pq.nq <= 0) return hipSuccess;
     // relative error of the split-bf16 dot product with fp32 accumulation:
     // products: each operand within 2^-16 relative of its value (hi + lo),
@@ -2524,7 +2615,49 @@ hipError_t launch_range_bounds(const PreparedQueries &pq, int64_t d, int metric,
     if (!exact_q) rel += 4.0 / 65536.0;
     if (coarse) rel += 4.0 / 256.0;
     range_bounds_kernel<<<dim3((unsigned)((pq.nq + 255) / 256)), dim3(256), 0, st>>>(
-        pq.qnorm, pq.nq, metric, radius, xnorm_max, (float)rel, athr);
+        pq.qnorm, pq.qres, pq.nq, metric, radius, xnorm_max, xres, (float)rel, athr);
+    return hipGetLastError();
+}
+
+// Bounds of a re-search, one wave per query: the k-th result's exact
+// accumulator plus the error bound of the merge's proof (merge_refine_kernel).
+__global__ __launch_bounds__(256) void bounded_thr_kernel(
+    const float *__restrict__ qf, const float *__restrict__ qnorm, const float *__restrict__ qres,
+    int64_t m, int64_t d, int metric, float xmax, float xres, float err_r, float err_g,
+    const float *__restrict__ D, const int32_t *__restrict__ list, int64_t k,
+    float *__restrict__ athr) {
+    const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (q >= m) return;
+    double qq = 0.0;
+    if (metric == 0) {
+        for (int64_t j = lane; j < d; j += 64) qq += (double)qf[q * d + j] * (double)qf[q * d + j];
+        for (int o = 32; o > 0; o >>= 1) qq += __shfl_xor(qq, o);
+    }
+    if (lane) return;
+    const double s = metric == 0 ? 2.0 : 1.0;
+    const double qn = qnorm[q], xm = xmax;
+    double err = 1.25 * ((double)err_r * s * qn * xm +
+                         (double)err_g * ((metric == 0 ? xm * xm : 0.0) + s * qn * xm)) +
+                 1e-30;
+    if (qres) err += 1.00001 * s * ((double)qres[q] * (xm + xres) + qn * xres);
+    const double score = D[(int64_t)list[q] * k + k - 1];
+    const double key = metric == 0 ? score : -score;
+    double ek = key + fabs(key) * (1.0 / 8388608.0);
+    if (metric == 0) ek -= qq * (1.0 - 1e-12);
+    const float t = (float)(ek + err), b = t + fabsf(t) * 1e-6f + 1e-30f;
+    // no finite bound (norms past fp32's range): no candidates, which sends
+    // the query on to the exact path
+    athr[q] = __builtin_isfinite(b) ? b : -VS_INF;
+}
+
+hipError_t launch_bounded_thresholds(const PreparedQueries &pq, int64_t d, int metric,
+                                     const TopkCheck &chk, const float *D, const int32_t *list,
+                                     int64_t k, float *athr, hipStream_t st) {
+    if (pq.nq <= 0) return hipSuccess;
+    bounded_thr_kernel<<<dim3((unsigned)((pq.nq + 3) / 4)), dim3(256), 0, st>>>(
+        pq.qf, pq.qnorm, chk.qres ? pq.qres : nullptr, pq.nq, d, metric, chk.xmax, chk.xres,
+        chk.err_r, chk.err_g, D, list, k, athr);
     return hipGetLastError();
 }
 

@@ -56,6 +56,9 @@ enum { VS_DTYPE_F32 = 0, VS_DTYPE_BF16 = 1 };
 
 /* Storage of the database rows in HBM.
  *   F32  -- fp32, as IndexFlat's Float32List storage (index_flat.dart:20);
+ *           searches and joins also keep a bf16 copy of the rows to select
+ *           candidates from, where it takes at most a quarter of the free
+ *           device memory (given back when an allocation needs it);
  *   BF16 -- bf16; fp32 input rows are rounded to nearest-even once at add;
  *   AUTO -- bf16 while every stored value is exactly a bf16 value (then
  *           results are those of fp32 storage), fp32 otherwise; the switch
@@ -270,9 +273,10 @@ VS_API int vs_index_sync(vs_index *idx);
  *   "gemm4"       1: the four-wave pipelined GEMM-tiled kernel where it applies (bf16
  *                 rows, one query plane; shape 2,2,4,4,32); 0 (default): the eight-wave one
  *   "share"       -1 rule (bf16 rows of 128 elements, batch >= 256), 0 off, 1 also 256
- *   "coarse"      1: one-pass bf16 selection of fp32 rows (range, self-join, k-means)
- *   "copy16"      1: that selection reads a bf16 copy of the rows
- *   "guess"       1: large batches start from thresholds estimated on a row sample
+ *   "coarse"      1: one-pass bf16 selection of fp32 rows (search, range, self-join, k-means)
+ *   "copy16"      1: that selection reads a bf16 copy of the rows (search: needs it)
+ *   "guess"       1: batches of 16 queries and more (256 from 2^18 rows) start from thresholds
+ *                 estimated on a row sample
  *   "prepass"     1: small batches seed their thresholds from a pre-pass
  *   "prepass_log2" 10..20: that pre-pass scans at least 2^value rows (default 16)
  *   "scan_kkw"    >0: per-list keep forced down (exercises the list verification)
