@@ -227,7 +227,7 @@ struct vs_index {
     size_t lds_max = 64 * 1024;
     // scratch (grown on demand, reused across calls)
     DevBuf stage, qp, qf, qnorm, flags, cand_v, cand_i, lcnt, gthr, lbound, vf, fbq, fbD, fbI, outD, outI,
-        athr, rq, ri, rs, rkeep, rcount, misc;
+        athr, rq, ri, rs, rtmp, rcount, misc;
     DevBuf km_cen16, km_c16n;  // k-means: bf16 copy of the centroid rows (and its unused norms)
     DevBuf km_cen, km_cxn, km_assign, km_best, km_fb, km_keys, km_order, km_tmp, km_counts,
         km_offsets, km_out, km_iota;
@@ -1712,19 +1712,43 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
     }
 }
 
+// Hits of a range search or self-join in malloc'ed arrays, sorted by (query,
+// id): n ids and scores, the queries too for a self-join, and for a range
+// search the nq + 1 limits.  What is not taken out is freed.
 struct RangeHits {
-    std::vector<int32_t> q, id;
-    std::vector<float> s;
+    int64_t n = 0;
+    int32_t *q = nullptr, *id = nullptr;
+    float *s = nullptr;
+    int64_t *lims = nullptr;
+    RangeHits() = default;
+    RangeHits(const RangeHits &) = delete;
+    RangeHits &operator=(const RangeHits &) = delete;
+    ~RangeHits() {
+        free(q);
+        free(id);
+        free(s);
+        free(lims);
+    }
+    // (no array is null, as the callers' results have none)
+    int alloc(int64_t hits, int64_t nlims, bool queries) {
+        n = hits;
+        const size_t m = (size_t)std::max<int64_t>(hits, 1);
+        id = (int32_t *)malloc(m * 4);
+        s = (float *)malloc(m * 4);
+        if (queries) q = (int32_t *)malloc(m * 4);
+        if (nlims) lims = (int64_t *)calloc((size_t)nlims, 8);
+        if (!id || !s || (queries && !q) || (nlims && !lims))
+            return set_err(VS_ERR_OOM, "host allocation");
+        return VS_OK;
+    }
 };
 
 // Candidate scan + exact re-test of nq query rows (device, `stride` elements
-// apart); hits sorted by (query, id).
+// apart).
 int range_core(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int64_t nq,
                double radius, int self_join, RangeHits *out) {
-    out->q.clear();
-    out->id.clear();
-    out->s.clear();
-    if (nq == 0 || x->ntotal == 0) return VS_OK;
+    const int64_t nlims = self_join ? 0 : nq + 1;
+    if (nq == 0 || x->ntotal == 0) return out->alloc(0, nlims, self_join != 0);
     select_rows(x);
     // One-pass selection of fp32 rows: the acceptance bounds widen to the
     // operands' rounding to bf16 and every hit is re-tested exactly.  It
@@ -1761,67 +1785,82 @@ int range_core(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int6
     VS_HIP(vs::launch_range_bounds(pq, x->d, x->metric, radius, xmax, exact_q, exact_x, coarse,
                                    copy ? x->copy_res : 0.f, x->athr.as<float>(), x->st),
            "range bounds");
-    VS_HIP(x->rcount.ensure(sizeof(unsigned long long)), "range counter");
+    VS_HIP(x->rcount.ensure(16), "range counter");
+    unsigned long long *count = x->rcount.as<unsigned long long>();  // candidates, then hits
+    VS_HIP(x->hio.ensure(kCtlBytes), "control words");
+    volatile unsigned long long *hcount = (unsigned long long *)(x->hio.as<char>() + 64);
     int64_t cap = std::max<int64_t>(1 << 20, pq.nq * 4);
-    unsigned long long found = 0;
     for (int attempt = 0; attempt < 2; ++attempt) {
         VS_HIP(x->rq.ensure((size_t)cap * 4), "range candidates");
         VS_HIP(x->ri.ensure((size_t)cap * 4), "range candidates");
-        VS_HIP(hipMemsetAsync(x->rcount.p, 0, sizeof(unsigned long long), x->st), "range counter");
+        VS_HIP(vs::launch_fill32(count, 4, 0u, x->st), "range counter");
         note_scan_kind(x, plan);
         {
             ProfScope ps(x, self_join ? "join" : "range");
             VS_HIP(vs::launch_scan_range(x->sel.rows, x->sel.storage, x->sel.ld, x->xn, x->ntotal,
                                          pq, plan, x->athr.as<float>(), self_join, x->metric,
-                                         x->rq.as<int32_t>(), x->ri.as<int32_t>(),
-                                         x->rcount.as<unsigned long long>(), cap, x->st),
+                                         x->rq.as<int32_t>(), x->ri.as<int32_t>(), count, cap,
+                                         x->st),
                    "range scan");
         }
-        VS_HIP(hipMemcpyAsync(&found, x->rcount.p, sizeof found, hipMemcpyDeviceToHost, x->st),
+        VS_HIP(hipMemcpyAsync((void *)hcount, count, 8, hipMemcpyDeviceToHost, x->st),
                "range count");
         VS_HIP(hipStreamSynchronize(x->st), "range scan");
-        if ((int64_t)found <= cap) break;
-        cap = (int64_t)found;  // second pass stores everything
+        if ((int64_t)*hcount <= cap) break;
+        cap = (int64_t)*hcount;  // second pass stores everything
     }
-    const int64_t m = (int64_t)found;
-    if (m == 0) return VS_OK;
-    VS_HIP(x->rs.ensure((size_t)m * 4), "range scores");
-    VS_HIP(x->rkeep.ensure((size_t)m), "range flags");
+    const int64_t m = (int64_t)*hcount;
+    if (m == 0) return out->alloc(0, nlims, self_join != 0);
+    // exact scores and sort keys (query << idbits | id; a candidate that fails
+    // the exact test sorts last), then the hits in order on the device
+    int idbits = 1, qbits = 1;
+    while (((int64_t)1 << idbits) < x->ntotal) ++idbits;
+    while (((int64_t)1 << qbits) < nq) ++qbits;
+    const int bits = idbits + qbits + 1;
+    size_t tmp_bytes = 0;
+    VS_HIP(vs::sort_pairs_u64(nullptr, tmp_bytes, nullptr, nullptr, nullptr, nullptr, m, bits, x->st),
+           "sort size");
+    VS_HIP(x->ex_keys.ensure((size_t)m * 16), "range keys");
+    VS_HIP(x->rs.ensure((size_t)m * 8), "range scores");
+    VS_HIP(x->rtmp.ensure(tmp_bytes + (size_t)nlims * 8 + 256), "range sort");
+    uint64_t *keys = x->ex_keys.as<uint64_t>(), *sorted = keys + m;
+    float *score = x->rs.as<float>(), *sscore = score + m;
+    int64_t *lims = x->rtmp.as<int64_t>();
     {
         ProfScope ps(x, "refine");
-        VS_HIP(hipMemsetAsync(x->flags.p, 0, sizeof(uint32_t), x->st), "clearing flags");
-        VS_HIP(vs::launch_range_refine(x->xb, x->storage, x->ld, x->d, x->metric, pq.qf,
-                                       x->rq.as<int32_t>(), x->ri.as<int32_t>(), m, radius,
-                                       x->rs.as<float>(), x->rkeep.as<uint8_t>(), x->ntotal, pq.nq,
-                                       x->flags.as<uint32_t>(), x->st),
+        VS_HIP(vs::launch_fill32(x->flags.p, 1, 0u, x->st), "clearing flags");
+        VS_HIP(vs::launch_range_keys(x->xb, x->storage, x->ld, x->d, x->metric, pq.qf,
+                                     x->rq.as<int32_t>(), x->ri.as<int32_t>(), m, radius, idbits,
+                                     keys, score, count + 1, x->ntotal, pq.nq,
+                                     x->flags.as<uint32_t>(), x->st),
                "range refine");
+        VS_HIP(vs::sort_pairs_u64((void *)(lims + nlims), tmp_bytes, keys, sorted, score, sscore, m,
+                                  bits, x->st),
+               "range sort");
+        // (the candidates' buffers hold the sorted queries and ids next)
+        VS_HIP(vs::launch_range_unpack(sorted, m, idbits, x->rq.as<int32_t>(), x->ri.as<int32_t>(),
+                                       nlims, lims, x->st),
+               "range results");
     }
-    std::vector<int32_t> cq(m), ci(m);
-    std::vector<float> cs(m);
-    std::vector<uint8_t> keep(m);
-    VS_HIP(hipMemcpyAsync(cq.data(), x->rq.p, (size_t)m * 4, hipMemcpyDeviceToHost, x->st), "D2H");
-    VS_HIP(hipMemcpyAsync(ci.data(), x->ri.p, (size_t)m * 4, hipMemcpyDeviceToHost, x->st), "D2H");
-    VS_HIP(hipMemcpyAsync(cs.data(), x->rs.p, (size_t)m * 4, hipMemcpyDeviceToHost, x->st), "D2H");
-    VS_HIP(hipMemcpyAsync(keep.data(), x->rkeep.p, (size_t)m, hipMemcpyDeviceToHost, x->st), "D2H");
-    uint32_t rflags = 0;
-    VS_HIP(hipMemcpyAsync(&rflags, x->flags.p, sizeof rflags, hipMemcpyDeviceToHost, x->st), "D2H");
+    VS_HIP(hipMemcpyAsync((void *)hcount, count + 1, 8, hipMemcpyDeviceToHost, x->st), "hit count");
+    volatile uint32_t *hflags = (uint32_t *)(x->hio.as<char>() + 72);
+    VS_HIP(hipMemcpyAsync((void *)hflags, x->flags.p, 4, hipMemcpyDeviceToHost, x->st),
+           "range flags");
     VS_HIP(hipStreamSynchronize(x->st), "range results");
-    if (rflags & vs::kFlagBadId)
+    if (*hflags & vs::kFlagBadId)
         return set_err(VS_ERR_HIP, "internal error: a range candidate outside the index");
-    std::vector<int64_t> idx;
-    idx.reserve(m);
-    for (int64_t t = 0; t < m; ++t)
-        if (keep[t]) idx.push_back(t);
-    std::sort(idx.begin(), idx.end(), [&](int64_t a, int64_t b) {
-        return cq[a] != cq[b] ? cq[a] < cq[b] : ci[a] < ci[b];
-    });
-    out->q.resize(idx.size());
-    out->id.resize(idx.size());
-    out->s.resize(idx.size());
-    for (size_t t = 0; t < idx.size(); ++t) {
-        out->q[t] = cq[idx[t]];
-        out->id[t] = ci[idx[t]];
-        out->s[t] = cs[idx[t]];
+    const int64_t hits = (int64_t)*hcount;
+    if ((rc = out->alloc(hits, nlims, self_join != 0))) return rc;
+    if (hits > 0) {
+        const size_t hb = (size_t)hits * 4;
+        VS_HIP(hipMemcpyAsync(out->id, x->ri.p, hb, hipMemcpyDeviceToHost, x->st), "hits");
+        VS_HIP(hipMemcpyAsync(out->s, sscore, hb, hipMemcpyDeviceToHost, x->st), "hits");
+        if (self_join)
+            VS_HIP(hipMemcpyAsync(out->q, x->rq.p, hb, hipMemcpyDeviceToHost, x->st), "hits");
+        else
+            VS_HIP(hipMemcpyAsync(out->lims, lims, (size_t)nlims * 8, hipMemcpyDeviceToHost, x->st),
+                   "limits");
+        VS_HIP(hipStreamSynchronize(x->st), "range results");
     }
     return VS_OK;
 }
@@ -1957,7 +1996,7 @@ void vs_index_destroy(vs_index *x) {
     DevBuf *bufs[] = {&x->stage,   &x->qp,        &x->qf,       &x->qnorm,    &x->flags, &x->gthr,
                       &x->lbound,  &x->vf,        &x->fbq,      &x->fbD,      &x->fbI,
                       &x->cand_v,  &x->cand_i,    &x->outD,     &x->outI,     &x->athr,
-                      &x->rq,      &x->ri,        &x->rs,       &x->rkeep,    &x->rcount,
+                      &x->rq,      &x->ri,        &x->rs,       &x->rtmp,     &x->rcount,
                       &x->misc,    &x->km_cen,    &x->km_cxn,   &x->km_assign, &x->km_best,
                       &x->km_fb,   &x->km_keys,   &x->km_order, &x->km_tmp,   &x->km_counts,
                       &x->km_offsets, &x->km_out, &x->km_iota, &x->lcnt,   &x->km_qp,
@@ -2262,26 +2301,14 @@ int vs_index_range_search(vs_index *x, const void *q, int q_dtype, int64_t nq, d
         VS_HIP(x->stage.ensure(qbytes), "query staging");
         VS_HIP(hipMemcpyAsync(x->stage.p, q, qbytes, hipMemcpyHostToDevice, x->st),
                "uploading queries");
-        int rc = range_core(x, x->stage.p, q_dtype, x->d, nq, radius, 0, &hits);
-        if (rc) return rc;
     }
+    if (int rc = range_core(x, x->stage.p, q_dtype, x->d, nq, radius, 0, &hits)) return rc;
     vs_range_result *r = (vs_range_result *)calloc(1, sizeof(vs_range_result));
     if (!r) return set_err(VS_ERR_OOM, "host allocation");
-    const size_t m = hits.q.size();
     r->nq = nq;
-    r->lims = (int64_t *)calloc((size_t)nq + 1, sizeof(int64_t));
-    r->D = (float *)malloc(std::max<size_t>(m, 1) * sizeof(float));
-    r->I = (int32_t *)malloc(std::max<size_t>(m, 1) * sizeof(int32_t));
-    if (!r->lims || !r->D || !r->I) {
-        vs_range_result_free(r);
-        return set_err(VS_ERR_OOM, "host allocation");
-    }
-    for (size_t t = 0; t < m; ++t) r->lims[hits.q[t] + 1]++;
-    for (int64_t qi = 0; qi < nq; ++qi) r->lims[qi + 1] += r->lims[qi];
-    if (m) {
-        memcpy(r->D, hits.s.data(), m * sizeof(float));
-        memcpy(r->I, hits.id.data(), m * sizeof(int32_t));
-    }
+    std::swap(r->lims, hits.lims);
+    std::swap(r->D, hits.s);
+    std::swap(r->I, hits.id);
     *out = r;
     return VS_OK;
 }
@@ -2463,26 +2490,15 @@ int vs_index_self_join(vs_index *x, double threshold, vs_pairs **out) {
     if (!std::isfinite(threshold)) return set_err(VS_ERR_INVALID, "threshold must be finite");
     DeviceGuard g(x->device);
     RangeHits hits;
-    if (x->ntotal > 1) {
-        int rc = range_core(x, x->xb, x->storage, x->ld, x->ntotal, threshold, 1, &hits);
-        if (rc) return rc;
-    }
+    if (int rc = range_core(x, x->xb, x->storage, x->ld, x->ntotal > 1 ? x->ntotal : 0, threshold, 1,
+                            &hits))
+        return rc;
     vs_pairs *p = (vs_pairs *)calloc(1, sizeof(vs_pairs));
     if (!p) return set_err(VS_ERR_OOM, "host allocation");
-    const size_t m = hits.q.size();
-    p->npairs = (int64_t)m;
-    p->i = (int32_t *)malloc(std::max<size_t>(m, 1) * 4);
-    p->j = (int32_t *)malloc(std::max<size_t>(m, 1) * 4);
-    p->s = (float *)malloc(std::max<size_t>(m, 1) * 4);
-    if (!p->i || !p->j || !p->s) {
-        vs_pairs_free(p);
-        return set_err(VS_ERR_OOM, "host allocation");
-    }
-    if (m) {
-        memcpy(p->i, hits.q.data(), m * 4);
-        memcpy(p->j, hits.id.data(), m * 4);
-        memcpy(p->s, hits.s.data(), m * 4);
-    }
+    p->npairs = hits.n;
+    std::swap(p->i, hits.q);
+    std::swap(p->j, hits.id);
+    std::swap(p->s, hits.s);
     *out = p;
     return VS_OK;
 }

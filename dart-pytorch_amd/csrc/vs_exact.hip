@@ -660,4 +660,68 @@ hipError_t launch_exact_pair_keys(const void *xb, int storage, int64_t ld, int64
     return hipGetLastError();
 }
 
+// Range candidates: score, sort key and test of each pair.
+template <int ST, int METRIC>
+__global__ __launch_bounds__(64) void range_keys_kernel(
+    const void *xb, int64_t ld, int64_t d, const float *qf, const int32_t *cq, const int32_t *ci,
+    int64_t m, double radius, int idbits, uint64_t *keys, float *score, unsigned long long *kept,
+    int64_t n, int64_t nq, uint32_t *flags) {
+    exact_pairs_wave<ST, METRIC>(
+        xb, ld, d, qf, cq, ci, m, nq, n, flags,
+        [&](int64_t t, int32_t q, int32_t id, bool ok, double s) {
+            const bool hit = ok && (METRIC == 0 ? s <= radius : s >= radius);
+            keys[t] = hit ? (uint64_t)q << idbits | (uint32_t)id : ~0ull;
+            score[t] = (float)s;
+            const uint64_t hits = __ballot(hit);
+            if (hits && (int)threadIdx.x == __builtin_ctzll(hits))
+                atomicAdd(kept, (unsigned long long)__builtin_popcountll(hits));
+        });
+}
+
+hipError_t launch_range_keys(const void *xb, int storage, int64_t ld, int64_t d, int metric,
+                             const float *qf, const int32_t *cq, const int32_t *ci, int64_t m,
+                             double radius, int idbits, uint64_t *keys, float *score,
+                             unsigned long long *kept, int64_t n, int64_t nq, uint32_t *flags,
+                             hipStream_t st) {
+    if (m <= 0) return hipSuccess;
+    if ((m + 63) / 64 > INT32_MAX) return hipErrorInvalidValue;
+    auto fn = storage == 1 ? (metric == 0 ? range_keys_kernel<1, 0> : range_keys_kernel<1, 1>)
+                           : (metric == 0 ? range_keys_kernel<0, 0> : range_keys_kernel<0, 1>);
+    hipLaunchKernelGGL(fn, dim3((unsigned)((m + 63) / 64)), dim3(64), 0, st, xb, ld, d, qf, cq, ci,
+                       m, radius, idbits, keys, score, kept, n, nq, flags);
+    return hipGetLastError();
+}
+
+__global__ __launch_bounds__(256) void range_unpack_kernel(const uint64_t *__restrict__ sorted,
+                                                           int64_t m, int idbits,
+                                                           int32_t *__restrict__ q,
+                                                           int32_t *__restrict__ id, int64_t nlims,
+                                                           int64_t *__restrict__ lims) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t < m) {
+        const uint64_t k = sorted[t];
+        q[t] = (int32_t)(k >> idbits);
+        id[t] = (int32_t)(k & (((uint64_t)1 << idbits) - 1));
+    }
+    if (t < nlims) {  // the first key of query t or a later one
+        const uint64_t key = (uint64_t)t << idbits;
+        int64_t lo = 0, hi = m;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if (sorted[mid] < key) lo = mid + 1;
+            else hi = mid;
+        }
+        lims[t] = lo;
+    }
+}
+
+hipError_t launch_range_unpack(const uint64_t *sorted, int64_t m, int idbits, int32_t *q,
+                               int32_t *id, int64_t nlims, int64_t *lims, hipStream_t st) {
+    const int64_t t = std::max(m, nlims);
+    if (t <= 0) return hipSuccess;
+    range_unpack_kernel<<<dim3((unsigned)((t + 255) / 256)), dim3(256), 0, st>>>(sorted, m, idbits,
+                                                                               q, id, nlims, lims);
+    return hipGetLastError();
+}
+
 }  // namespace vs

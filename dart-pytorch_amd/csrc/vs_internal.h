@@ -290,12 +290,22 @@ hipError_t launch_scan_range(const void *xb, int storage, int64_t ld, const floa
                              int self_join, int metric, int32_t *out_q, int32_t *out_i,
                              unsigned long long *count, int64_t cap, hipStream_t st);
 
-// Exact fp64 re-test of range candidates: s = fp64 score of (q, id); keep[j]
-// = s <= radius (L2) or s >= radius (IP); out_s[j] = fp32(s).
-hipError_t launch_range_refine(const void *xb, int storage, int64_t ld, int64_t d, int metric,
-                               const float *qf, const int32_t *cq, const int32_t *ci, int64_t m,
-                               double radius, float *out_s, uint8_t *keep, int64_t nrows,
-                               int64_t nq, uint32_t *flags, hipStream_t st);
+// Exact fp64 re-test of range candidates: score[t] = fp32 of the fp64 score
+// of pair t; keys[t] = cq[t] << idbits | ci[t] where it passes the radius (<=
+// for L2, >= for IP), all ones elsewhere; *kept += the number that pass.
+hipError_t launch_range_keys(const void *xb, int storage, int64_t ld, int64_t d, int metric,
+                             const float *qf, const int32_t *cq, const int32_t *ci, int64_t m,
+                             double radius, int idbits, uint64_t *keys, float *score,
+                             unsigned long long *kept, int64_t n, int64_t nq, uint32_t *flags,
+                             hipStream_t st);
+// Sorted keys to queries and ids, and (nlims > 0) lims[q] = the number of
+// hits of queries below q, q < nlims.
+hipError_t launch_range_unpack(const uint64_t *sorted, int64_t m, int idbits, int32_t *q,
+                               int32_t *id, int64_t nlims, int64_t *lims, hipStream_t st);
+// Sort of (64-bit key, fp32 value) pairs by the keys' low `bits` bits (query
+// tmp_bytes with tmp == nullptr).
+hipError_t sort_pairs_u64(void *tmp, size_t &tmp_bytes, const uint64_t *kin, uint64_t *kout,
+                          const float *vin, float *vout, int64_t n, int bits, hipStream_t st);
 
 // Per-query acceptance bounds for the range scan (accumulator space).  With
 // pq.qres, the operands are rounded to one bf16 plane each: xres is the

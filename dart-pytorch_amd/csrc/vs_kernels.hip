@@ -2661,53 +2661,6 @@ hipError_t launch_bounded_thresholds(const PreparedQueries &pq, int64_t d, int m
     return hipGetLastError();
 }
 
-template <int ST>
-__global__ void range_refine_kernel(const void *xb, int64_t ld, int64_t d, int metric,
-                                    const float *__restrict__ qf, const int32_t *__restrict__ cq,
-                                    const int32_t *__restrict__ ci, int64_t m, double radius,
-                                    float *__restrict__ out_s, uint8_t *__restrict__ keep,
-                                    int64_t nrows, int64_t nq, uint32_t *flags) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= m) return;
-    const int64_t q = cq[t], id = ci[t];
-    if (q < 0 || q >= nq || id < 0 || id >= nrows) {
-        atomicOr(flags, kFlagBadId);
-        out_s[t] = 0.f;
-        keep[t] = 0;
-        return;
-    }
-    const float *qrow = qf + q * d;
-    double s = 0.0;
-    for (int64_t j = 0; j < d; ++j) {
-        const double xv = ST == 1 ? (double)bf16_to_f32(((const uint16_t *)xb)[id * ld + j])
-                                  : (double)((const float *)xb)[id * ld + j];
-        const double qv = (double)qrow[j];
-        if (metric == 0) {
-            const double diff = qv - xv;
-            s = s + diff * diff;
-        } else {
-            s = s + qv * xv;
-        }
-    }
-    out_s[t] = (float)s;
-    keep[t] = metric == 0 ? (s <= radius) : (s >= radius);
-}
-
-hipError_t launch_range_refine(const void *xb, int storage, int64_t ld, int64_t d, int metric,
-                               const float *qf, const int32_t *cq, const int32_t *ci, int64_t m,
-                               double radius, float *out_s, uint8_t *keep, int64_t nrows,
-                               int64_t nq, uint32_t *flags, hipStream_t st) {
-    if (m <= 0) return hipSuccess;
-    const dim3 grid((unsigned)((m + 255) / 256)), block(256);
-    if (storage == 1)
-        range_refine_kernel<1><<<grid, block, 0, st>>>(xb, ld, d, metric, qf, cq, ci, m, radius,
-                                                       out_s, keep, nrows, nq, flags);
-    else
-        range_refine_kernel<0><<<grid, block, 0, st>>>(xb, ld, d, metric, qf, cq, ci, m, radius,
-                                                       out_s, keep, nrows, nq, flags);
-    return hipGetLastError();
-}
-
 __global__ __launch_bounds__(256) void max_reduce_kernel(const float *__restrict__ x, int64_t n,
                                                          float *out) {
     __shared__ float wm[4];

@@ -1,9 +1,10 @@
 // vs_sort.hip -- the sorting paths of libvs_hip.so (rocPRIM radix sorts):
 //   - the stable key sort of the k-means update (point ids grouped by
 //     cluster in increasing point order);
+//   - range hits and self-join pairs by (query, id);
 //   - exact top-k beyond the selection's k: 64-bit keys (order-preserving code
 //     of the fp32 score, then the id), sorted per query.
-#include <cstring>
+#include <algorithm>
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "vs_device.h"
@@ -31,6 +32,12 @@ __global__ void extract_topk_kernel(const uint64_t *__restrict__ sorted, int64_t
         D[t] = metric == 0 ? VS_INF : -VS_INF;
         I[t] = -1;
     }
+}
+
+hipError_t sort_pairs_u64(void *tmp, size_t &tmp_bytes, const uint64_t *kin, uint64_t *kout,
+                          const float *vin, float *vout, int64_t n, int bits, hipStream_t st) {
+    return rocprim::radix_sort_pairs(tmp, tmp_bytes, kin, kout, vin, vout, (size_t)n, 0,
+                                     (unsigned)std::min(bits, 64), st);
 }
 
 hipError_t sort_topk_keys(const uint64_t *keys, int64_t n, int64_t k, int metric, float *D,
