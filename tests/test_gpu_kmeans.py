@@ -200,3 +200,20 @@ def test_kmeans_nonfinite_centroids(vs, bad):
     cr, cntr, _ = oracle.kmeans_update(x, ar, c1, 1, u)
     assert np.array_equal(a2, ar) and obj2 == objr and np.array_equal(cnt2, cntr)
     assert np.array_equal(c2.view(np.uint32), cr.view(np.uint32))
+
+
+@pytest.mark.parametrize("n,d,K", [(700, 64, 2), (1500, 65, 3), (4100, 130, 2), (3000, 200, 1)])
+def test_update_batches(vs, n, d, K):
+    """Clusters of many rows (whole and partial batches of 64 or 128 rows,
+    one or several dimension chunks): the running sums in point order."""
+    x = syn.normal_unit(n, d, n, 0)
+    cen = x[:K].copy()
+    pts = vs.GpuIndexFlat.l2(d, storage="f32")
+    pts.add(x)
+    u = np.full(K * d, 0.5)
+    a, newc, cnt, obj = vs.kmeans_step(pts, cen, 1, u)
+    pts.close()
+    ar, _, objr = oracle.kmeans_assign(x, cen, oracle.default_threads())
+    cr, cntr, _ = oracle.kmeans_update(x, ar, cen, 1, u)
+    assert np.array_equal(a, ar) and obj == objr and np.array_equal(cnt, cntr)
+    assert np.array_equal(newc.view(np.uint32), cr.view(np.uint32))
