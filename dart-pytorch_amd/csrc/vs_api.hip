@@ -228,7 +228,7 @@ struct vs_index {
     // scratch (grown on demand, reused across calls)
     DevBuf stage, qp, qf, qnorm, flags, cand_v, cand_i, lcnt, gthr, lbound, vf, fbq, fbD, fbI, outD, outI,
         athr, rq, ri, rs, rtmp, rcount, misc;
-    DevBuf km_cen16, km_c16n;  // k-means: bf16 copy of the centroid rows (and its unused norms)
+    DevBuf km_cen16;  // k-means: bf16 copy of the centroid rows
     DevBuf km_cen, km_cxn, km_assign, km_best, km_fb, km_keys, km_order, km_tmp, km_counts,
         km_offsets, km_out, km_iota;
     // k-means: the points prepared as queries, kept while the rows are unchanged
@@ -254,6 +254,8 @@ struct vs_index {
     vs::PreparedQueries km_pq;
     uint32_t km_pflags = 0;
     uint64_t km_prep_version = ~0ull;
+    int64_t km_prep_ld = 0;  // the planes' stride
+    DevBuf km_pres;          // the largest rounding residual of a point
     // bf16 copy of fp32 rows for the one-pass selection (search, range,
     // self-join): rows [0, copy_n) of stride copy_ld, zero rows after them
     DevBuf xb16;
@@ -2000,7 +2002,7 @@ void vs_index_destroy(vs_index *x) {
                       &x->misc,    &x->km_cen,    &x->km_cxn,   &x->km_assign, &x->km_best,
                       &x->km_fb,   &x->km_keys,   &x->km_order, &x->km_tmp,   &x->km_counts,
                       &x->km_offsets, &x->km_out, &x->km_iota, &x->lcnt,   &x->km_qp,
-                      &x->km_qf,   &x->km_qnorm,  &x->km_cen16, &x->km_c16n, &x->qres, &x->fbl,
+                      &x->km_qf,   &x->km_qnorm,  &x->km_cen16, &x->km_pres, &x->qres, &x->fbl,
                       &x->vx,        &x->ctl,      &x->km_shift, &x->km_init,
                       &x->km_pkeys, &x->km_part, &x->ex_qd,   &x->ex_keys, &x->ex_part};
     for (DevBuf *b : bufs) b->release();
@@ -2557,11 +2559,13 @@ int vs_kmeans_step(vs_index *x, const float *centroids_in, int64_t K, int64_t mi
     VS_HIP(x->km_cxn.ensure((size_t)(K + kRowSlack) * 4), "centroid norms");
     VS_HIP(hipMemsetAsync(x->km_cen.p, 0, (size_t)(K + kRowSlack) * ld * 4, x->st), "clear");
     VS_HIP(hipMemsetAsync(x->km_cxn.p, 0, (size_t)(K + kRowSlack) * 4, x->st), "clear");
+    float pmax = 0.f;
+    VS_TAKE(xnorm_max(x, A, &pmax));  // (uses misc too)
     // misc: [0] the largest centroid norm, [1] the centroids' flags, [2] the
     // accumulator bound -- all on the device: no host round trip separates
     // the centroids from the assign scan (the flags are read with the
     // pick's results, before any exhaustive pass)
-    VS_HIP(x->misc.ensure(16), "misc");
+    VS_HIP(x->misc.ensure(16), "misc");  // ([3]: the largest rounding residual)
     float *kmisc = x->misc.as<float>();
     uint32_t *cflags_dev = (uint32_t *)(kmisc + 1);
     VS_HIP(vs::launch_fill32(cflags_dev, 1, 0u, x->st), "flags");
@@ -2571,17 +2575,6 @@ int vs_kmeans_step(vs_index *x, const float *centroids_in, int64_t K, int64_t mi
     VS_HIP(vs::launch_max_reduce(x->km_cxn.as<float>(), K, kmisc, x->st), "max");
     VS_HIP(x->flags.ensure(4), "flags");
 
-    // points as prepared queries against the centroid "database" (kept
-    // across iterations while the stored rows are unchanged)
-    if (x->km_prep_version != x->version) {
-        select_rows(x);
-        x->km_prep_version = ~0ull;
-        int rc0 = prepare_queries(x, A, x->xb, 0, ld, n, &x->km_pq, &x->km_pflags, x->km_qp,
-                                  x->km_qf, x->km_qnorm);
-        if (rc0) return rc0;
-        x->km_prep_version = x->version;
-    }
-    const vs::PreparedQueries pq = x->km_pq;
     int rc = VS_OK;
     // the distance kernels index the centroid rows with the points' ld
     vs_index cview;
@@ -2590,32 +2583,75 @@ int vs_kmeans_step(vs_index *x, const float *centroids_in, int64_t K, int64_t mi
     cview.lds_max = x->lds_max;
     cview.num_cu = x->num_cu;
     cview.opt = x->opt;
-    // one-pass selection (bf16 hi planes of points and centroids) where the
-    // GEMM-tiled scan runs it; the shortlist proof below widens its bound
+    // One-pass selection (bf16 planes of points and centroids): on a bf16 copy
+    // of the centroids (option km16) the row-shared scan up to 256 elements,
+    // the GEMM-tiled one beyond; without the copy, where a scan rounds the
+    // fp32 centroids itself.  The pick's proof covers the rounding.
+    const int64_t ld16 = vs::storage_ld(d, 1);
     vs::ScanPlan plan;
-    bool coarse = x->opt.coarse != 0;
-    if (coarse) coarse = plan_scan(&cview, n, K, 1, 16, vs::kSelectCoarse, &plan) == VS_OK &&
-                         (plan.kind == 2 || plan.kind == 3);
+    bool coarse = x->opt.coarse != 0, near = false, copy16 = false;
+    if (coarse && x->opt.km16) {
+        cview.sel.ld = ld16;
+        copy16 = plan_scan(&cview, n, K, 1, 16, vs::kSelectCoarse, &plan) == VS_OK && plan.kind == 3;
+        if (!copy16) {
+            cview.opt.gemm4 = 0;
+            plan = vs::ScanPlan();
+            near = copy16 = plan_scan(&cview, n, K, 1, 8, 1, &plan, false, 0, true) == VS_OK &&
+                            plan.kind == 2;
+        }
+        if (!copy16) cview.sel.ld = ld;
+    }
+    if (!copy16) {
+        plan = vs::ScanPlan();
+        if (coarse)
+            coarse = plan_scan(&cview, n, K, 1, 16, vs::kSelectCoarse, &plan) == VS_OK &&
+                     (plan.kind == 2 || plan.kind == 3);
+    }
+    // points as prepared queries against the centroid "database" (kept
+    // across iterations while the stored rows are unchanged)
+    if (x->km_prep_version != x->version || x->km_prep_ld != cview.sel.ld) {
+        select_rows(x);
+        x->sel.ld = cview.sel.ld;
+        x->km_prep_version = ~0ull;
+        rc = prepare_queries(x, A, x->xb, 0, ld, n, &x->km_pq, &x->km_pflags, x->km_qp, x->km_qf,
+                             x->km_qnorm, nullptr, false, true);
+        if (rc) return rc;
+        VS_HIP(x->km_pres.ensure(4), "residual maximum");
+        VS_HIP(vs::launch_max_reduce(x->km_pq.qres, n, x->km_pres.as<float>(), x->st),
+               "residual maximum");
+        x->km_prep_ld = cview.sel.ld;
+        x->km_prep_version = x->version;
+    }
+    const vs::PreparedQueries pq = x->km_pq;
     if (!coarse) {
         plan = vs::ScanPlan();
         rc = plan_scan(&cview, n, K, pq.planes, 16, 0, &plan);
         if (rc) return rc;
     }
-    float pmax = 0.f;
-    VS_TAKE(xnorm_max(x, A, &pmax));
+    if (copy16) {
+        VS_HIP(x->km_cen16.ensure((size_t)(K + kRowSlack) * ld16 * 2), "centroid copy");
+        VS_HIP(hipMemsetAsync(x->km_cen16.as<char>() + (size_t)K * ld16 * 2, 0,
+                              (size_t)kRowSlack * ld16 * 2, x->st),
+               "clear");
+        VS_HIP(vs::launch_copy_rows16(x->km_cen.p, ld, K, ld16, x->km_cen16.p, kmisc + 3, x->st),
+               "centroid copy");
+    }
     // Error of the accumulator |c|^2 - 2 x.c (point x, centroid c):
-    //  - operands: each product of the MFMA operands lies within r |2 x_j c_j|
-    //    of -2 x_j c_j, r = 2^-8 for the one-pass selection (both operands
-    //    rounded to bf16, 2^-9 each) and 2^-15 for the split-bf16 passes (hi
-    //    + lo within 2^-18 of each value, the dropped lo * q1 term);
+    //  - operands: on the centroids' copy, the measured norms of the points'
+    //    and centroids' rounding residuals (|error| <= 2 (r_x |c| + |x16| r_c));
+    //    otherwise each product of the MFMA operands lies within r |2 x_j c_j|
+    //    of -2 x_j c_j, r = 2^-7 for the one-pass selection (both operands
+    //    rounded to bf16, at most 2^-8 each) and 2^-15 for the split-bf16
+    //    passes (hi + lo within 2^-18 of each value, the dropped lo * q1 term);
     //  - fp32 accumulation (accum_gamma) of one pass (one-pass selection) or
-    //    of three (split-bf16 points and centroids);
-    // so |error| <= 2 r |x| |c| + gamma (|c|^2 + 2 |x| |c|) (Cauchy-Schwarz),
-    // taken with a 25% margin.
-    const double r = coarse ? 1.0 / 256.0 : 1.0 / 32768.0;
+    //    of three (split-bf16 points and centroids), with a 25% margin:
+    //    gamma (|c|^2 + 2 |x| |c|).
+    const double r = coarse ? 1.0 / 128.0 : 1.0 / 32768.0;
     const double gam = accum_gamma(d, coarse ? 1 : 3);
     float *bound_dev = kmisc + 2;
-    VS_HIP(vs::launch_kmeans_bound(kmisc, (double)pmax, r, gam, bound_dev, x->st), "bound");
+    VS_HIP(vs::launch_kmeans_bound(kmisc, (double)pmax, r, gam, x->km_pres.as<float>(),
+                                   copy16 ? kmisc + 3 : nullptr, bound_dev, x->st),
+           "bound");
     plan.dev_bound = bound_dev;
     const float bound = 0.f;  // (the kernels read bound_dev)
     // On the row-shared scan each lane appends every value below its running
@@ -2624,18 +2660,23 @@ int vs_kmeans_step(vs_index *x, const float *centroids_in, int64_t K, int64_t mi
     if (coarse && plan.kind == 3) {
         plan.share_kmin = 1;
         plan.kmin_margin = 0.f;  // 2.5 * bound_dev, read by the kernels
-        // option km16_nqb 4: 64 points per wave on the bf16 copy of the
-        // centroids (32-row tiles keep it at two waves per SIMD); decided
-        // here, before the lists are sized
-        if (x->opt.km16_nqb == 4 && x->opt.km16 && plan.tile_st == vs::kSelectCoarse &&
-            plan.nks == 8) {
-            const size_t lds = vs::share_lds_bytes(plan.nks, 4, 2, plan.cap, 1);
-            if (lds <= x->lds_max) {
-                plan.bn = 256;
-                plan.tm = 2;
-                plan.lds_bytes = lds;
-                plan.nqblk = (n + plan.bn - 1) / plan.bn;
-            }
+        if (copy16) {
+            // 64 points per wave; rows of 256 elements in 32-row tiles (two
+            // waves per SIMD), of 128 in 64-row tiles.  Options km16_nqb 2 and
+            // km16_rt: 32 points per wave, in tiles of 32 or 64 rows.
+            const bool wide = plan.nks == 4 || x->opt.km16_nqb == 4;
+            const int nqb = wide ? 4 : 2;
+            const int rt = plan.nks == 4 ? 4 : wide ? 2 : x->opt.km16_rt;
+            const size_t lds = vs::share_lds_bytes(plan.nks, nqb, rt, plan.cap, 1);
+            if (lds > x->lds_max)
+                return set_err(VS_ERR_UNSUPPORTED, "internal: k-means tiles exceed the LDS");
+            plan.tile_st = 1;
+            plan.bn = 64 * nqb;
+            plan.tm = rt;
+            plan.lds_bytes = lds;
+            plan.nqblk = (n + plan.bn - 1) / plan.bn;
+            plan.rows_per_split = round_up(plan.rows_per_split, 16 * rt);
+            plan.nsplit = std::max<int64_t>(1, (K + plan.rows_per_split - 1) / plan.rows_per_split);
         }
         // the running minima start at the previous assignment's bound
         if (prev && x->opt.kmin_init) {
@@ -2656,50 +2697,44 @@ int vs_kmeans_step(vs_index *x, const float *centroids_in, int64_t K, int64_t mi
         }
     }
     if ((rc = scan_fits(plan, pq))) return rc;
-    const size_t nlists = (size_t)plan.nqblk * plan.nsplit * plan.lw * plan.bn;
-    const size_t nlist = nlists * plan.cap;
+    // (the GEMM-tiled scan's lists: one per point)
+    constexpr int kNearCap = 32;
+    const size_t nlists =
+        near ? (size_t)n : (size_t)plan.nqblk * plan.nsplit * plan.lw * plan.bn;
+    const size_t nlist = nlists * (near ? kNearCap : plan.cap);
     VS_HIP(x->cand_v.ensure(nlist * 4), "candidate lists");
     VS_HIP(x->cand_i.ensure(nlist * 4), "candidate lists");
     VS_HIP(x->lcnt.ensure((nlists + 1) * 4), "list counts");
-    VS_HIP(hipMemsetAsync(x->lcnt.as<int32_t>() + nlists, 0, 4, x->st), "list counts");
+    VS_HIP(hipMemsetAsync(x->lcnt.as<int32_t>() + (near ? 0 : nlists), 0, near ? nlists * 4 : 4,
+                          x->st),
+           "list counts");
     VS_HIP(x->gthr.ensure((size_t)pq.nq_pad * 4), "shared thresholds");
     VS_HIP(hipMemsetD32Async((hipDeviceptr_t)x->gthr.p, (int)vs::kGthrInit, (size_t)pq.nq_pad, x->st),
            "shared thresholds");
-    // the one-pass selection multiplies the bf16 rounding of the centroids:
-    // the row-shared scan reads a bf16 copy of them (half the bytes of the
-    // fp32 rows it would round itself) with the fp32 rows' norms
-    const void *scan_rows = x->km_cen.p;
-    int scan_storage = 0;
-    if (plan.kind == 3 && plan.share_kmin && plan.tile_st == vs::kSelectCoarse && plan.nks == 8 &&
-        x->opt.km16) {
-        VS_HIP(x->km_cen16.ensure((size_t)(K + kRowSlack) * ld * 2), "centroid copy");
-        VS_HIP(x->km_c16n.ensure((size_t)(K + kRowSlack) * 4), "centroid copy");
-        VS_HIP(hipMemsetAsync(x->km_cen16.p, 0, (size_t)(K + kRowSlack) * ld * 2, x->st), "clear");
-        VS_HIP(vs::launch_store_rows(x->km_cen.p, 0, ld, K, ld, x->km_cen16.p, 1, ld,
-                                     x->km_c16n.as<float>(), x->flags.as<uint32_t>(), x->st),
-               "centroid copy");
-        plan.tile_st = 1;
-        // bf16 rows stage twice the rows per tile in the same registers
-        const int rt = x->opt.km16_rt;
-        if (rt == 4 && plan.bn == 128) {
-            const size_t lds = vs::share_lds_bytes(plan.nks, plan.bn / 64, 4, plan.cap, 1);
-            if (lds <= x->lds_max) {
-                plan.tm = 4;
-                plan.lds_bytes = lds;
-                plan.rows_per_split = round_up(plan.rows_per_split, 64);
-                plan.nsplit = std::max<int64_t>(1, (K + plan.rows_per_split - 1) / plan.rows_per_split);
-            }
-        }
-        scan_rows = x->km_cen16.p;
-        scan_storage = 1;
-    }
     note_scan_kind(x, plan);
     {
         ProfScope ps(x, "assign");
-        VS_HIP(vs::launch_scan_topk(scan_rows, scan_storage, ld, x->km_cxn.as<float>(), K, 0, pq, plan,
-                                    x->cand_v.as<float>(), x->cand_i.as<int32_t>(),
-                                    x->gthr.as<uint32_t>(), nullptr, x->lcnt.as<int32_t>(), x->st),
-               "assign scan");
+        if (near)
+            VS_HIP(vs::launch_gemm_near(x->km_cen16.p, ld16, x->km_cxn.as<float>(), K, pq, plan,
+                                        x->gthr.as<uint32_t>(), bound_dev, kNearCap,
+                                        x->cand_v.as<float>(), x->cand_i.as<int32_t>(),
+                                        x->lcnt.as<int32_t>(), x->st),
+                   "assign scan");
+        else
+            VS_HIP(vs::launch_scan_topk(copy16 ? x->km_cen16.p : x->km_cen.p, copy16 ? 1 : 0,
+                                        cview.sel.ld, x->km_cxn.as<float>(), K, 0, pq, plan,
+                                        x->cand_v.as<float>(), x->cand_i.as<int32_t>(),
+                                        x->gthr.as<uint32_t>(), nullptr, x->lcnt.as<int32_t>(),
+                                        x->st),
+                   "assign scan");
+    }
+    if (near) {  // the pick reads lists of the row-shared scan's kind
+        plan.kind = 3;
+        plan.share_kmin = 1;
+        plan.bn = 256;
+        plan.lw = 1;
+        plan.nsplit = 1;
+        plan.cap = kNearCap;
     }
 
     VS_HIP(x->km_assign.ensure((size_t)n * 4), "assignments");

@@ -367,8 +367,11 @@ hipError_t launch_kmeans_init(const int32_t *assign, const double *best_sq, cons
 // *bound = the k-means accumulator bound from the largest centroid norm *cmax
 // and the largest point norm pmax (fp64 arithmetic, rounded to fp32), so
 // that no host round trip separates the centroids' norms from the scan.
-hipError_t launch_kmeans_bound(const float *cmax, double pmax, double r, double gam, float *bound,
-                               hipStream_t st);
+// r: the operands' relative error, used where cres is null; otherwise the
+// measured rounding residuals, *pres the largest of a point, *cres of a
+// centroid.
+hipError_t launch_kmeans_bound(const float *cmax, double pmax, double r, double gam, const float *pres,
+                               const float *cres, float *bound, hipStream_t st);
 hipError_t launch_exclusive_scan_i32(const int32_t *in, int64_t n, int32_t *out, hipStream_t st);
 
 // Stable sort of (key, value) int32 pairs by key (rocPRIM radix sort).
@@ -427,6 +430,16 @@ int share_blocks_per_cu(int st, int nks, int bn, int rt, int64_t ld, size_t lds,
 // m of the row-shared scan's register top-m variant (threshold estimates):
 // values kept per lane and query.
 int share_topm_est();
+
+// k-means on the GEMM-tiled scan (bf16 rows, one query plane; plan.kind 2, not
+// g_pipe): per query, gthr (starting at kGthrInit) receives its smallest
+// accumulator's code and cand_v / cand_i [nq][cap] the values up to 2.5
+// *dev_bound above it, list_cnt [nq] (starting at 0) their number, which may
+// exceed cap.
+hipError_t launch_gemm_near(const void *rows, int64_t ld, const float *xn, int64_t n,
+                            const PreparedQueries &pq, const ScanPlan &plan, uint32_t *gthr,
+                            const float *dev_bound, int cap, float *cand_v, int32_t *cand_i,
+                            int32_t *list_cnt, hipStream_t st);
 
 struct ScanKArgs;
 hipError_t launch_share_scan(const ScanPlan &plan, const ScanKArgs &args, hipStream_t st);

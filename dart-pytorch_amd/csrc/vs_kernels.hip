@@ -2569,22 +2569,24 @@ hipError_t launch_kmeans_init(const int32_t *assign, const double *best_sq, cons
 // device) and the largest point norm pmax: 1.25 (2 r pmax sqrt(cmax) +
 // gam (cmax + 2 pmax sqrt(cmax))) + 1e-6, in fp64, rounded to fp32.
 __global__ void kmeans_bound_kernel(const float *cmax, double pmax, double r, double gam,
-                                    float *bound) {
+                                    const float *pres, const float *cres, float *bound) {
     if (threadIdx.x != 0) return;
-    const double c = (double)*cmax;
-    const double pc = pmax * sqrt(c);
-    *bound = (float)(1.25 * (2.0 * r * pc + gam * (c + 2.0 * pc)) + 1e-6);
+    const double c = (double)*cmax, cn = sqrt(c) * (1.0 + 1e-6);
+    const double pc = pmax * cn;
+    double b = 1.25 * gam * (c + 2.0 * pc);
+    if (cres)
+        b += 2.00002 * ((double)*pres * cn + (pmax + *pres) * (double)*cres);
+    else
+        b += 1.25 * 2.0 * r * pc;
+    *bound = (float)(b * (1.0 + 1e-6) + 1e-6);
 }
 
-hipError_t launch_kmeans_bound(const float *cmax, double pmax, double r, double gam, float *bound,
-                               hipStream_t st) {
-    kmeans_bound_kernel<<<dim3(1), dim3(64), 0, st>>>(cmax, pmax, r, gam, bound);
+hipError_t launch_kmeans_bound(const float *cmax, double pmax, double r, double gam, const float *pres,
+                               const float *cres, float *bound, hipStream_t st) {
+    kmeans_bound_kernel<<<dim3(1), dim3(64), 0, st>>>(cmax, pmax, r, gam, pres, cres, bound);
     return hipGetLastError();
 }
 
-// Exclusive prefix sums of the cluster counts (the first point of every
-// cluster in the grouped order): one workgroup walks the counts in tiles of
-// 1024, carrying the running total.
 __global__ __launch_bounds__(1024) void exclusive_scan_i32_kernel(const int32_t *in, int64_t n,
                                                                   int32_t *out) {
     __shared__ int32_t part[1024];

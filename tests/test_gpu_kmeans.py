@@ -217,3 +217,28 @@ def test_update_batches(vs, n, d, K):
     cr, cntr, _ = oracle.kmeans_update(x, ar, cen, 1, u)
     assert np.array_equal(a, ar) and obj == objr and np.array_equal(cnt, cntr)
     assert np.array_equal(newc.view(np.uint32), cr.view(np.uint32))
+
+
+# the row-shared scan on the centroids' copy (rows padded to 128 or 256
+# elements) and the two GEMM passes beyond, tile edges in points and
+# centroids, duplicated centroids (full lists go to the exhaustive pass), and
+# centroids far longer than the points
+@pytest.mark.parametrize("n,d,K", [(300, 20, 7), (2000, 64, 65), (1500, 150, 130), (600, 257, 3),
+                                   (2500, 300, 257), (700, 520, 64), (515, 384, 129)])
+@pytest.mark.parametrize("kind", ["mixture", "copies", "long"])
+def test_assign_any_dimension(vs, n, d, K, kind):
+    x, _ = syn.gaussian_mixture(n, d, 9, 0.05, n)
+    cen = x[syn.seeded_subset(n, K, 5)].copy()
+    if kind == "copies":
+        cen[:] = cen[np.arange(K) % 2]
+    if kind == "long":
+        cen *= np.float32(50.0)
+    pts = vs.GpuIndexFlat.l2(d, storage="f32")
+    pts.add(x)
+    u = syn.rng(6, 0).random(K * d)
+    for _ in range(2):  # the second from the first one's centroids
+        a, newc, cnt, obj = vs.kmeans_step(pts, cen, 1, u)
+        ar, _, objr = oracle.kmeans_assign(x, cen, oracle.default_threads())
+        assert np.array_equal(a, ar) and obj == objr
+        cen = newc
+    pts.close()
