@@ -236,6 +236,8 @@ struct vs_index {
     // k-means: pinned copies of the distances, assignments and new centroids
     HostBuf km_hbest, km_hassign, km_hcen, km_hfb;
     HostBuf rstage;  // reconstruct: pinned staging of stored rows
+    DevBuf sub_ids, sub_meta;  // subset search: ids; segments, key places and their order
+    HostBuf hsub;              // subset search: pinned segments
     DevBuf ex_qd, ex_keys, ex_part;  // exact keys: fp64 queries, keys, segments' best
     // pinned: control words (kCtlBytes), then a small host search's queries and
     // results
@@ -2004,7 +2006,8 @@ void vs_index_destroy(vs_index *x) {
                       &x->km_offsets, &x->km_out, &x->km_iota, &x->lcnt,   &x->km_qp,
                       &x->km_qf,   &x->km_qnorm,  &x->km_cen16, &x->km_pres, &x->qres, &x->fbl,
                       &x->vx,        &x->ctl,      &x->km_shift, &x->km_init,
-                      &x->km_pkeys, &x->km_part, &x->ex_qd,   &x->ex_keys, &x->ex_part};
+                      &x->km_pkeys, &x->km_part, &x->ex_qd,   &x->ex_keys, &x->ex_part,
+                      &x->sub_ids, &x->sub_meta};
     for (DevBuf *b : bufs) b->release();
     x->km_hbest.release();
     x->km_hassign.release();
@@ -2012,6 +2015,7 @@ void vs_index_destroy(vs_index *x) {
     x->km_hfb.release();
     x->rstage.release();
     x->hio.release();
+    x->hsub.release();
     if (x->st_copy) {
         (void)hipStreamSynchronize(x->st_copy);
         (void)hipStreamDestroy(x->st_copy);
@@ -2338,11 +2342,11 @@ int vs_index_score_all(vs_index *x, const float *q, float *out) {
 
 }  // extern "C"
 
-// Subset search beyond the list path's keep (k > 409): per query, the fp64
+// Subset search beyond the key selection's k: per query, the fp64
 // score of every row its segments name, as (fp32 key code, id) keys sorted
 // on the device (exact_sort_topk_ids); the k first are the answer, sentinel
 // padded past the subset's size.  The ids are checked on the host (the
-// list path checks them in its kernels).
+// selection's path checks them in its kernel).
 static int search_subsets_sorted(vs_index *x, Arena &A, const vs::PreparedQueries &pq, int64_t k,
                                  const int32_t *ids, const int64_t *seg_off,
                                  const int64_t *seg_len, int64_t nseg, float *D, int32_t *I) {
@@ -2409,7 +2413,6 @@ int vs_index_search_subsets(vs_index *x, const void *q, int q_dtype, int64_t nq,
         return set_err(VS_ERR_INVALID, "nq, k, nids and nseg must be >= 0");
     if (nq == 0) return VS_OK;
     if (k == 0) return set_err(VS_ERR_INVALID, "k must be >= 1");
-    const int64_t kk = std::max<int64_t>(8, next_pow2(k + std::max<int64_t>(4, k / 4)));
     if (k > INT32_MAX) return set_err(VS_ERR_INVALID, "k = %lld is too large", (long long)k);
     if (!q || !D || !I || (nq * nseg > 0 && (!seg_off || !seg_len)) || (nids > 0 && !ids))
         return set_err(VS_ERR_INVALID, "null buffer");
@@ -2423,57 +2426,113 @@ int vs_index_search_subsets(vs_index *x, const void *q, int q_dtype, int64_t nq,
     const size_t qbytes = (size_t)nq * x->d * (q_dtype == 1 ? 2 : 4);
     VS_HIP(x->stage.ensure(qbytes), "query staging");
     VS_HIP(hipMemcpyAsync(x->stage.p, q, qbytes, hipMemcpyHostToDevice, x->st), "uploading queries");
-    vs::PreparedQueries pq;
-    select_rows(x);
-    if (int rc = prepare_queries(x, A, x->stage.p, q_dtype, x->d, nq, &pq, nullptr)) return rc;
-    if (kk > 512) return search_subsets_sorted(x, A, pq, k, ids, seg_off, seg_len, nseg, D, I);
-    const int64_t ns = std::max<int64_t>(1, nseg);
-    void *pids, *poff, *plen, *pv, *pi, *pf, *pD, *pI;
-    VS_TAKE(A.tmp((size_t)std::max<int64_t>(nids, 1) * 4, &pids, "ids"));
-    VS_TAKE(A.tmp((size_t)nq * ns * 8, &poff, "segments"));
-    VS_TAKE(A.tmp((size_t)nq * ns * 8, &plen, "segments"));
-    VS_TAKE(A.tmp((size_t)nq * ns * kk * 4, &pv, "lists"));
-    VS_TAKE(A.tmp((size_t)nq * ns * kk * 4, &pi, "lists"));
-    VS_TAKE(A.tmp(4, &pf, "flags"));
-    VS_TAKE(A.tmp((size_t)nq * k * 4, &pD, "results"));
-    VS_TAKE(A.tmp((size_t)nq * k * 4, &pI, "results"));
-    if (nids > 0)
-        VS_HIP(hipMemcpyAsync(pids, ids, (size_t)nids * 4, hipMemcpyHostToDevice, x->st), "ids");
-    if (nseg > 0) {
-        VS_HIP(hipMemcpyAsync(poff, seg_off, (size_t)nq * nseg * 8, hipMemcpyHostToDevice, x->st),
-               "segments");
-        VS_HIP(hipMemcpyAsync(plen, seg_len, (size_t)nq * nseg * 8, hipMemcpyHostToDevice, x->st),
-               "segments");
-    } else {  // one empty segment per query
-        VS_HIP(vs::launch_fill32(poff, nq * 2, 0u, x->st), "segments");
-        VS_HIP(vs::launch_fill32(plen, nq * 2, 0u, x->st), "segments");
+    if (!vs::select_keys_cap(k) ||
+        (size_t)vs::select_keys_cap(k) * 8 + 8192 + 1024 > x->lds_max) {
+        vs::PreparedQueries pq;
+        select_rows(x);
+        if (int rc = prepare_queries(x, A, x->stage.p, q_dtype, x->d, nq, &pq, nullptr)) return rc;
+        return search_subsets_sorted(x, A, pq, k, ids, seg_off, seg_len, nseg, D, I);
     }
-    VS_HIP(vs::launch_fill32(pf, 1, 0u, x->st), "flags");
-    VS_HIP(vs::launch_exact_lists(x->xb, x->storage, x->ld, x->d, x->metric, pq.qf, nq, x->ntotal,
-                                  (int)kk, ns, 0, (float *)pv, (int32_t *)pi, x->st,
-                                  (const int32_t *)pids, (const int64_t *)poff,
-                                  (const int64_t *)plen, (uint32_t *)pf),
-           "subset lists");
-    vs::ScanPlan plan;
-    plan.kind = 0;
-    plan.bn = 1;
-    plan.lw = 1;
-    plan.kk = (int)kk;
-    plan.kk_final = (int)kk;
-    plan.cap = (int)kk;
-    plan.nqblk = nq;
-    plan.nsplit = ns;
-    VS_HIP(vs::launch_merge_refine(x->xb, x->storage, x->ld, x->d, x->metric, pq, plan,
-                                   (float *)pv, (int32_t *)pi, nullptr, nullptr, nullptr, nullptr,
-                                   k, (float *)pD, (int32_t *)pI, x->ntotal, (uint32_t *)pf, 0,
-                                   nullptr, nullptr, x->st),
-           "subset merge");
-    uint32_t f = 0;
-    VS_HIP(hipMemcpyAsync(&f, pf, 4, hipMemcpyDeviceToHost, x->st), "flags");
-    VS_HIP(hipMemcpyAsync(D, pD, (size_t)nq * k * 4, hipMemcpyDeviceToHost, x->st), "results");
-    VS_HIP(hipMemcpyAsync(I, pI, (size_t)nq * k * 4, hipMemcpyDeviceToHost, x->st), "results");
+    // every named row's exact key, grouped by query, then the k smallest of
+    // each group: in chunks of queries of at most 2^25 keys (one query's at
+    // least)
+    VS_HIP(x->sub_ids.ensure((size_t)std::max<int64_t>(nids, 1) * 4), "ids");
+    if (nids > 0)
+        VS_HIP(hipMemcpyAsync(x->sub_ids.p, ids, (size_t)nids * 4, hipMemcpyHostToDevice, x->st),
+               "ids");
+    const int64_t ldd = vs::exact_ldd(x->d);
+    VS_HIP(x->ex_qd.ensure((size_t)nq * ldd * 8), "query rows");
+    double *qd = x->ex_qd.as<double>();
+    // flags: [0] the kernels', then one word per query
+    VS_HIP(x->flags.ensure((size_t)(nq + 1) * 4), "flags");
+    uint32_t *fl = x->flags.as<uint32_t>();
+    VS_HIP(vs::launch_fill32(fl, 1, 0u, x->st), "flags");
+    VS_HIP(vs::launch_exact_queries(x->stage.p, q_dtype, x->d, nq, x->d, qd, fl + 1, x->st),
+           "query rows");
+    VS_HIP(x->outD.ensure((size_t)nq * k * 4), "results");
+    VS_HIP(x->outI.ensure((size_t)nq * k * 4), "results");
+    // per chunk: offsets, lengths and key places of its pairs, then per query
+    // the place and number of its keys, then the pairs' order; through one
+    // pinned block
+    std::vector<int64_t> qkeys((size_t)nq, 0);
+    for (int64_t t = 0; t < nq * nseg; ++t) qkeys[(size_t)(t / nseg)] += seg_len[t];
+    for (int64_t q0 = 0; q0 < nq;) {
+        int64_t q1 = q0, total = 0;
+        while (q1 < nq && (q1 == q0 || total + qkeys[(size_t)q1] <= ((int64_t)1 << 25)))
+            total += qkeys[(size_t)q1++];
+        if (total > (int64_t)INT32_MAX)
+            return set_err(VS_ERR_UNSUPPORTED, "a query's subsets hold %lld rows", (long long)total);
+        const int64_t m = q1 - q0, np = m * nseg;
+        const bool sorted = np >= 1024 && nids <= (int64_t)INT32_MAX;
+        const size_t meta = (size_t)np * 24 + (size_t)m * 8 + (sorted ? (size_t)np * 8 : 0);
+        VS_HIP(x->hsub.ensure(meta + 16), "pinned segments");
+        VS_HIP(x->sub_meta.ensure(meta + (sorted ? (size_t)np * 8 : 0) + 16), "segments");
+        int64_t *ho = x->hsub.as<int64_t>(), *hl = ho + np, *hk = hl + np;
+        int32_t *hqo = (int32_t *)(hk + np), *hqc = hqo + m, *hkey = hqc + m, *hidx = hkey + np;
+        int64_t at = 0;
+        for (int64_t i = 0; i < m; ++i) {
+            hqo[i] = (int32_t)at;
+            hqc[i] = (int32_t)qkeys[(size_t)(q0 + i)];
+            for (int64_t s = 0; s < nseg; ++s) {
+                const int64_t t = i * nseg + s;
+                ho[t] = seg_off[q0 * nseg + t];
+                hl[t] = seg_len[q0 * nseg + t];
+                hk[t] = at;
+                at += hl[t];
+                if (sorted) {
+                    hkey[t] = (int32_t)ho[t];
+                    hidx[t] = (int32_t)t;
+                }
+            }
+        }
+        char *dm = x->sub_meta.as<char>();
+        VS_HIP(hipMemcpyAsync(dm, x->hsub.p, meta, hipMemcpyHostToDevice, x->st), "segments");
+        const int64_t *d_o = (const int64_t *)dm, *d_l = d_o + np, *d_k = d_l + np;
+        const int32_t *d_qo = (const int32_t *)(d_k + np), *d_qc = d_qo + m, *d_key = d_qc + m,
+                      *d_idx = d_key + np;
+        int32_t *perm = nullptr;
+        if (sorted) {
+            int32_t *kout = (int32_t *)d_idx + np;
+            perm = kout + np;
+            int bits = 1;
+            while (((int64_t)1 << bits) < nids) ++bits;
+            size_t tb = 0;
+            VS_HIP(vs::sort_pairs_by_key(nullptr, tb, d_key, kout, d_idx, perm, np, bits, x->st),
+                   "sort size");
+            VS_HIP(x->rtmp.ensure(tb + 16), "sort scratch");
+            VS_HIP(vs::sort_pairs_by_key(x->rtmp.p, tb, d_key, kout, d_idx, perm, np, bits, x->st),
+                   "segment order");
+        }
+        void *keys;
+        const size_t kb = (size_t)std::max<int64_t>(total, 1) * 8;
+        if (kb <= (size_t)1 << 28) VS_TAKE(A.get(x->ex_keys, kb, &keys, "keys"));
+        else VS_TAKE(A.tmp(kb, &keys, "keys"));
+        {
+            ProfScope ps(x, "scan");
+            VS_HIP(vs::launch_subset_keys(x->xb, x->storage, x->ld, x->d, x->metric, qd + q0 * ldd,
+                                          m, x->ntotal, x->sub_ids.as<int32_t>(), d_o, d_l, d_k,
+                                          perm, nseg, (uint64_t *)keys, fl, x->st),
+                   "subset keys");
+        }
+        VS_HIP(vs::launch_select_groups((const uint64_t *)keys, d_qo, d_qc, m, k, x->metric,
+                                        x->outD.as<float>() + q0 * k, x->outI.as<int32_t>() + q0 * k,
+                                        nullptr, x->st),
+               "subset selection");
+        q0 = q1;
+        // (the pinned block is refilled for the next chunk)
+        if (q0 < nq) VS_HIP(hipStreamSynchronize(x->st), "subset search");
+    }
+    std::vector<uint32_t> hf((size_t)nq + 1);
+    VS_HIP(hipMemcpyAsync(hf.data(), fl, hf.size() * 4, hipMemcpyDeviceToHost, x->st), "flags");
     VS_HIP(hipStreamSynchronize(x->st), "subset search");
-    if (f & vs::kFlagBadId) return set_err(VS_ERR_INVALID, "an id in the lists is outside [0, ntotal)");
+    for (int64_t i = 1; i <= nq; ++i)
+        if (hf[(size_t)i] & vs::kFlagNonFinite)
+            return set_err(VS_ERR_NONFINITE, "queries contain NaN or infinity");
+    if (hf[0] & vs::kFlagBadId)
+        return set_err(VS_ERR_INVALID, "an id in the lists is outside [0, ntotal)");
+    VS_HIP(hipMemcpyAsync(D, x->outD.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, x->st), "results");
+    VS_HIP(hipMemcpyAsync(I, x->outI.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, x->st), "results");
+    VS_HIP(hipStreamSynchronize(x->st), "subset search");
     return VS_OK;
 }
 

@@ -235,8 +235,8 @@ hipError_t launch_exact_tile(const void *xb, int storage, int64_t ld, int64_t d,
 // those (the distances of a query spread over few exponents, so bins on the
 // keys' top bits would hold nearly all of them), once to collect the keys up
 // to the k-th's bin into LDS, where they are sorted.  While that bin holds
-// more than the buffer takes, it is divided again; keys are distinct, so a
-// step of one key ends it.
+// more than the buffer takes, it is divided again, at the end down to one key
+// (a subset may name a row more than once).
 // Measured: k = 1000 of 200,000 keys for 100 queries: 117 us (a device radix
 // sort per query: 7 ms); k = 10 of 10,000 keys: 10 us.
 // ---------------------------------------------------------------------------
@@ -260,8 +260,8 @@ struct SelectKeysArgs {
     int64_t nflags;
     uint32_t *hflags;
     // groups instead of equal rows of keys (off non-null): query q's keys are
-    // keys[off[q] .. + cnt[q]); kFlagShort goes to *short_flag for one of
-    // fewer than k
+    // keys[off[q] .. + cnt[q]); kFlagShort goes to *short_flag (or null) for
+    // one of fewer than k
     const int32_t *off, *cnt;
     uint32_t *short_flag;
 };
@@ -291,14 +291,14 @@ __global__ __launch_bounds__(kSelThreads) void select_keys_kernel(SelectKeysArgs
     int *hist = (int *)(buf + a.cap);        // [kSelBins]
     __shared__ uint64_t s_lo[16], s_hi[16];
     __shared__ int s_n[16];
-    __shared__ int s_bin, s_before, s_in, s_fill;
+    __shared__ int s_bin, s_before, s_in, s_fill, s_eq;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t q = blockIdx.x / a.nseg;
     const int seg = (int)(blockIdx.x % a.nseg);
     const int64_t k0 = (int64_t)seg * a.seglen;
     const int m = a.off ? a.cnt[q] : (int)max((int64_t)0, min(a.seglen, a.n - k0));
     const uint64_t *kp = a.keys + (a.off ? (int64_t)a.off[q] : q * a.kstride + k0);
-    if (a.off && tid == 0 && m < a.k) atomicOr(a.short_flag, kFlagShort);
+    if (a.short_flag && tid == 0 && m < a.k) atomicOr(a.short_flag, kFlagShort);
 
     uint32_t flag = 0;
     if (a.rowflags) {
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(kSelThreads) void select_keys_kernel(SelectKeysArgs
         s_hi[wave] = hi;
         s_n[wave] = cnt;
     }
-    if (tid == 0) s_fill = 0;
+    if (tid == 0) s_fill = s_eq = 0;
     __syncthreads();
     lo = s_lo[0];
     hi = s_hi[0];
@@ -365,6 +365,7 @@ __global__ __launch_bounds__(kSelThreads) void select_keys_kernel(SelectKeysArgs
 
     uint64_t top = hi;  // every key up to top is collected
     int take = cnt;
+    int eq_want = INT_MAX;  // of those equal to top, this many
     if (cnt > a.cap) {
         int rank = (int)a.k, below = 0;  // (k <= cap < cnt)
         for (;;) {
@@ -401,6 +402,11 @@ __global__ __launch_bounds__(kSelThreads) void select_keys_kernel(SelectKeysArgs
             top = last < hi ? last : hi;
             take = below + before + in;
             if (take <= a.cap) break;
+            if (shift == 0) {  // one key, more often than the buffer takes
+                eq_want = rank - before;
+                take = below + before + eq_want;
+                break;
+            }
             below += before;
             rank -= before;
             lo += (uint64_t)bin << shift;
@@ -408,7 +414,8 @@ __global__ __launch_bounds__(kSelThreads) void select_keys_kernel(SelectKeysArgs
         }
     }
     each([&](uint64_t v) {
-        if (v <= top) buf[atomicAdd(&s_fill, 1)] = v;
+        if (v < top || (v == top && (eq_want == INT_MAX || atomicAdd(&s_eq, 1) < eq_want)))
+            buf[atomicAdd(&s_fill, 1)] = v;
     });
     __syncthreads();
     int p2 = 2;
@@ -502,7 +509,7 @@ hipError_t launch_select_groups(const uint64_t *keys, const int32_t *off, const 
                                 uint32_t *flags, hipStream_t st) {
     if (nq <= 0) return hipSuccess;
     const int cap = select_keys_cap(k);
-    if (!cap || k < 1 || nq > INT32_MAX || !off || !cnt || !flags) return hipErrorInvalidValue;
+    if (!cap || k < 1 || nq > INT32_MAX || !off || !cnt) return hipErrorInvalidValue;
     SelectKeysArgs a{};
     a.keys = keys;
     a.k = k;
@@ -721,6 +728,155 @@ hipError_t launch_range_unpack(const uint64_t *sorted, int64_t m, int idbits, in
     if (t <= 0) return hipSuccess;
     range_unpack_kernel<<<dim3((unsigned)((t + 255) / 256)), dim3(256), 0, st>>>(sorted, m, idbits,
                                                                                q, id, nlims, lims);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Exact keys of row subsets: pair p = (query p / nseg, segment p % nseg) names
+// the rows ids[seg_off[p] .. + seg_len[p]); its keys go to keys[koff[p] ..).
+// A workgroup takes `group` pairs: each wave takes 64 rows at a time through
+// its own LDS buffer in 32-element chunks (eight lanes read 128 contiguous
+// bytes of a row, the next chunk in flight), a lane sums one row, and the
+// queries' values come through scalar loads as in exact_tile_kernel.
+//
+// Bound by the row reads from L2 (one pair at a time: 7.8 TB/s), so `perm`
+// (or null) walks the pairs in the order of their segments, each XCD a
+// contiguous part of it, and four pairs of one segment (an inverted list that
+// many queries probe) share each row read.  1,000 queries x 16 of 256 lists of
+// 200,000 x 128 rows, 5.2e7 rows in all: one thread per row 4.2 ms, one pair
+// at a time 3.3 ms, four 2.2 ms.
+// ---------------------------------------------------------------------------
+struct SubsetKArgs {
+    const void *xb;
+    int64_t ld, d, ldd, n;
+    const double *qd;
+    const int32_t *ids;
+    const int64_t *seg_off, *seg_len, *koff;
+    const int32_t *perm;
+    int64_t nseg, npairs;
+    int group;
+    uint64_t *keys;
+    uint32_t *flags;
+};
+constexpr int kSubsetGroup = 4;
+
+// The keys of QT pairs of one segment.
+template <int ST, int METRIC, int QT>
+__device__ __forceinline__ void subset_keys_run(const SubsetKArgs &a, const int64_t *pair,
+                                                float (*xs)[kPairLd], int wave, int lane) {
+    const int64_t len = a.seg_len[pair[0]], i0 = a.seg_off[pair[0]];
+    const_f64_t q[QT];
+    uint64_t *out[QT];
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+        q[u] = (const_f64_t)(uintptr_t)(a.qd + pair[u] / a.nseg * a.ldd);
+        out[u] = a.keys + a.koff[pair[u]];
+    }
+    constexpr int PE = ST == 1 ? 8 : 4, TPR = kPairK / PE, NPR = TPR;
+    for (int64_t base = wave * 64; base < len; base += 256) {
+        const bool in = base + lane < len;
+        int32_t id = in ? a.ids[i0 + base + lane] : 0;
+        bool ok = in;
+        if (id < 0 || id >= a.n) {
+            atomicOr(a.flags, kFlagBadId);
+            ok = false;
+            id = 0;
+        }
+        u32x4_t xr[NPR];
+        auto load = [&](int64_t k0) {
+#pragma unroll
+            for (int i = 0; i < NPR; ++i) {
+                const int r = i * (64 / TPR) + lane / TPR;
+                const int64_t e = (int64_t)__shfl(id, r) * a.ld + k0 + (lane % TPR) * PE;
+                xr[i] = *(const u32x4_t *)((const char *)a.xb + e * (ST == 1 ? 2 : 4));
+            }
+        };
+        double s[QT];
+#pragma unroll
+        for (int u = 0; u < QT; ++u) s[u] = 0.0;
+        load(0);
+        for (int64_t k0 = 0; k0 < a.d; k0 += kPairK) {
+            lds_wave_sync();
+#pragma unroll
+            for (int i = 0; i < NPR; ++i) {
+                float *dst = &xs[i * (64 / TPR) + lane / TPR][(lane % TPR) * PE];
+                const u32x4_t v = xr[i];
+                if constexpr (ST == 1) {
+                    *(u32x4_t *)dst = u32x4_t{v.x << 16, v.x & 0xFFFF0000u, v.y << 16, v.y & 0xFFFF0000u};
+                    *(u32x4_t *)(dst + 4) = u32x4_t{v.z << 16, v.z & 0xFFFF0000u, v.w << 16, v.w & 0xFFFF0000u};
+                } else {
+                    *(u32x4_t *)dst = v;
+                }
+            }
+            lds_wave_sync();
+            if (k0 + kPairK < a.d) load(k0 + kPairK);
+            // (elements past d are zero on both sides: their terms add +0)
+#pragma unroll 2
+            for (int j = 0; j < kPairK; j += 4) {
+                const float4 x4 = *(const float4 *)&xs[lane][j];
+                const double x[4] = {(double)x4.x, (double)x4.y, (double)x4.z, (double)x4.w};
+#pragma unroll
+                for (int u = 0; u < QT; ++u) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const double qv = q[u][k0 + j + c];
+                        if constexpr (METRIC == 0) {
+                            const double diff = qv - x[c];
+                            s[u] = s[u] + diff * diff;
+                        } else {
+                            s[u] = __builtin_fma(qv, x[c], s[u]);
+                        }
+                    }
+                }
+            }
+        }
+        if (in) {
+#pragma unroll
+            for (int u = 0; u < QT; ++u) {
+                const float key = METRIC == 0 ? (float)s[u] : -(float)s[u];
+                out[u][base + lane] = ok ? ((uint64_t)enc_order(key) << 32) | (uint32_t)id : kNoKey;
+            }
+        }
+    }
+}
+
+template <int ST, int METRIC>
+__global__ __launch_bounds__(256) void subset_keys_kernel(SubsetKArgs a) {
+    __shared__ __align__(16) float xsh[4][64][kPairLd];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t groups = (a.npairs + a.group - 1) / a.group, per = (groups + 7) / 8;
+    const int64_t w = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int64_t)(blockIdx.x >> 3) >= per || w >= groups) return;
+    const int64_t p0 = w * a.group, np = min((int64_t)a.group, a.npairs - p0);
+    int64_t pair[kSubsetGroup];
+    bool same = np == kSubsetGroup;
+    for (int u = 0; u < kSubsetGroup; ++u) {
+        const int64_t t = p0 + min((int64_t)u, np - 1);
+        pair[u] = a.perm ? (int64_t)a.perm[t] : t;
+        same = same && a.seg_off[pair[u]] == a.seg_off[pair[0]] &&
+               a.seg_len[pair[u]] == a.seg_len[pair[0]];
+    }
+    if (same) {
+        subset_keys_run<ST, METRIC, kSubsetGroup>(a, pair, xsh[wave], wave, lane);
+    } else {
+        for (int u = 0; u < np; ++u) subset_keys_run<ST, METRIC, 1>(a, pair + u, xsh[wave], wave, lane);
+    }
+}
+
+hipError_t launch_subset_keys(const void *xb, int storage, int64_t ld, int64_t d, int metric,
+                              const double *qd, int64_t nq, int64_t n, const int32_t *ids,
+                              const int64_t *seg_off, const int64_t *seg_len, const int64_t *koff,
+                              const int32_t *perm, int64_t nseg, uint64_t *keys, uint32_t *flags,
+                              hipStream_t st) {
+    if (nq <= 0 || nseg <= 0) return hipSuccess;
+    SubsetKArgs a{xb,   ld,   d,    exact_ldd(d), n,    qd,   ids, seg_off, seg_len, koff,
+                  perm, nseg, nq * nseg, perm ? kSubsetGroup : 1, keys, flags};
+    const int64_t groups = (a.npairs + a.group - 1) / a.group, grid = (groups + 7) / 8 * 8;
+    if (grid > INT32_MAX) return hipErrorInvalidValue;
+    auto fn = storage == 1 ? (metric == 0 ? subset_keys_kernel<1, 0> : subset_keys_kernel<1, 1>)
+                           : (metric == 0 ? subset_keys_kernel<0, 0> : subset_keys_kernel<0, 1>);
+    hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

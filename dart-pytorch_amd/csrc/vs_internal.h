@@ -195,15 +195,10 @@ hipError_t launch_merge_refine(const void *xb, int storage, int64_t ld, int64_t 
 // are [s * rows_per_split, ...); lists cand_v / cand_i [nq][nsplit][kk] hold
 // (fp32 key, id), key = score (L2) or -score (IP), sentinels (+inf, -1).
 // kk: a multiple of 4 in [4, 512].
-// With ids non-null, list (q, s) covers the rows ids[seg_off[q nsplit + s]
-// .. + seg_len[q nsplit + s]) instead of a split (ids outside [0, n) set
-// kFlagBadId in *flags and are skipped).
 hipError_t launch_exact_lists(const void *xb, int storage, int64_t ld, int64_t d, int metric,
                               const float *qf, int64_t nq, int64_t n, int kk, int64_t nsplit,
                               int64_t rows_per_split, float *cand_v, int32_t *cand_i,
-                              hipStream_t st, const int32_t *ids = nullptr,
-                              const int64_t *seg_off = nullptr, const int64_t *seg_len = nullptr,
-                              uint32_t *flags = nullptr);
+                              hipStream_t st);
 
 // out[r] = fp32 of the exact fp64 score of each of the n rows against the
 // fp32 query qf[d] (L2: squared distance, IP: dot).
@@ -243,10 +238,19 @@ hipError_t launch_select_keys(const uint64_t *keys, int64_t nq, int64_t n, int64
                               hipStream_t st);
 
 // The same over one group of keys per query: keys[off[q] .. + cnt[q]), any
-// number; kFlagShort is set in *flags for a query with fewer than k.
+// number; kFlagShort is set in *flags (or null) for a query with fewer than k.
 hipError_t launch_select_groups(const uint64_t *keys, const int32_t *off, const int32_t *cnt,
                                 int64_t nq, int64_t k, int metric, float *D, int32_t *I,
                                 uint32_t *flags, hipStream_t st);
+// Exact keys of row subsets: pair p = (query p / nseg, segment p % nseg) covers
+// the rows ids[seg_off[p] .. + seg_len[p]), whose keys go to keys[koff[p] ..)
+// (all ones, and kFlagBadId in *flags, for an id outside [0, n)).  perm: the
+// pairs in the order to walk them, or null.
+hipError_t launch_subset_keys(const void *xb, int storage, int64_t ld, int64_t d, int metric,
+                              const double *qd, int64_t nq, int64_t n, const int32_t *ids,
+                              const int64_t *seg_off, const int64_t *seg_len, const int64_t *koff,
+                              const int32_t *perm, int64_t nseg, uint64_t *keys, uint32_t *flags,
+                              hipStream_t st);
 // cnt[q] += the number of pairs of query q.
 hipError_t launch_count_pairs(const int32_t *cq, int64_t m, int64_t nq, int32_t *cnt,
                               hipStream_t st);

@@ -1393,8 +1393,8 @@ hipError_t launch_merge_refine(const void *xb, int storage, int64_t ld, int64_t 
 // kk best (key, id) pairs, key = fp32 score (L2) or -fp32 score (IP), in
 // (key, id) order -- the order the merge's re-rank sorts by.  The lists
 // ([nq][nsplit][kk], sentinels (+inf, -1)) then go through the merge, whose
-// selection over exact keys is exact.  This is the path for queries whose
-// approximate selection could not be proven exact.
+// selection over exact keys is exact.  This is the fallback of the fixed-scratch
+// search, which has no room for a key matrix.
 // ---------------------------------------------------------------------------
 struct ExactKArgs {
     const void *xb;
@@ -1406,11 +1406,6 @@ struct ExactKArgs {
     int64_t nsplit, rows_per_split;
     float *cand_v;
     int32_t *cand_i;
-    // row subsets instead of splits (ids non-null): list (q, s) scans the
-    // rows ids[seg_off[q nsplit + s] .. + seg_len[q nsplit + s])
-    const int32_t *ids;
-    const int64_t *seg_off, *seg_len;
-    uint32_t *flags;  // kFlagBadId for an id outside [0, n)
 };
 
 template <int ST>
@@ -1440,34 +1435,19 @@ __global__ __launch_bounds__(256) void exact_lists_kernel(ExactKArgs a) {
     }
     for (int64_t j = tid; j < a.ld; j += 256) qsh[j] = j < a.d ? a.qf[q * a.d + j] : 0.0f;
     __syncthreads();
-    // rows [r0, r1) of the split, or positions [r0, r1) of the id list
-    int64_t r0 = split * a.rows_per_split;
-    int64_t r1 = min(a.n, r0 + a.rows_per_split);
-    if (a.ids) {
-        r0 = a.seg_off[q * a.nsplit + split];
-        r1 = r0 + a.seg_len[q * a.nsplit + split];
-    }
+    const int64_t r0 = split * a.rows_per_split;
+    const int64_t r1 = min(a.n, r0 + a.rows_per_split);
     for (int64_t base = r0; base < r1; base += 256) {
-        const int64_t t = base + tid;
-        if (t < r1) {
-            int64_t row = t;
-            if (a.ids) {
-                row = a.ids[t];
-                if (row < 0 || row >= a.n) {
-                    atomicOr(a.flags, kFlagBadId);
-                    row = -1;
-                }
-            }
-            if (row >= 0) {
-                const double ex = exact_score<ST>(qsh, a.xb, a.ld, row, a.d, a.metric);
-                const float key = a.metric == 0 ? (float)ex : -(float)ex;
-                const float th = s_thr;
-                const int thi = s_thr_id;
-                if (key < th || (key == th && (int)row < thi)) {
-                    const int pos = atomicAdd(&s_cnt, 1);
-                    bv[kk + pos] = key;
-                    bi[kk + pos] = (int)row;
-                }
+        const int64_t row = base + tid;
+        if (row < r1) {
+            const double ex = exact_score<ST>(qsh, a.xb, a.ld, row, a.d, a.metric);
+            const float key = a.metric == 0 ? (float)ex : -(float)ex;
+            const float th = s_thr;
+            const int thi = s_thr_id;
+            if (key < th || (key == th && (int)row < thi)) {
+                const int pos = atomicAdd(&s_cnt, 1);
+                bv[kk + pos] = key;
+                bi[kk + pos] = (int)row;
             }
         }
         __syncthreads();
@@ -1489,15 +1469,12 @@ __global__ __launch_bounds__(256) void exact_lists_kernel(ExactKArgs a) {
 hipError_t launch_exact_lists(const void *xb, int storage, int64_t ld, int64_t d, int metric,
                               const float *qf, int64_t nq, int64_t n, int kk, int64_t nsplit,
                               int64_t rows_per_split, float *cand_v, int32_t *cand_i,
-                              hipStream_t st, const int32_t *ids, const int64_t *seg_off,
-                              const int64_t *seg_len, uint32_t *flags) {
+                              hipStream_t st) {
     if (nq <= 0) return hipSuccess;
     if (kk < 4 || kk > kMergeKeepMax || (kk & 3) || nsplit < 1 || nq * nsplit > INT32_MAX)
         return hipErrorInvalidValue;
-    if (ids && (!seg_off || !seg_len || !flags)) return hipErrorInvalidValue;
     ExactKArgs a{xb,     ld,     d,      metric,         qf,      nq,      n,
-                 kk,     nsplit, rows_per_split, cand_v, cand_i, ids, seg_off,
-                 seg_len, flags};
+                 kk,     nsplit, rows_per_split, cand_v, cand_i};
     const size_t lds = merge_lds(ld);
     void (*fn)(ExactKArgs) = storage == 1 ? exact_lists_kernel<1> : exact_lists_kernel<0>;
     if (lds > 64 * 1024) {

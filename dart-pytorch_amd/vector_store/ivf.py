@@ -38,6 +38,7 @@ class IndexIVFFlat(Index):
         self._store = GpuIndexFlat(d, self.metric, storage="f32", device=device)
         self.is_trained = False
         self._lists = [[] for _ in range(self.nlist)]
+        self._flat = None  # (ids of every list one after another, starts, sizes)
 
     @property
     def ntotal(self) -> int:
@@ -46,6 +47,7 @@ class IndexIVFFlat(Index):
     @property
     def inv_lists(self):
         """invLists (index_ivf_flat.dart:52-55): ids per cell, insertion order."""
+        self._flat = None  # the caller may change them
         return self._lists
 
     def close(self) -> None:
@@ -73,6 +75,19 @@ class IndexIVFFlat(Index):
         self._store.add(x)
         for i, c in enumerate(cells.tolist()):
             self._lists[c].append(base + i)
+        self._flat = None
+
+    def _flat_lists(self):
+        """The inverted lists as one id array, laid out again when rows or
+        lists have changed."""
+        total = sum(map(len, self._lists))
+        if self._flat is None or self._flat[0].size != total:
+            sizes = np.array([len(l) for l in self._lists], np.int64)
+            starts = np.zeros(self.nlist + 1, np.int64)
+            np.cumsum(sizes, out=starts[1:])
+            ids = np.fromiter((i for l in self._lists for i in l), np.int32, count=int(starts[-1]))
+            self._flat = (ids, starts, sizes)
+        return self._flat
 
     def search(self, queries, k: int) -> SearchResult:
         if not self.is_trained:
@@ -82,10 +97,7 @@ class IndexIVFFlat(Index):
         if nq == 0:
             return SearchResult(np.zeros((0, k), np.float32), np.zeros((0, k), np.int32))
         probes = self.quantizer.search(q, self.nprobe).ids  # (nq, nprobe), -1 past nlist
-        sizes = np.array([len(l) for l in self._lists], np.int64)
-        starts = np.zeros(self.nlist + 1, np.int64)
-        np.cumsum(sizes, out=starts[1:])
-        ids = np.fromiter((i for l in self._lists for i in l), np.int32, count=int(starts[-1]))
+        ids, starts, sizes = self._flat_lists()
         valid = probes >= 0
         cell = np.where(valid, probes, 0)
         seg_off = np.where(valid, starts[cell], 0)

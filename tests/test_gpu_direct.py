@@ -103,3 +103,51 @@ def test_scores_past_fp32(vs, metric, k):
     xq = (syn.normal_unit(3, 8, 5, 1) * np.float32(100.0)).astype(np.float32)
     _check(vs, xb, xq, 40 if k == 5 else k, metric, "f32")
     _check(vs, xb, xq, k, metric, "f32")
+
+
+@pytest.mark.parametrize("storage,metric,d", [("f32", 0, 70), ("f32", 1, 32), ("bf16", 0, 33), ("bf16", 1, 128)])
+@pytest.mark.parametrize("nq,nseg,k", [(3, 1, 5), (40, 30, 10), (5, 4, 1500), (2, 3, 8192)])
+def test_subset_keys(vs, storage, metric, d, nq, nseg, k):
+    """Segments of every length from 0 to past four waves' rows, pairs walked
+    in index order and by segment (1,024 pairs and more), k past the subset."""
+    g = syn.rng(nq, nseg)
+    xb = g.standard_normal((5000, d)).astype(np.float32)
+    xq = g.standard_normal((nq, d)).astype(np.float32)
+    if storage == "bf16":
+        xb = syn.bf16_bits_to_f32(syn.to_bf16_bits(xb))
+    idx = vs.GpuIndexFlat(d, vs.Metric(metric), storage=storage)
+    idx.add(xb)
+    ids = g.permutation(5000).astype(np.int32)
+    cut = np.sort(g.choice(5001, size=nseg * 2, replace=False))
+    off = np.stack([cut[0::2]] * nq)
+    ln = np.stack([(cut[1::2] - cut[0::2]) * (np.arange(nseg) % 3 != 1)] * nq)
+    ln[0] = 0
+    r = idx.search_subsets(xq, k, ids, off, ln)
+    idx.close()
+    for q in range(nq):
+        rows = np.concatenate([ids[o:o + l] for o, l in zip(off[q], ln[q])]).astype(np.int64)
+        m = min(k, len(rows))
+        assert np.all(r.ids[q, m:] == -1)
+        if m:
+            order = np.sort(rows)
+            Dr, Ir = oracle.flat_search(xb[order], xq[q:q + 1], m, metric, 1)
+            assert np.array_equal(r.distances[q, :m], Dr[0])
+            assert_knn_parity(r.distances[q:q + 1, :m], r.ids[q:q + 1, :m], Dr,
+                              order[Ir].astype(np.int32), metric, rtol=0.0, atol=0.0)
+
+
+def test_subset_repeats_and_bad_ids(vs):
+    """A row named thousands of times (past the selection's buffer) comes back
+    as often; an id outside the index fails the call."""
+    xb = syn.normal_unit(100, 16, 3, 0)
+    idx = vs.GpuIndexFlat.l2(16, storage="f32")
+    idx.add(xb)
+    ids = np.concatenate([np.full(9000, 7), np.arange(100)]).astype(np.int32)
+    r = idx.search_subsets(xb[7:8] + np.float32(0.01), 20, ids, [[0]], [[len(ids)]])
+    assert np.all(r.ids == 7) and np.all(r.distances == r.distances[0, 0])
+    r = idx.search_subsets(xb[50:51], 20, ids, [[0]], [[len(ids)]])
+    assert r.ids[0, 0] == 50
+    ids[-1] = 100
+    with pytest.raises(ValueError):
+        idx.search_subsets(xb[:1], 2, ids, [[0]], [[len(ids)]])
+    idx.close()
