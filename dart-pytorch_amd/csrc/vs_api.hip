@@ -423,29 +423,6 @@ int ensure_capacity(vs_index *x, int64_t need) {
     return VS_OK;
 }
 
-// Validation of n rows already on the device: returns flags.
-int device_flags(vs_index *x, const void *src, int dtype, int64_t stride, int64_t n, uint32_t *out) {
-    VS_HIP(x->flags.ensure(sizeof(uint32_t)), "flags buffer");
-    VS_HIP(hipMemsetAsync(x->flags.p, 0, sizeof(uint32_t), x->st), "clearing flags");
-    // store_rows with a throw-away destination computes the flags: use the
-    // misc buffer sized for one chunk of rows.
-    const int64_t chunk = 1 << 16;
-    for (int64_t r = 0; r < n; r += chunk) {
-        const int64_t m = std::min(chunk, n - r);
-        const int64_t dst_ld = vs::storage_ld(x->d, 0);
-        VS_HIP(x->misc.ensure((size_t)m * dst_ld * 4 + (size_t)m * 4), "validation scratch");
-        const char *s = (const char *)src + (size_t)r * stride * (dtype == 1 ? 2 : 4);
-        VS_HIP(vs::launch_store_rows(s, dtype, stride, m, x->d, x->misc.p, 0, dst_ld,
-                                     (float *)((char *)x->misc.p + (size_t)m * dst_ld * 4),
-                                     x->flags.as<uint32_t>(), x->st),
-               "validating rows");
-    }
-    VS_HIP(hipMemcpyAsync(out, x->flags.p, sizeof(uint32_t), hipMemcpyDeviceToHost, x->st),
-           "reading flags");
-    VS_HIP(hipStreamSynchronize(x->st), "validating rows");
-    return VS_OK;
-}
-
 // Switch bf16 storage to fp32 (AUTO storage meeting a non-bf16 value).
 int widen_storage(vs_index *x) {
     const int64_t new_ld = vs::storage_ld(x->d, 0);
@@ -480,24 +457,62 @@ int widen_storage(vs_index *x) {
     return VS_OK;
 }
 
-int add_device_rows(vs_index *x, const void *src, int dtype, int64_t n) {
-    uint32_t f = 0;
-    int rc = device_flags(x, src, dtype, x->d, n, &f);
-    if (rc) return rc;
-    if (f & vs::kFlagNonFinite)
-        return set_err(VS_ERR_NONFINITE, "vectors contain NaN or infinity");
-    if (x->mode == VS_STORAGE_AUTO && x->storage == 1 && (f & vs::kFlagNotBf16)) {
-        rc = widen_storage(x);
-        if (rc) return rc;
-    }
-    rc = ensure_capacity(x, x->ntotal + n);
-    if (rc) return rc;
+// Stores n device rows from row `at` on (at >= ntotal, within the capacity)
+// and reads their flags.  One pass validates and stores: the rows count only
+// once the caller raises ntotal.
+int store_checked(vs_index *x, const void *src, int dtype, int64_t at, int64_t n, uint32_t *f) {
     VS_HIP(x->flags.ensure(sizeof(uint32_t)), "flags buffer");
-    char *dst = (char *)x->xb + (size_t)x->ntotal * row_bytes(x);
-    VS_HIP(vs::launch_store_rows(src, dtype, x->d, n, x->d, dst, x->storage, x->ld,
-                                 x->xn + x->ntotal, x->flags.as<uint32_t>(), x->st),
+    VS_HIP(vs::launch_fill32(x->flags.p, 1, 0u, x->st), "clearing flags");
+    char *dst = (char *)x->xb + (size_t)at * row_bytes(x);
+    VS_HIP(vs::launch_store_rows(src, dtype, x->d, n, x->d, dst, x->storage, x->ld, x->xn + at,
+                                 x->flags.as<uint32_t>(), x->st),
            "storing rows");
+    VS_HIP(hipMemcpyAsync(f, x->flags.p, sizeof(uint32_t), hipMemcpyDeviceToHost, x->st),
+           "reading flags");
     VS_HIP(hipStreamSynchronize(x->st), "storing rows");
+    return VS_OK;
+}
+
+// Rows past ntotal are zero again, up to row `end` (an add that failed, or
+// starts over, after it stored some).
+int clear_rows(vs_index *x, int64_t end) {
+    if (end <= x->ntotal) return VS_OK;
+    const size_t m = (size_t)(end - x->ntotal);
+    VS_HIP(hipMemsetAsync((char *)x->xb + (size_t)x->ntotal * row_bytes(x), 0, m * row_bytes(x),
+                          x->st),
+           "clearing rows");
+    VS_HIP(hipMemsetAsync(x->xn + x->ntotal, 0, m * sizeof(float), x->st), "clearing norms");
+    VS_HIP(hipStreamSynchronize(x->st), "clearing rows");
+    return VS_OK;
+}
+
+// Appends n rows, all or none: chunks of `chunk` rows, fetch(r, m) giving the
+// device address of rows [r, r + m).
+template <typename Fetch>
+int add_rows(vs_index *x, int dtype, int64_t n, int64_t chunk, Fetch &&fetch) {
+    if (int rc = ensure_capacity(x, x->ntotal + n)) return rc;
+    for (int64_t r = 0; r < n;) {
+        const int64_t m = std::min(chunk, n - r);
+        const void *src = nullptr;
+        uint32_t f = 0;
+        int rc = fetch(r, m, &src);
+        if (!rc) rc = store_checked(x, src, dtype, x->ntotal + r, m, &f);
+        if (!rc && (f & vs::kFlagNonFinite))
+            rc = set_err(VS_ERR_NONFINITE, "vectors contain NaN or infinity");
+        if (rc) {
+            (void)clear_rows(x, x->ntotal + r + m);
+            return rc;
+        }
+        if (x->mode == VS_STORAGE_AUTO && x->storage == 1 && (f & vs::kFlagNotBf16)) {
+            // fp32 from here on: the rows so far are stored again
+            rc = clear_rows(x, x->ntotal + r + m);
+            if (!rc) rc = widen_storage(x);
+            if (rc) return rc;
+            r = 0;
+            continue;
+        }
+        r += m;
+    }
     x->ntotal += n;
     ++x->version;
     return VS_OK;
@@ -2063,43 +2078,18 @@ int vs_index_add(vs_index *x, const void *xs, int src_dtype, int64_t n) {
     DeviceGuard g(x->device);
     const int64_t es = src_dtype == 1 ? 2 : 4;
     const int64_t rowb = x->d * es;
-    // validate everything before storing anything (add is all-or-nothing)
     const int64_t chunk = std::max<int64_t>(1, (int64_t)(256 << 20) / rowb);
-    bool any_not_bf16 = false;
-    for (int64_t r = 0; r < n; r += chunk) {
-        const int64_t m = std::min(chunk, n - r);
+    int64_t held = -1;  // the staging buffer holds the chunk at this row
+    return add_rows(x, src_dtype, n, chunk, [&](int64_t r, int64_t m, const void **src) {
         VS_HIP(x->stage.ensure((size_t)m * rowb), "staging buffer");
-        VS_HIP(hipMemcpyAsync(x->stage.p, (const char *)xs + (size_t)r * rowb, (size_t)m * rowb,
-                              hipMemcpyHostToDevice, x->st),
-               "uploading vectors");
-        uint32_t f = 0;
-        int rc = device_flags(x, x->stage.p, src_dtype, x->d, m, &f);
-        if (rc) return rc;
-        if (f & vs::kFlagNonFinite)
-            return set_err(VS_ERR_NONFINITE, "vectors contain NaN or infinity");
-        any_not_bf16 |= (f & vs::kFlagNotBf16) != 0;
-    }
-    if (x->mode == VS_STORAGE_AUTO && x->storage == 1 && any_not_bf16) {
-        int rc = widen_storage(x);
-        if (rc) return rc;
-    }
-    int rc = ensure_capacity(x, x->ntotal + n);
-    if (rc) return rc;
-    VS_HIP(x->flags.ensure(sizeof(uint32_t)), "flags buffer");
-    for (int64_t r = 0; r < n; r += chunk) {
-        const int64_t m = std::min(chunk, n - r);
-        VS_HIP(hipMemcpyAsync(x->stage.p, (const char *)xs + (size_t)r * rowb, (size_t)m * rowb,
-                              hipMemcpyHostToDevice, x->st),
-               "uploading vectors");
-        char *dst = (char *)x->xb + (size_t)(x->ntotal + r) * row_bytes(x);
-        VS_HIP(vs::launch_store_rows(x->stage.p, src_dtype, x->d, m, x->d, dst, x->storage, x->ld,
-                                     x->xn + x->ntotal + r, x->flags.as<uint32_t>(), x->st),
-               "storing rows");
-        VS_HIP(hipStreamSynchronize(x->st), "storing rows");
-    }
-    x->ntotal += n;
-    ++x->version;
-    return VS_OK;
+        if (held != r)
+            VS_HIP(hipMemcpyAsync(x->stage.p, (const char *)xs + (size_t)r * rowb, (size_t)m * rowb,
+                                  hipMemcpyHostToDevice, x->st),
+                   "uploading vectors");
+        held = r;
+        *src = x->stage.p;
+        return (int)VS_OK;
+    });
 }
 
 int vs_index_add_device(vs_index *x, const void *xs_dev, int src_dtype, int64_t n) {
@@ -2111,7 +2101,10 @@ int vs_index_add_device(vs_index *x, const void *xs_dev, int src_dtype, int64_t 
     if (x->ntotal + n > (int64_t)INT32_MAX)
         return set_err(VS_ERR_INVALID, "ids are int32: ntotal + n must stay below 2^31");
     DeviceGuard g(x->device);
-    return add_device_rows(x, xs_dev, src_dtype, n);
+    return add_rows(x, src_dtype, n, n, [&](int64_t, int64_t, const void **src) {
+        *src = xs_dev;
+        return (int)VS_OK;
+    });
 }
 
 int vs_index_reconstruct(vs_index *x, int64_t i0, int64_t n, float *out) {

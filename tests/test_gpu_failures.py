@@ -121,3 +121,33 @@ def test_device_probes(vs):
     assert 100.0 < vals[1] <= 2600.0 and 100.0 < vals[2] <= 2600.0
     v = ctypes.c_double(0.0)
     assert lib.vs_dev_probe(0, 3, 0, ctypes.byref(v)) == N.VS_ERR_INVALID
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16", "auto"])
+def test_add_is_all_or_nothing(vs, storage):
+    """Rows are stored while they are checked: an add that meets a NaN leaves
+    the index as it was, and so does the space it had written to (the next
+    add, and tiles read past the last row, find zeros there)."""
+    xb, xq = syn.int_grid(700, 24, 3, 0), syn.int_grid(9, 24, 3, 1)
+    idx = vs.GpuIndexFlat.l2(24, storage=storage)
+    idx.add(xb[:300])
+    bad = xb[300:].copy()
+    bad[333, 7] = np.nan
+    with pytest.raises(vs.VsError):
+        idx.add(bad)
+    assert idx.ntotal == 300
+    for rows in (xb[:300], xb):
+        if len(rows) > 300:
+            idx.add(xb[300:])
+        idx.set_option("direct", 0)
+        r = idx.search(xq, 12)
+        Dr, Ir = oracle.flat_search(rows, xq, 12, 0, NT)
+        assert_knn_parity(r.distances, r.ids, Dr, Ir, 0, rtol=0.0, atol=0.0, xb=rows, xq=xq)
+    if storage == "auto":  # and one that widens the storage
+        idx.add(xb[:50] + np.float32(0.3))
+        rows = np.concatenate([xb, xb[:50] + np.float32(0.3)])
+        r = idx.search(xq, 12)
+        Dr, Ir = oracle.flat_search(rows, xq, 12, 0, NT)
+        assert idx.storage == "f32"
+        assert_knn_parity(r.distances, r.ids, Dr, Ir, 0, rtol=0.0, atol=0.0, xb=rows, xq=xq)
+    idx.close()
