@@ -263,6 +263,7 @@ struct vs_index {
     DevBuf xb16;
     int64_t copy_ld = 0, copy_n = 0, copy_cap = 0;
     float copy_res = 0.f;  // largest |row - copied row| (an upper bound)
+    uint64_t copy_asked = ~0ull;  // version of the rows at a call that went without the copy
     std::atomic_flag copy_busy = ATOMIC_FLAG_INIT;  // held by a call that reads the copy
     // the rows that the current call's scans and planning read
     struct {
@@ -1171,13 +1172,23 @@ int xnorm_max(vs_index *x, Arena &A, float *out) {
 }
 
 // Brings the bf16 copy of fp32 rows up to date (rows added since the last
-// call are appended); false if there is none: the copy is optional, and taken
-// only where it leaves three quarters of the free memory to others.  The
-// caller holds it (CopyHold).  One wait, when rows were copied.
-bool ensure_copy16(vs_index *x) {
+// call are appended) for a call of nq queries; false if there is none: the
+// copy is optional, and taken only where it leaves three quarters of the free
+// memory to others.  The caller holds it (CopyHold).  One wait, when rows were
+// copied.  Copying a row costs about three times what a small batch saves by
+// reading the copy instead (6 bytes against 2), and a batch of 200 saves that
+// much again in matrix passes: a call that would copy more than it saves does
+// so only if it is not the first on these rows.
+bool ensure_copy16(vs_index *x, int64_t nq) {
     if (x->storage != 0 || x->ntotal == 0) return false;
     const int64_t ld16 = vs::storage_ld(x->d, 1);
     if (x->copy_n == x->ntotal && x->copy_cap >= x->ntotal) return std::isfinite(x->copy_res);
+    const int64_t pending = x->copy_cap < x->ntotal ? x->ntotal : x->ntotal - x->copy_n;
+    if ((double)pending > (double)x->ntotal * (0.3 + (double)nq / 200.0) &&
+        x->copy_asked != x->version) {
+        x->copy_asked = x->version;
+        return false;
+    }
     const size_t rb = (size_t)ld16 * 2;
     auto fail = [&] {
         (void)hipGetLastError();
@@ -1582,7 +1593,7 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
     select_rows(x);
     CopyHold hold(x);
     const bool coarse = !safe && !A.fixed() && hold.mine && coarse_search(x, k) &&
-                        ensure_copy16(x);
+                        ensure_copy16(x, nq);
     if (coarse) select_copy(x);
     // control words: merge flags, the counts of the two lists, then the
     // query flags of bf16 queries (read with the results)
@@ -1775,7 +1786,7 @@ int range_core(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int6
     // without one, rounds them in the GEMM-tiled scan where that applies.
     CopyHold hold(x);
     const bool copy = x->storage == 0 && x->opt.coarse && x->opt.copy16 && hold.mine &&
-                      ensure_copy16(x);
+                      ensure_copy16(x, nq);
     if (copy) select_copy(x);
     Arena A;
     vs::PreparedQueries pq;

@@ -22,7 +22,9 @@ def _index(vs, xb, metric, **options):
 
 
 def _check(idx, xb, xq, k, metric, sub=1):
+    first = idx.search(xq, k)  # (a small batch copies the rows from its second call on)
     r = idx.search(xq, k)
+    assert np.array_equal(first.distances, r.distances) and np.array_equal(first.ids, r.ids)
     s = np.arange(0, len(xq), sub)
     Dr, Ir = oracle.flat_search(xb, xq[s], k, metric, NT)
     assert_knn_parity(r.distances[s], r.ids[s], Dr, Ir, metric, rtol=0.0, atol=0.0)
