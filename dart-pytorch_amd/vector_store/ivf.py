@@ -39,6 +39,7 @@ class IndexIVFFlat(Index):
         self.is_trained = False
         self._lists = [[] for _ in range(self.nlist)]
         self._flat = None  # (ids of every list one after another, starts, sizes)
+        self._lent = False  # a caller holds the lists and may change them at any time
 
     @property
     def ntotal(self) -> int:
@@ -47,7 +48,7 @@ class IndexIVFFlat(Index):
     @property
     def inv_lists(self):
         """invLists (index_ivf_flat.dart:52-55): ids per cell, insertion order."""
-        self._flat = None  # the caller may change them
+        self._lent = True
         return self._lists
 
     def close(self) -> None:
@@ -78,16 +79,16 @@ class IndexIVFFlat(Index):
         self._flat = None
 
     def _flat_lists(self):
-        """The inverted lists as one id array, laid out again when rows or
-        lists have changed."""
-        total = sum(map(len, self._lists))
-        if self._flat is None or self._flat[0].size != total:
+        """The inverted lists as one id array, kept until rows are added; laid
+        out for every call once `inv_lists` has given the lists away."""
+        flat = None if self._lent else self._flat
+        if flat is None:
             sizes = np.array([len(l) for l in self._lists], np.int64)
             starts = np.zeros(self.nlist + 1, np.int64)
             np.cumsum(sizes, out=starts[1:])
             ids = np.fromiter((i for l in self._lists for i in l), np.int32, count=int(starts[-1]))
-            self._flat = (ids, starts, sizes)
-        return self._flat
+            flat = self._flat = (ids, starts, sizes)
+        return flat
 
     def search(self, queries, k: int) -> SearchResult:
         if not self.is_trained:
