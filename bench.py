@@ -287,7 +287,6 @@ def run_search(vs, NN, workload, args, ctx, full=False):
     bf16 = idx.storage == "bf16"
     traffic, tsrc = MEASURED_TRAFFIC.get((workload, n, nq, k), (None, None))
     roof = roofline("mfma", 2.0 * nq * n * d, scan_s, ctx["peaks"], "scan", nscan, traffic, tsrc,
-                    peak_div=1 if bf16 else 3,
                     extra={"scan_kinds": {f: idx.prof_get(f)[0] for f in
                                           ("shared", "gemm", "streamed", "direct")
                                           if idx.prof_get(f)[0]},
