@@ -242,6 +242,13 @@ hipError_t launch_exact_tile(const void *xb, int storage, int64_t ld, int64_t d,
 // ---------------------------------------------------------------------------
 constexpr uint64_t kNoKey = ~0ull;
 constexpr int kSelBins = 2048, kSelThreads = 1024, kSelRegKeys = 10;
+// Places in a segment of up to INT32_MAX keys.  The walk looks up to eight
+// rounds past the last key, which 32 signed bits do not count to.
+typedef uint32_t sel_pos_t;
+constexpr int kSelUnroll = 8;
+static_assert((uint64_t)INT32_MAX + 2ull * kSelUnroll * kSelThreads <= (sel_pos_t)~(sel_pos_t)0 &&
+                  (sel_pos_t)~(sel_pos_t)0 > 0,
+              "a place past the last key neither wraps nor turns negative");
 
 struct SelectKeysArgs {
     const uint64_t *keys;
@@ -321,15 +328,16 @@ __global__ __launch_bounds__(kSelThreads) void select_keys_kernel(SelectKeysArgs
             for (int u = 0; u < kSelRegKeys; ++u)
                 if (reg[u] != kNoKey) f(reg[u]);
         } else {
-            for (int t0 = tid; t0 < m; t0 += 8 * kSelThreads) {
-                uint64_t v[8];  // eight loads in flight
+            const sel_pos_t end = (sel_pos_t)m;
+            for (sel_pos_t t0 = tid; t0 < end; t0 += kSelUnroll * kSelThreads) {
+                uint64_t v[kSelUnroll];  // that many loads in flight
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const int t = t0 + u * kSelThreads;
-                    v[u] = t < m ? kp[t] : kNoKey;
+                for (int u = 0; u < kSelUnroll; ++u) {
+                    const sel_pos_t t = t0 + u * kSelThreads;
+                    v[u] = t < end ? kp[t] : kNoKey;
                 }
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
+                for (int u = 0; u < kSelUnroll; ++u)
                     if (v[u] != kNoKey) f(v[u]);
             }
         }
