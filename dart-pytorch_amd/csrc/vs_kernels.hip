@@ -954,6 +954,11 @@ __device__ void select_block(float *sv, int *si, int n, int kk, float *tmp_v, in
     __syncthreads();
 }
 
+// Whether partial sums of at most this magnitude (|x|^2 + s |q| |x| bounds
+// those of an accumulator) stay numbers in fp32, rounding of the operands
+// included; false for NaN.
+__device__ __forceinline__ bool acc_in_range(double most) { return most < 1e38; }
+
 template <int ST, int MODE, int MU>
 __global__ __launch_bounds__(256) void merge_refine_kernel(MergeKArgs a) {
     constexpr int MBUF = kMergeBuf * MU;
@@ -1200,8 +1205,6 @@ __global__ __launch_bounds__(256) void merge_refine_kernel(MergeKArgs a) {
                 for (int64_t j = tid; j < a.d; j += 64) qq += (double)qsh[j] * (double)qsh[j];
                 for (int o = 32; o > 0; o >>= 1) qq += __shfl_xor(qq, o);
             }
-            // (an operand past bf16's range leaves accumulators that are not
-            // numbers, and fewer candidates than rows)
             // One-pass selection: rows the merge does not hold lie at or above
             // its kk-th value, the query's final shared threshold or their
             // list's own, whichever is lowest.
@@ -1210,10 +1213,21 @@ __global__ __launch_bounds__(256) void merge_refine_kernel(MergeKArgs a) {
                 dropped = fminf(dropped, tfinal);
                 if (a.lbound || a.guess) dropped = fminf(dropped, s_lo);
             }
-            const bool lost = a.qres && (bi[a.k - 1] == INT_MAX ? a.nrows >= a.k
-                                                                : dropped == VS_INF && a.nrows >= kk);
+            // An operand past bf16's range, or a row norm past fp32's, leaves
+            // accumulators that are infinite or not numbers: their rows are
+            // in no list, and the merge holds fewer than a selection within
+            // bounds always finds.  Such a query is searched again -- after
+            // an estimate, which may have been too tight, with full lists
+            // first.
+            const int64_t most = min(a.nrows, (int64_t)kk);
+            const bool lost = a.qres ? (bi[a.k - 1] == INT_MAX ? a.nrows >= a.k
+                                                               : dropped == VS_INF && a.nrows >= kk)
+                                     : bi[most - 1] == INT_MAX;
             if (tid == 0 && !s_vf && lost) {
-                a.vf_list[atomicAdd(a.vf_count, 1)] = (int32_t)qg;
+                if (a.qres)
+                    a.vf_list[atomicAdd(a.vf_count, 1)] = (int32_t)qg;
+                else
+                    a.vx_list[atomicAdd(a.vx_count, 1)] = (int32_t)qg;
             } else if (tid == 0 && !s_vf && bi[a.k - 1] != INT_MAX && dropped < VS_INF) {
                 const double s = a.metric == 0 ? 2.0 : 1.0;
                 const double qn = a.qnorm[qg], xm = a.xmax;
@@ -1226,7 +1240,10 @@ __global__ __launch_bounds__(256) void merge_refine_kernel(MergeKArgs a) {
                 const double key = bv[a.k - 1];
                 double ek = key + fabs(key) * (1.0 / 8388608.0);
                 if (a.metric == 0) ek -= qq * (1.0 - 1e-12);  // qq: fp64 sum, error < d 2^-53 qq
-                if (!(ek < (double)dropped - err)) a.vx_list[atomicAdd(a.vx_count, 1)] = (int32_t)qg;
+                // (err bounds accumulators that stay within fp32's range)
+                if (!(ek < (double)dropped - err) ||
+                    !acc_in_range((a.metric == 0 ? xm * xm : 0.0) + s * qn * xm))
+                    a.vx_list[atomicAdd(a.vx_count, 1)] = (int32_t)qg;
             }
         }
     } else {
@@ -2652,10 +2669,15 @@ __global__ __launch_bounds__(256) void bounded_thr_kernel(
     const int lane = threadIdx.x & 63;
     if (q >= m) return;
     double qq = 0.0;
-    if (metric == 0) {
-        for (int64_t j = lane; j < d; j += 64) qq += (double)qf[q * d + j] * (double)qf[q * d + j];
-        for (int o = 32; o > 0; o >>= 1) qq += __shfl_xor(qq, o);
+    bool past = false;  // an element whose operand bf16 rounds to infinity
+    const float scale = metric == 0 ? 2.0f : 1.0f;
+    for (int64_t j = lane; j < d; j += 64) {
+        const float v = qf[q * d + j];
+        qq += (double)v * (double)v;
+        past |= (f32_to_bf16_rne(fabsf(v * scale)) & 0x7F80u) == 0x7F80u;
     }
+    for (int o = 32; o > 0; o >>= 1) qq += __shfl_xor(qq, o);
+    past = __ballot(past) != 0;
     if (lane) return;
     const double s = metric == 0 ? 2.0 : 1.0;
     const double qn = qnorm[q], xm = xmax;
@@ -2668,9 +2690,12 @@ __global__ __launch_bounds__(256) void bounded_thr_kernel(
     double ek = key + fabs(key) * (1.0 / 8388608.0);
     if (metric == 0) ek -= qq * (1.0 - 1e-12);
     const float t = (float)(ek + err), b = t + fabsf(t) * 1e-6f + 1e-30f;
-    // no finite bound (norms past fp32's range): no candidates, which sends
-    // the query on to the exact path
-    athr[q] = __builtin_isfinite(b) ? b : -VS_INF;
+    // accumulators that may be infinite or not numbers: a bound that none of
+    // them meets (-inf would meet -inf), so that no candidates send the query
+    // on to the exact path
+    const bool ok = __builtin_isfinite(b) && !past &&
+                    acc_in_range((metric == 0 ? xm * xm : 0.0) + s * qn * xm);
+    athr[q] = ok ? b : __builtin_nanf("");
 }
 
 hipError_t launch_bounded_thresholds(const PreparedQueries &pq, int64_t d, int metric,

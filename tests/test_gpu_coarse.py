@@ -93,16 +93,66 @@ def test_copy_follows_the_rows(vs):
     assert np.array_equal(rr.limits, lims) and np.array_equal(rr.ids, I)
 
 
-@pytest.mark.parametrize("scale", [1e-25, 1e15, 3.395e38])
-def test_extreme_magnitudes(vs, scale):
-    """Rows whose rounding residual underflows or whose bf16 rounding
-    overflows: proven or searched again, never wrong."""
+@pytest.mark.parametrize("metric", [0, 1])
+@pytest.mark.parametrize("scale", [1e-25, 1e15, 3.395e38, 3.4e38])
+def test_extreme_magnitudes(vs, scale, metric):
+    """Rows whose rounding residual underflows, is large, has a square past
+    fp32 (the rows are then not copied) or is itself infinite (the largest
+    elements round past bf16's range): proven or searched again, never wrong."""
     xb = (syn.normal_unit(3000, 16, 4, 0)).astype(np.float32)
     xb /= np.abs(xb).max()
     xb = (xb * np.float32(scale)).astype(np.float32)
     xq = syn.normal_unit(20, 16, 4, 1) * np.float32(1e-3)
-    idx = _index(vs, xb, 1)
-    _check(idx, xb, xq, 7, 1)
+    idx = _index(vs, xb, metric)
+    _check(idx, xb, xq, 7, metric)
+    idx.close()
+
+
+@pytest.mark.parametrize("spread", [1e12, 1e14])
+def test_accumulators_past_fp32(vs, spread):
+    """Operands that bf16 holds whose partial sums leave fp32's range on the
+    way to a score within it: the best rows' accumulators are not numbers."""
+    g = syn.rng(9, 0)
+    xb = np.zeros((4000, 24), np.float32)
+    xb[:, 0] = np.float32(spread) * g.random(4000, dtype=np.float32)
+    xb[100:120, 0] = 1e15
+    xb[100:120, 1] = -1e15 * (0.7 + 0.01 * np.arange(20))
+    xq = np.zeros((20, 24), np.float32)
+    xq[:, :2] = 1e24
+    xq[:, 2:] = g.standard_normal((20, 22))
+    for storage in ("f32", "bf16"):
+        rows = xb if storage == "f32" else syn.bf16_bits_to_f32(syn.to_bf16_bits(xb))
+        idx = vs.GpuIndexFlat(24, vs.Metric(1), storage=storage)
+        idx.set_option("direct", 0)
+        idx.add(rows)
+        for _ in range(2):
+            r = idx.search(xq, 9)
+            Dr, Ir = oracle.flat_search(rows, xq, 9, 1, NT)
+            assert_knn_parity(r.distances, r.ids, Dr, Ir, 1, rtol=0.0, atol=0.0)
+        idx.close()
+
+
+# streaming scan without and with an estimate, row-shared and GEMM-tiled scan
+@pytest.mark.parametrize("n,d,nq", [(3000, 16, 3), (20_000, 40, 40), (20_000, 128, 300), (5000, 300, 600)])
+@pytest.mark.parametrize("metric,storage", [(0, "f32"), (1, "f32"), (1, "bf16")])
+def test_queries_past_bf16(vs, n, d, nq, metric, storage):
+    """Queries that bf16 rounds to infinity: accumulators are not numbers, and
+    the scans find fewer candidates than rows, or none."""
+    xb = syn.normal_unit(n, d, 4, 0)
+    xq = syn.normal_unit(nq, d, 4, 1)
+    xq[:nq // 2 + 1] /= np.abs(xq[:nq // 2 + 1]).max(axis=1, keepdims=True)
+    xq[:nq // 2 + 1] *= np.float32(3.4e38)
+    xb *= np.float32(0.1)
+    if storage == "bf16":
+        xb = syn.bf16_bits_to_f32(syn.to_bf16_bits(xb))
+    idx = vs.GpuIndexFlat(d, vs.Metric(metric), storage=storage)
+    idx.set_option("direct", 0)
+    idx.add(xb)
+    for _ in range(2):
+        r = idx.search(xq, 7)
+        assert np.all(r.ids >= 0)
+        Dr, Ir = oracle.flat_search(xb, xq[::7], 7, metric, NT)
+        assert_knn_parity(r.distances[::7], r.ids[::7], Dr, Ir, metric, rtol=0.0, atol=0.0)
     idx.close()
 
 
