@@ -1,0 +1,75 @@
+"""Rows long enough that a scan's query block only just fits the LDS: range
+search takes every dimension up to the block's own size, and a query that has
+to be searched again is."""
+import numpy as np
+import pytest
+
+import oracle
+from _parity import assert_knn_parity, assert_range_parity
+from vector_store import synthetic as syn
+
+pytestmark = pytest.mark.gpu
+NT = oracle.default_threads()
+
+
+def _bf16(x):
+    return syn.bf16_bits_to_f32(syn.to_bf16_bits(x))
+
+
+def _index(vs, xb, metric, storage, **options):
+    idx = vs.GpuIndexFlat(xb.shape[1], vs.Metric(metric), storage=storage)
+    idx.set_option("direct", 0)
+    for name, value in options.items():
+        idx.set_option(name, value)
+    idx.add(xb)
+    return idx
+
+
+# the longest rows of the streaming scan, whose 16-query block then fills the
+# LDS but for 64-entry wave buffers: two query planes beside fp32 rows and
+# beside bf16 rows, and one plane
+EDGES = [("f32", 2496, False), ("f32", 2400, False), ("bf16", 2432, False), ("bf16", 4992, True),
+         ("f32", 4992, True)]
+
+
+@pytest.mark.parametrize("storage,d,bf16_queries", EDGES)
+@pytest.mark.parametrize("copy16", [0, 1])
+def test_range_at_the_longest_rows(vs, storage, d, bf16_queries, copy16):
+    xb, xq = syn.normal_unit(600, d, d, 0), syn.normal_unit(9, d, d, 1)
+    xb[:90] = np.repeat(xq, 10, axis=0) + 0.005 * xb[:90]
+    if storage == "bf16":
+        xb = _bf16(xb)
+    if bf16_queries:
+        xq = _bf16(xq)
+    for metric, radius in ((0, 0.5), (1, 0.8)):
+        idx = _index(vs, xb, metric, storage, copy16=copy16)
+        got = [idx.range_search(xq, radius) for _ in range(2)]
+        idx.close()
+        lims, D, I = oracle.flat_range_search(xb, xq, radius, metric, NT)
+        assert lims[-1] >= 90
+        for rr in got:
+            assert_range_parity(rr.limits, rr.distances, rr.ids, lims, D, I)
+
+
+@pytest.mark.parametrize("storage,d,bf16_queries", EDGES)
+def test_unproven_queries_of_the_longest_rows(vs, storage, d, bf16_queries):
+    """Near-copies of the queries, closer to each other than the selection's
+    error: every query is searched again."""
+    g = syn.rng(d, 5)
+    base = syn.normal_unit(3, d, d, 6)
+    xb = np.concatenate([np.repeat(base, 200, axis=0), syn.normal_unit(400, d, d, 7)])
+    j = g.integers(0, d, (600, 4))
+    for r in range(600):  # a few elements moved by less than the others' rounding
+        xb[r, j[r]] *= np.float32(1.0 + 2.0 ** -12 if storage == "f32" else 1.0 + 2.0 ** -7)
+    if storage == "bf16":
+        xb = _bf16(xb)
+    xq = _bf16(base) if bf16_queries else base
+    for metric in (0, 1):
+        idx = _index(vs, xb, metric, storage, copy16=0)
+        idx.prof_reset()
+        r = idx.search(xq, 10)
+        again = idx.prof_get("exact_fallback")[0]
+        idx.close()
+        Dr, Ir = oracle.flat_search(xb, xq, 10, metric, NT)
+        assert_knn_parity(r.distances, r.ids, Dr, Ir, metric, rtol=0.0, atol=0.0)
+        assert storage == "bf16" or again == 3
