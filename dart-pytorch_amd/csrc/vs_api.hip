@@ -742,8 +742,7 @@ int plan_scan_core(const vs_index *x, int64_t nq, int64_t nrows, int planes, int
     if (safe) kk = kk_final;
     p->kk_final = (int)kk_final;
     p->kk = (int)kk;
-    // range: the cap is that of the waves' pair buffers
-    p->cap = range ? 256 : (int)next_pow2(kk + 48);
+    p->cap = (int)next_pow2(kk + 48);
     // 16-row blocks per wave tile: one for short rows (d <= 128: measured
     // faster on 1M x 128, the epilogue dominates), two otherwise
     p->tm = x->sel.ld <= 128 && storage == 1 ? 1 : 2;
@@ -762,11 +761,16 @@ int plan_scan_core(const vs_index *x, int64_t nq, int64_t nrows, int planes, int
         if (bn > 16 && round_up(nq, 16) < bn) continue;
         const bool qreg = storage == 1 && planes == 1 && (nks == 4 || nks == 8) &&
                           nks * (bn / 16) <= 16;
-        if (vs::scan_lds_bytes(bn, qreg ? 0 : planes, x->sel.ld, p->cap, 4) <= x->lds_max) {
+        // range: the cap is that of the waves' pair buffers, 256 entries or as
+        // many of them as fit beside the query block (64 always did)
+        for (int cap = range ? 256 : p->cap; cap >= (range ? 64 : p->cap); cap /= 2) {
+            if (vs::scan_lds_bytes(bn, qreg ? 0 : planes, x->sel.ld, cap, 4) > x->lds_max) continue;
             p->bn = bn;
             p->nks = qreg ? nks : 0;
+            p->cap = cap;
             break;
         }
+        if (p->bn) break;
     }
     if (!p->bn)
         return set_err(VS_ERR_UNSUPPORTED,
