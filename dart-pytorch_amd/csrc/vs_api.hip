@@ -1461,8 +1461,8 @@ bool coarse_search(const vs_index *x, int64_t k) {
 // same rows (x->sel) under that bound finds them all; the candidates are
 // scored exactly and the k best selected.  One more scan, whatever the data:
 // rows in clusters tighter than the error leave hundreds of candidates per
-// query, not thousands of products with every row.  Past 2^27 candidates, the
-// exact path.
+// query, not thousands of products with every row.  Past 2^27 candidates, and
+// where the rows are too long for a range scan of m queries, the exact path.
 int bounded_research(vs_index *x, Arena &A, const vs::PreparedQueries &pq, int planes,
                      const vs::TopkCheck &chk, const int32_t *list_dev, int64_t m, int64_t k,
                      float *D, int32_t *I) {
@@ -1485,9 +1485,19 @@ int bounded_research(vs_index *x, Arena &A, const vs::PreparedQueries &pq, int p
                              chk.qres != nullptr);
     if (rc) return rc;
     rq.planes = planes;  // (both planes are written)
+    // the results of the listed queries to their places
+    auto scatter = [&]() -> int {
+        VS_HIP(vs::launch_scatter_rows(fD, (const int32_t *)lst, m, k, D, x->st), "re-search scatter");
+        VS_HIP(vs::launch_scatter_rows(fI, (const int32_t *)lst, m, k, I, x->st), "re-search scatter");
+        return VS_OK;
+    };
+    auto exact = [&]() -> int {
+        const int e = exact_search(x, A, (const float *)fq, m, k, (float *)fD, (int32_t *)fI);
+        return e ? e : scatter();
+    };
     vs::ScanPlan plan;
-    rc = plan_scan(x, m, x->ntotal, planes, 8, x->sel.storage, &plan, false, 0, true);
-    if (rc) return rc;
+    if (plan_scan(x, m, x->ntotal, planes, 8, x->sel.storage, &plan, false, 0, true) != VS_OK)
+        return exact();
     if ((rc = scan_fits(plan, rq))) return rc;
     VS_HIP(x->athr.ensure((size_t)m * 4), "re-search bounds");
     VS_HIP(vs::launch_bounded_thresholds(rq, x->d, x->metric, chk, D, (const int32_t *)lst, k,
@@ -1549,13 +1559,8 @@ int bounded_research(vs_index *x, Arena &A, const vs::PreparedQueries &pq, int p
             return set_err(VS_ERR_HIP, "internal error: a re-search candidate outside the index");
         ok = !(*herr & vs::kFlagShort);
     }
-    if (!ok) {  // too many candidates, or fewer than k (accumulators past fp32)
-        rc = exact_search(x, A, (const float *)fq, m, k, (float *)fD, (int32_t *)fI);
-        if (rc) return rc;
-    }
-    VS_HIP(vs::launch_scatter_rows(fD, (const int32_t *)lst, m, k, D, x->st), "re-search scatter");
-    VS_HIP(vs::launch_scatter_rows(fI, (const int32_t *)lst, m, k, I, x->st), "re-search scatter");
-    return VS_OK;
+    // too many candidates, or fewer than k (accumulators past fp32)
+    return ok ? scatter() : exact();
 }
 
 // Top-k search of nq device query rows into device D / I [nq][k].  safe:
@@ -1625,6 +1630,13 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
         vs::ScanPlan plan;
         rc = plan_scan(x, nq, x->ntotal, pq.planes, kk, x->sel.storage, &plan, safe, 0, false, 8,
                        list_budget);
+        if (rc == VS_ERR_UNSUPPORTED && safe) {
+            // a re-search whose rows are too long for the query block of any
+            // scan (a few queries of a larger batch, or with longer lists)
+            if ((rc = exact_search(x, A, pq.qf, nq, k, D, I))) return rc;
+            VS_HIP(hipStreamSynchronize(x->st), "search");
+            return VS_OK;
+        }
         if (rc) return rc;
         if ((rc = scan_fits(plan, pq))) return rc;
         bool guess = !safe && needs_guess(x, plan, nq);

@@ -73,3 +73,44 @@ def test_unproven_queries_of_the_longest_rows(vs, storage, d, bf16_queries):
         Dr, Ir = oracle.flat_search(xb, xq, 10, metric, NT)
         assert_knn_parity(r.distances, r.ids, Dr, Ir, metric, rtol=0.0, atol=0.0)
         assert storage == "bf16" or again == 3
+
+
+def _close_rows(base, n, d, seed):
+    """n rows per base row: it with a few elements moved by less than bf16 sees."""
+    xb = np.repeat(base, n, axis=0)
+    j = syn.rng(seed, 5).integers(0, d, (len(xb), 4))
+    for r in range(len(xb)):
+        xb[r, j[r]] *= np.float32(1.0 + 2.0 ** -12)
+    return xb
+
+
+@pytest.mark.parametrize("d,copy16", [(3072, 0), (6000, 1)])
+def test_few_unproven_queries_of_a_large_batch(vs, d, copy16):
+    """The GEMM-tiled scan takes rows of any length, from 512 queries on; the
+    three queries it cannot prove have no scan of their own."""
+    base = syn.normal_unit(3, d, d, 6)
+    xb = np.concatenate([_close_rows(base, 100, d, d), syn.normal_unit(500, d, d, 7)])
+    xq = np.concatenate([base, syn.normal_unit(517, d, d, 8)])
+    for metric in (0, 1):
+        idx = _index(vs, xb, metric, "f32", copy16=copy16)
+        for _ in range(2):
+            r = idx.search(xq, 10)
+            s = np.arange(0, 520) < 20
+            Dr, Ir = oracle.flat_search(xb, xq[s], 10, metric, NT)
+            assert_knn_parity(r.distances[s], r.ids[s], Dr, Ir, metric, rtol=0.0, atol=0.0)
+        idx.close()
+
+
+def test_query_past_bf16_on_the_copy(vs):
+    """Found short on the copy, then without a scan of the rows themselves."""
+    d = 3072
+    xb, xq = syn.normal_unit(1500, d, d, 0), syn.normal_unit(150, d, d, 1)
+    xq[2] /= np.abs(xq[2]).max()
+    xq[2] *= np.float32(3.4e38)
+    xb *= np.float32(1e-3)
+    idx = _index(vs, xb, 1, "f32")
+    Dr, Ir = oracle.flat_search(xb, xq, 10, 1, NT)
+    for _ in range(2):
+        r = idx.search(xq, 10)
+        assert_knn_parity(r.distances, r.ids, Dr, Ir, 1, rtol=0.0, atol=0.0)
+    idx.close()
