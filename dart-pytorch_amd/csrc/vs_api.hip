@@ -1182,13 +1182,14 @@ int xnorm_max(vs_index *x, Arena &A, float *out) {
 // copied.  Copying a row costs about three times what a small batch saves by
 // reading the copy instead (6 bytes against 2), and a batch of 200 saves that
 // much again in matrix passes: a call that would copy more than it saves does
-// so only if it is not the first on these rows.
-bool ensure_copy16(vs_index *x, int64_t nq) {
+// so only if it is not the first on these rows, or if it needs the copy (has no
+// scan of the rows themselves).
+bool ensure_copy16(vs_index *x, int64_t nq, bool needed = false) {
     if (x->storage != 0 || x->ntotal == 0) return false;
     const int64_t ld16 = vs::storage_ld(x->d, 1);
     if (x->copy_n == x->ntotal && x->copy_cap >= x->ntotal) return std::isfinite(x->copy_res);
     const int64_t pending = x->copy_cap < x->ntotal ? x->ntotal : x->ntotal - x->copy_n;
-    if ((double)pending > (double)x->ntotal * (0.3 + (double)nq / 200.0) &&
+    if (!needed && (double)pending > (double)x->ntotal * (0.3 + (double)nq / 200.0) &&
         x->copy_asked != x->version) {
         x->copy_asked = x->version;
         return false;
@@ -1249,6 +1250,16 @@ void select_copy(vs_index *x) {
     x->sel.rows = x->xb16.p;
     x->sel.storage = 1;
     x->sel.ld = x->copy_ld;
+}
+
+// Whether the current call's rows (x->sel) have a scan for nq queries in
+// `planes` planes that keeps kk candidates.  Only rows of thousands of
+// elements can lack one, for fewer than 512 queries: no 16-query block fits
+// the LDS then.
+bool has_plan(const vs_index *x, int64_t nq, int planes, int64_t kk, bool range) {
+    if (vs::scan_lds_bytes(16, planes, x->sel.ld, 512, 8) <= x->lds_max) return true;
+    vs::ScanPlan p;
+    return plan_scan(x, nq, x->ntotal, planes, kk, x->sel.storage, &p, false, 0, range) == VS_OK;
 }
 
 // Accumulator error model of a top-k scan of these rows with these queries
@@ -1454,6 +1465,10 @@ bool coarse_search(const vs_index *x, int64_t k) {
            !o.gemm4 && !o.scan_kkw && !o.scan_nw8;
 }
 
+// The candidates that the one-pass selection keeps instead of kk where it
+// starts without an estimate.
+int64_t coarse_keep(int64_t nq, int64_t kk) { return std::max<int64_t>(nq <= 64 ? 64 : 32, 2 * kk); }
+
 // Exact top-k of the m queries listed in list_dev (device) whose selection the
 // merge could not prove, given k results each (any k rows: the k-th exact
 // score e_k among them bounds the true one).  A row of the true top-k has an
@@ -1601,9 +1616,14 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
     int64_t kk = std::max<int64_t>(8, next_pow2(k + std::max<int64_t>(4, k / 4)));
     select_rows(x);
     CopyHold hold(x);
-    const bool coarse = !safe && !A.fixed() && hold.mine && coarse_search(x, k) &&
-                        ensure_copy16(x, nq);
-    if (coarse) select_copy(x);
+    bool coarse = !safe && !A.fixed() && hold.mine && coarse_search(x, k) && ensure_copy16(x, nq);
+    if (coarse) {
+        select_copy(x);
+        // (the copy's rows may be padded further than the rows are)
+        coarse = has_plan(x, nq, 1, kk, false) &&
+                 (kk > 256 || has_plan(x, nq, 1, coarse_keep(nq, kk), false));
+        if (!coarse) select_rows(x);
+    }
     // control words: merge flags, the counts of the two lists, then the
     // query flags of bf16 queries (read with the results)
     void *p_ctl;
@@ -1630,9 +1650,15 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
         vs::ScanPlan plan;
         rc = plan_scan(x, nq, x->ntotal, pq.planes, kk, x->sel.storage, &plan, safe, 0, false, 8,
                        list_budget);
-        if (rc == VS_ERR_UNSUPPORTED && safe) {
-            // a re-search whose rows are too long for the query block of any
-            // scan (a few queries of a larger batch, or with longer lists)
+        if (rc == VS_ERR_UNSUPPORTED && (safe || !A.fixed())) {
+            // rows too long for the query block of any scan: the exact path,
+            // which has no limit on them (their copy may have a scan, so that
+            // a refusal would depend on the calls before)
+            uint32_t qflags = 0;
+            VS_HIP(hipMemcpyAsync(&qflags, ctl + 3, 4, hipMemcpyDeviceToHost, x->st), "query flags");
+            VS_HIP(hipStreamSynchronize(x->st), "query flags");
+            if (qflags & vs::kFlagNonFinite)
+                return set_err(VS_ERR_NONFINITE, "queries contain NaN or infinity");
             if ((rc = exact_search(x, A, pq.qf, nq, k, D, I))) return rc;
             VS_HIP(hipStreamSynchronize(x->st), "search");
             return VS_OK;
@@ -1648,7 +1674,7 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
         } else if (coarse && kk <= 256 && !coarse_wide) {
             // thresholds tighten to the kk-th value: ask for more candidates
             coarse_wide = true;
-            kk = std::max<int64_t>(nq <= 64 ? 64 : 32, 2 * kk);
+            kk = coarse_keep(nq, kk);
             --attempt;
             continue;
         }
@@ -1801,9 +1827,13 @@ int range_core(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int6
     // multiplies the bf16 copy of the rows (with the fp32 rows' norms), or,
     // without one, rounds them in the GEMM-tiled scan where that applies.
     CopyHold hold(x);
-    const bool copy = x->storage == 0 && x->opt.coarse && x->opt.copy16 && hold.mine &&
-                      ensure_copy16(x, nq);
-    if (copy) select_copy(x);
+    bool copy = x->storage == 0 && x->opt.coarse && x->opt.copy16 && hold.mine &&
+                ensure_copy16(x, nq, !has_plan(x, nq, 2, 8, true));
+    if (copy) {
+        select_copy(x);
+        copy = has_plan(x, nq, 1, 8, true);  // (its rows may be padded further)
+        if (!copy) select_rows(x);
+    }
     Arena A;
     vs::PreparedQueries pq;
     uint32_t qflags = 0;

@@ -1,6 +1,7 @@
-"""Rows long enough that a scan's query block only just fits the LDS: range
-search takes every dimension up to the block's own size, and a query that has
-to be searched again is."""
+"""Rows long enough that a scan's query block only just fits the LDS, or no
+longer does: range search takes every dimension up to the block's own size, a
+query that has to be searched again is, and a call gives the same answer
+whether it is the first on its rows or a later one (on their copy)."""
 import numpy as np
 import pytest
 
@@ -114,3 +115,48 @@ def test_query_past_bf16_on_the_copy(vs):
         r = idx.search(xq, 10)
         assert_knn_parity(r.distances, r.ids, Dr, Ir, 1, rtol=0.0, atol=0.0)
     idx.close()
+
+
+# fp32 rows whose own scan does not fit (one exists on the copy up to 4,736
+# elements, none at 6,000): the first call, a later one, and with the copy off
+@pytest.mark.parametrize("d,nq,k", [(3072, 8, 10), (3000, 70, 25), (4990, 5, 3), (6000, 4, 10),
+                                    (3072, 3, 300)])
+def test_first_and_later_calls_agree(vs, d, nq, k):
+    xb, xq = syn.normal_unit(1500, d, d, 0), syn.normal_unit(nq, d, d, 1)
+    for copy16 in (1, 0):
+        for metric in (0, 1):
+            idx = _index(vs, xb, metric, "f32", copy16=copy16)
+            got = [idx.search(xq, k) for _ in range(3)]
+            idx.close()
+            Dr, Ir = oracle.flat_search(xb, xq, k, metric, NT)
+            for r in got:
+                assert_knn_parity(r.distances, r.ids, Dr, Ir, metric, rtol=0.0, atol=0.0)
+
+
+@pytest.mark.parametrize("d", [2600, 3072])
+def test_first_range_search(vs, d):
+    xb, xq = syn.normal_unit(1500, d, d, 0), syn.normal_unit(6, d, d, 1)
+    xb[:30] = np.repeat(xq, 5, axis=0) + 0.005 * xb[:30]
+    idx = _index(vs, xb, 0, "f32")
+    got = [idx.range_search(xq, 0.5) for _ in range(2)]
+    idx.close()
+    lims, D, I = oracle.flat_range_search(xb, xq, 0.5, 0, NT)
+    for rr in got:
+        assert_range_parity(rr.limits, rr.distances, rr.ids, lims, D, I)
+
+
+def test_long_rows_report_nonfinite_queries(vs):
+    xb, xq = syn.normal_unit(700, 6000, 1, 0), syn.normal_unit(3, 6000, 1, 1)
+    for storage, bits in (("f32", False), ("bf16", False), ("bf16", True)):
+        idx = _index(vs, xb, 0, storage)
+        bad = xq.copy()
+        bad[1, 5] = np.nan
+        with pytest.raises(vs.VsError) as e:
+            idx.search(syn.to_bf16_bits(bad) if bits else bad, 4)
+        assert e.value.code == vs._native.VS_ERR_NONFINITE
+        rows = xb if storage == "f32" else _bf16(xb)
+        q = _bf16(xq) if bits else xq
+        r = idx.search(syn.to_bf16_bits(xq) if bits else xq, 4)
+        idx.close()
+        Dr, Ir = oracle.flat_search(rows, q, 4, 0, NT)
+        assert_knn_parity(r.distances, r.ids, Dr, Ir, 0, rtol=0.0, atol=0.0)
