@@ -264,6 +264,7 @@ struct vs_index {
     int64_t copy_ld = 0, copy_n = 0, copy_cap = 0;
     float copy_res = 0.f;  // largest |row - copied row| (an upper bound)
     uint64_t copy_asked = ~0ull;  // version of the rows at a call that went without the copy
+    uint64_t copy_denied = ~0ull; // version of the rows at a call whose scratch needed its room
     std::atomic_flag copy_busy = ATOMIC_FLAG_INIT;  // held by a call that reads the copy
     // the rows that the current call's scans and planning read
     struct {
@@ -858,9 +859,7 @@ struct Arena {
     Arena() = default;
     Arena(const Arena &) = delete;
     Arena &operator=(const Arena &) = delete;
-    ~Arena() {
-        for (auto &b : local) b.release();
-    }
+    ~Arena() { release_local(); }
     bool fixed() const { return base != nullptr; }
     int carve(size_t bytes, void **p, const char *what) {
         const size_t off = (used + 255) & ~(size_t)255;
@@ -886,6 +885,10 @@ struct Arena {
         VS_HIP(local.back().ensure(bytes), what);
         *p = local.back().p;
         return VS_OK;
+    }
+    void release_local() {
+        for (auto &b : local) b.release();
+        local.clear();
     }
     size_t mark() const { return used; }
     void reset(size_t m) { used = m; }
@@ -1185,7 +1188,7 @@ int xnorm_max(vs_index *x, Arena &A, float *out) {
 // so only if it is not the first on these rows, or if it needs the copy (has no
 // scan of the rows themselves).
 bool ensure_copy16(vs_index *x, int64_t nq, bool needed = false) {
-    if (x->storage != 0 || x->ntotal == 0) return false;
+    if (x->storage != 0 || x->ntotal == 0 || x->copy_denied == x->version) return false;
     const int64_t ld16 = vs::storage_ld(x->d, 1);
     if (x->copy_n == x->ntotal && x->copy_cap >= x->ntotal) return std::isfinite(x->copy_res);
     const int64_t pending = x->copy_cap < x->ntotal ? x->ntotal : x->ntotal - x->copy_n;
@@ -1236,6 +1239,20 @@ bool ensure_copy16(vs_index *x, int64_t nq, bool needed = false) {
     x->copy_res = std::max(x->copy_res, res);
     x->copy_n = x->ntotal;
     return std::isfinite(x->copy_res);
+}
+
+// A call ran out of memory while it held its own rows' copy, which no
+// allocation takes from it: frees the copy, for as long as the rows stay as
+// they are.  The call then starts over without it.
+void give_up_copy(vs_index *x) {
+    (void)hipStreamSynchronize(x->st);
+    CopyHold hold(x);
+    if (hold.mine) {
+        std::lock_guard<std::mutex> lk(g_copies_mu);
+        drop_copy(x);
+    }
+    x->copy_denied = x->version;
+    x->prof["copy_given_up"].launches++;
 }
 
 // The scans of this call read the stored rows.
@@ -1578,13 +1595,15 @@ int bounded_research(vs_index *x, Arena &A, const vs::PreparedQueries &pq, int p
     return ok ? scatter() : exact();
 }
 
+int select_search(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t nq, int64_t k,
+                  float *D, int32_t *I, bool safe, size_t list_budget, bool with_copy, bool *copied);
+
 // Top-k search of nq device query rows into device D / I [nq][k].  safe:
 // full-length lists and no threshold estimates (the re-search of queries
 // the merge could not prove exact), on every plane of fp32 rows.  list_budget > 0 bounds the bytes of
 // the candidate lists (the streaming scan's split count adapts).
 int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t nq, int64_t k,
                   float *D, int32_t *I, bool safe, size_t list_budget) {
-    int rc0 = VS_OK;
     if (nq < 0 || k < 0) return set_err(VS_ERR_INVALID, "nq and k must be >= 0");
     if (nq == 0) return VS_OK;
     if (k == 0) {
@@ -1604,7 +1623,7 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
         VS_HIP(x->hio.ensure(kCtlBytes), "control words");
         uint32_t *hf = x->hio.as<uint32_t>();
         *hf = 0;
-        if ((rc0 = exact_topk(x, A, q_dev, q_dtype, x->d, nq, k, D, I, hf))) return rc0;
+        if (int rc = exact_topk(x, A, q_dev, q_dtype, x->d, nq, k, D, I, hf)) return rc;
         // counted with the queries that the selection sent to the exact path
         x->prof["exact_fallback"].launches += nq;
         x->prof["direct"].launches++;
@@ -1613,10 +1632,26 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
             return set_err(VS_ERR_NONFINITE, "queries contain NaN or infinity");
         return VS_OK;
     }
+    bool copied = false;
+    int rc = select_search(x, A, q_dev, q_dtype, nq, k, D, I, safe, list_budget, true, &copied);
+    if (rc == VS_ERR_OOM && copied) {
+        give_up_copy(x);
+        A.release_local();
+        rc = select_search(x, A, q_dev, q_dtype, nq, k, D, I, safe, list_budget, false, &copied);
+    }
+    return rc;
+}
+
+// The selecting search: a scan's candidates, merged and proven.  with_copy:
+// on the copy of fp32 rows where that pays (*copied is set then).
+int select_search(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t nq, int64_t k,
+                  float *D, int32_t *I, bool safe, size_t list_budget, bool with_copy, bool *copied) {
     int64_t kk = std::max<int64_t>(8, next_pow2(k + std::max<int64_t>(4, k / 4)));
     select_rows(x);
     CopyHold hold(x);
-    bool coarse = !safe && !A.fixed() && hold.mine && coarse_search(x, k) && ensure_copy16(x, nq);
+    bool coarse = with_copy && !safe && !A.fixed() && hold.mine && coarse_search(x, k) &&
+                  ensure_copy16(x, nq);
+    *copied = coarse;
     if (coarse) {
         select_copy(x);
         // (the copy's rows may be padded further than the rows are)
@@ -1795,14 +1830,19 @@ struct RangeHits {
     RangeHits() = default;
     RangeHits(const RangeHits &) = delete;
     RangeHits &operator=(const RangeHits &) = delete;
-    ~RangeHits() {
+    ~RangeHits() { clear(); }
+    void clear() {
         free(q);
         free(id);
         free(s);
         free(lims);
+        q = id = nullptr;
+        s = nullptr;
+        lims = nullptr;
     }
     // (no array is null, as the callers' results have none)
     int alloc(int64_t hits, int64_t nlims, bool queries) {
+        clear();
         n = hits;
         const size_t m = (size_t)std::max<int64_t>(hits, 1);
         id = (int32_t *)malloc(m * 4);
@@ -1816,9 +1856,9 @@ struct RangeHits {
 };
 
 // Candidate scan + exact re-test of nq query rows (device, `stride` elements
-// apart).
-int range_core(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int64_t nq,
-               double radius, int self_join, RangeHits *out) {
+// apart).  with_copy and *copied as for select_search.
+int range_pass(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int64_t nq,
+               double radius, int self_join, bool with_copy, bool *copied, RangeHits *out) {
     const int64_t nlims = self_join ? 0 : nq + 1;
     if (nq == 0 || x->ntotal == 0) return out->alloc(0, nlims, self_join != 0);
     select_rows(x);
@@ -1827,8 +1867,9 @@ int range_core(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int6
     // multiplies the bf16 copy of the rows (with the fp32 rows' norms), or,
     // without one, rounds them in the GEMM-tiled scan where that applies.
     CopyHold hold(x);
-    bool copy = x->storage == 0 && x->opt.coarse && x->opt.copy16 && hold.mine &&
+    bool copy = with_copy && x->storage == 0 && x->opt.coarse && x->opt.copy16 && hold.mine &&
                 ensure_copy16(x, nq, !has_plan(x, nq, 2, 8, true));
+    *copied = copy;
     if (copy) {
         select_copy(x);
         copy = has_plan(x, nq, 1, 8, true);  // (its rows may be padded further)
@@ -1939,6 +1980,19 @@ int range_core(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int6
         VS_HIP(hipStreamSynchronize(x->st), "range results");
     }
     return VS_OK;
+}
+
+int range_core(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int64_t nq,
+               double radius, int self_join, RangeHits *out) {
+    bool copied = false;
+    int rc = range_pass(x, q_dev, q_dtype, stride, nq, radius, self_join, true, &copied, out);
+    if (rc == VS_ERR_OOM && copied) {
+        give_up_copy(x);
+        rc = range_pass(x, q_dev, q_dtype, stride, nq, radius, self_join, false, &copied, out);
+        if (rc == VS_ERR_UNSUPPORTED)  // (rows so long that only their copy has a scan)
+            rc = set_err(VS_ERR_OOM, "range search: out of device memory beside the row copy");
+    }
+    return rc;
 }
 
 }  // namespace

@@ -151,3 +151,47 @@ def test_add_is_all_or_nothing(vs, storage):
         assert idx.storage == "f32"
         assert_knn_parity(r.distances, r.ids, Dr, Ir, 0, rtol=0.0, atol=0.0, xb=rows, xq=xq)
     idx.close()
+
+
+def _copied(vs, xb, xq, k):
+    """An index of fp32 rows that holds their copy (built by its second search)."""
+    idx = vs.GpuIndexFlat.l2(xb.shape[1], storage="f32")
+    idx.set_option("direct", 0)
+    idx.add(xb)
+    for _ in range(2):
+        idx.search(xq, k)
+    return idx
+
+
+def test_search_gives_up_its_own_copy(vs):
+    """Scratch that does not fit beside the search's own row copy: the copy
+    goes, and the call succeeds without it."""
+    from vector_store import _native as NN
+
+    xb, xq = syn.normal_unit(20_000, 96, 3, 0), syn.normal_unit(200, 96, 3, 1)
+    Dr, Ir = oracle.flat_search(xb, xq, 10, 0, NT)
+    lims, Dx, Ix = oracle.flat_range_search(xb, xq, 1.6, 0, NT)
+    qb, Db, Ib = NN.DeviceBuffer(xq.nbytes), NN.DeviceBuffer(200 * 40), NN.DeviceBuffer(200 * 40)
+    qb.upload(xq)
+    D, I = np.empty((200, 10), np.float32), np.empty((200, 10), np.int32)
+    for n in (1, 2, 3):
+        idx = _copied(vs, xb, xq[:5], 10)
+        idx.set_option("fail_alloc", n)
+        idx.search_device(qb, 200, 10, Db, Ib)
+        idx.set_option("fail_alloc", 0)
+        assert idx.prof_get("copy_given_up")[0] == 1
+        Db.download(D)
+        Ib.download(I)
+        assert_knn_parity(D, I, Dr, Ir, 0, rtol=0.0, atol=0.0)
+        r = idx.search(xq, 10)
+        assert_knn_parity(r.distances, r.ids, Dr, Ir, 0, rtol=0.0, atol=0.0)
+        idx.close()
+    idx = _copied(vs, xb, xq[:5], 10)
+    idx.set_option("fail_alloc", 2)  # (the first is the query staging, before the rows are chosen)
+    rr = idx.range_search(xq, 1.6)
+    idx.set_option("fail_alloc", 0)
+    assert idx.prof_get("copy_given_up")[0] == 1
+    idx.close()
+    for b in (qb, Db, Ib):
+        b.free()
+    assert_range_parity(rr.limits, rr.distances, rr.ids, lims, Dx, Ix)
