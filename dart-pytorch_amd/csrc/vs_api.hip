@@ -1623,14 +1623,19 @@ int search_device(vs_index *x, Arena &A, const void *q_dev, int q_dtype, int64_t
         VS_HIP(x->hio.ensure(kCtlBytes), "control words");
         uint32_t *hf = x->hio.as<uint32_t>();
         *hf = 0;
-        if (int rc = exact_topk(x, A, q_dev, q_dtype, x->d, nq, k, D, I, hf)) return rc;
-        // counted with the queries that the selection sent to the exact path
-        x->prof["exact_fallback"].launches += nq;
-        x->prof["direct"].launches++;
-        VS_HIP(hipStreamSynchronize(x->st), "search");
-        if (*(volatile uint32_t *)hf & vs::kFlagNonFinite)
-            return set_err(VS_ERR_NONFINITE, "queries contain NaN or infinity");
-        return VS_OK;
+        const int rc = exact_topk(x, A, q_dev, q_dtype, x->d, nq, k, D, I, hf);
+        if (rc == VS_OK) {
+            // counted with the queries that the selection sent to the exact path
+            x->prof["exact_fallback"].launches += nq;
+            x->prof["direct"].launches++;
+            VS_HIP(hipStreamSynchronize(x->st), "search");
+            if (*(volatile uint32_t *)hf & vs::kFlagNonFinite)
+                return set_err(VS_ERR_NONFINITE, "queries contain NaN or infinity");
+            return VS_OK;
+        }
+        // (no room for the keys, up to 256 MiB: the selection takes less)
+        if (rc != VS_ERR_OOM) return rc;
+        A.release_local();
     }
     bool copied = false;
     int rc = select_search(x, A, q_dev, q_dtype, nq, k, D, I, safe, list_budget, true, &copied);

@@ -195,3 +195,37 @@ def test_search_gives_up_its_own_copy(vs):
     for b in (qb, Db, Ib):
         b.free()
     assert_range_parity(rr.limits, rr.distances, rr.ids, lims, Dx, Ix)
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+def test_no_room_for_the_key_matrix(vs, storage):
+    """A small search whose exact keys (its second and third allocation) do not
+    fit takes the selection, which then reads host queries from pinned memory."""
+    from vector_store import _native as NN
+
+    xb, xq = syn.int_grid(5000, 64, 3, 0), syn.int_grid(6, 64, 3, 1)
+    Dr, Ir = oracle.flat_search(xb, xq, 10, 0, NT)
+    qb, Db, Ib = NN.DeviceBuffer(xq.nbytes), NN.DeviceBuffer(240), NN.DeviceBuffer(240)
+    qb.upload(xq)
+    D, I = np.empty((6, 10), np.float32), np.empty((6, 10), np.int32)
+    for n in (2, 3):
+        idx = vs.GpuIndexFlat.l2(64, storage=storage)
+        idx.add(xb)
+        idx.set_option("fail_alloc", n)  # (the first is the pinned control block)
+        idx.search_device(qb, 6, 10, Db, Ib)
+        assert idx.prof_get("direct")[0] == 0
+        Db.download(D)
+        Ib.download(I)
+        assert_knn_parity(D, I, Dr, Ir, 0, rtol=0.0, atol=0.0, xb=xb, xq=xq)
+        idx.search_device(qb, 6, 10, Db, Ib)
+        assert idx.prof_get("direct")[0] == 1
+        idx.close()
+        idx = vs.GpuIndexFlat.l2(64, storage=storage)
+        idx.add(xb)
+        idx.set_option("fail_alloc", n)
+        r = idx.search(xq, 10)
+        idx.set_option("fail_alloc", 0)
+        idx.close()
+        assert_knn_parity(r.distances, r.ids, Dr, Ir, 0, rtol=0.0, atol=0.0, xb=xb, xq=xq)
+    for b in (qb, Db, Ib):
+        b.free()
