@@ -64,22 +64,31 @@ struct DeviceGuard {
 // failure paths of every caller (and show that a path allocates nothing).
 // Per thread, like the error text.
 thread_local int64_t g_fail_alloc = 0;
+// Option "full_alloc": when > 0, the device allocation that brings it to 0
+// finds the device full at its first try.
+thread_local int64_t g_full_alloc = 0;
 
 bool release_idle_copies();  // below: frees row copies on the current device
 
-// Every device allocation of an index goes through here.  A full device
-// takes the row copies of indexes that no call is using back first.
-hipError_t dev_malloc(void **p, size_t bytes) {
-    if (g_fail_alloc > 0 && --g_fail_alloc == 0) {
-        *p = nullptr;
-        return hipErrorOutOfMemory;
-    }
-    hipError_t e = hipMalloc(p, bytes);
+// A full device takes the row copies of indexes that no call is using back
+// first.
+hipError_t malloc_evicting(void **p, size_t bytes, bool full = false) {
+    *p = nullptr;
+    hipError_t e = full ? hipErrorOutOfMemory : hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory && release_idle_copies()) {
         (void)hipGetLastError();
         e = hipMalloc(p, bytes);
     }
     return e;
+}
+
+// Every device allocation of an index goes through here.
+hipError_t dev_malloc(void **p, size_t bytes) {
+    if (g_fail_alloc > 0 && --g_fail_alloc == 0) {
+        *p = nullptr;
+        return hipErrorOutOfMemory;
+    }
+    return malloc_evicting(p, bytes, g_full_alloc > 0 && --g_full_alloc == 0);
 }
 
 // Every pinned host allocation of an index goes through here.
@@ -266,6 +275,7 @@ struct vs_index {
     uint64_t copy_asked = ~0ull;  // version of the rows at a call that went without the copy
     uint64_t copy_denied = ~0ull; // version of the rows at a call whose scratch needed its room
     std::atomic_flag copy_busy = ATOMIC_FLAG_INIT;  // held by a call that reads the copy
+    std::atomic<int64_t> copies_taken{0};  // times an allocation took the copy
     // the rows that the current call's scans and planning read
     struct {
         const void *rows = nullptr;
@@ -287,9 +297,10 @@ struct vs_index {
 
 namespace {
 
-// Indexes that hold a row copy.  A copy belongs to its handle's thread while
-// copy_busy is set (every call that reads it holds it until its GPU work is
-// done); otherwise any thread short of memory may free it under this lock.
+// Indexes that hold a row copy.  A copy and its state (xb16, copy_n, copy_cap)
+// belong to their handle's thread while copy_busy is set (every call that
+// reads the copy holds it until its GPU work is done); otherwise they change
+// under this lock alone, where any thread short of memory may free the copy.
 std::mutex g_copies_mu;
 std::vector<vs_index *> g_copies;
 
@@ -299,15 +310,25 @@ void drop_copy(vs_index *x) {  // the caller holds g_copies_mu
     g_copies.erase(std::remove(g_copies.begin(), g_copies.end(), x), g_copies.end());
 }
 
+// The copied rows are no longer those of the index.
+void forget_copied_rows(vs_index *x) {
+    std::lock_guard<std::mutex> lk(g_copies_mu);
+    x->copy_n = 0;
+}
+
 bool release_idle_copies() {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) return false;
     std::lock_guard<std::mutex> lk(g_copies_mu);
     bool any = false;
-    const std::vector<vs_index *> all = g_copies;
-    for (vs_index *y : all) {
-        if (y->device != dev || y->copy_busy.test_and_set(std::memory_order_acquire)) continue;
+    for (size_t i = 0; i < g_copies.size();) {
+        vs_index *y = g_copies[i];
+        if (y->device != dev || y->copy_busy.test_and_set(std::memory_order_acquire)) {
+            ++i;
+            continue;
+        }
         drop_copy(y);
+        ++y->copies_taken;
         y->copy_busy.clear(std::memory_order_release);
         any = true;
     }
@@ -454,7 +475,7 @@ int widen_storage(vs_index *x) {
     x->cap = nc;
     x->ld = new_ld;
     x->storage = 0;
-    x->copy_n = 0;
+    forget_copied_rows(x);
     ++x->version;
     return VS_OK;
 }
@@ -1221,8 +1242,12 @@ bool ensure_copy16(vs_index *x, int64_t nq, bool needed = false) {
         x->xb16.bytes = bytes;
         x->copy_ld = ld16;
         x->copy_cap = x->cap;
-        std::lock_guard<std::mutex> lk(g_copies_mu);
-        g_copies.push_back(x);
+        try {
+            std::lock_guard<std::mutex> lk(g_copies_mu);
+            g_copies.push_back(x);
+        } catch (const std::bad_alloc &) {
+            return fail();
+        }
     }
     float *res_dev = (float *)(x->xb16.as<char>() + x->xb16.bytes);
     if (x->copy_n == 0) x->copy_res = 0.f;
@@ -2173,7 +2198,7 @@ int vs_index_reset(vs_index *x) {
         VS_HIP(hipStreamSynchronize(x->st), "reset");
     }
     x->ntotal = 0;
-    x->copy_n = 0;
+    forget_copied_rows(x);
     ++x->version;
     return VS_OK;
 }
@@ -2298,7 +2323,7 @@ int vs_index_remove_ids(vs_index *x, const int64_t *ids, int64_t n, int64_t *nre
     x->xb = nxb;
     x->xn = nxn;
     x->ntotal = w;
-    x->copy_n = 0;
+    forget_copied_rows(x);
     ++x->version;
     if (nremoved) *nremoved = removed;
     return VS_OK;
@@ -3338,7 +3363,7 @@ int vs_dev_alloc(int device, int64_t bytes, void **out) {
     if (!out || bytes < 0) return set_err(VS_ERR_INVALID, "bad arguments");
     DeviceGuard g(device);
     if (g.err != hipSuccess) return hip_err(g.err, "hipSetDevice");
-    VS_HIP(hipMalloc(out, (size_t)std::max<int64_t>(bytes, 1)), "hipMalloc");
+    VS_HIP(malloc_evicting(out, (size_t)std::max<int64_t>(bytes, 1)), "hipMalloc");
     return VS_OK;
 }
 
@@ -3468,6 +3493,11 @@ int vs_prof_get(vs_index *x, const char *family, int64_t *launches, double *tota
     if (!family) return set_err(VS_ERR_INVALID, "null family");
     DeviceGuard g(x->device);
     prof_collect(x);
+    if (strcmp(family, "copy_taken") == 0) {  // (counted by other threads)
+        if (launches) *launches = x->copies_taken;
+        if (total_ms) *total_ms = 0.0;
+        return VS_OK;
+    }
     auto it = x->prof.find(family);
     if (launches) *launches = it == x->prof.end() ? 0 : it->second.launches;
     if (total_ms) *total_ms = it == x->prof.end() ? 0.0 : it->second.total_ms;
@@ -3526,6 +3556,11 @@ int vs_index_set_option(vs_index *x, const char *name, int64_t value) {
     if (strcmp(name, "fail_alloc") == 0) {  // not a planner option: this thread's countdown
         if (value < 0) return set_err(VS_ERR_INVALID, "option fail_alloc: value %lld < 0", (long long)value);
         g_fail_alloc = value;
+        return VS_OK;
+    }
+    if (strcmp(name, "full_alloc") == 0) {  // nor is this
+        if (value < 0) return set_err(VS_ERR_INVALID, "option full_alloc: value %lld < 0", (long long)value);
+        g_full_alloc = value;
         return VS_OK;
     }
     for (const Opt &o : opts) {

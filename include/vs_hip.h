@@ -292,6 +292,9 @@ VS_API int vs_index_sync(vs_index *idx);
  *                 batch size)
  *   "fail_alloc"  n > 0: the n-th device allocation of any index from now on, on
  *                 this thread, fails as VS_ERR_OOM (failure-path tests; 0 clears it)
+ *   "full_alloc"  n > 0: that allocation finds the device full instead, and succeeds if it
+ *                 can take another index's idle row copy (families "copy_taken" and
+ *                 "copy_given_up" of vs_prof_get count what became of an index's own)
  * Unknown names and out-of-range values: VS_ERR_INVALID. */
 VS_API int vs_index_set_option(vs_index *idx, const char *name, int64_t value);
 

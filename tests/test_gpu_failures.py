@@ -229,3 +229,76 @@ def test_no_room_for_the_key_matrix(vs, storage):
         assert_knn_parity(r.distances, r.ids, Dr, Ir, 0, rtol=0.0, atol=0.0, xb=xb, xq=xq)
     for b in (qb, Db, Ib):
         b.free()
+
+
+def test_idle_copies_are_given_back(vs):
+    """An allocation that finds the device full takes the row copies of other
+    indexes and succeeds; their next searches are exact, and copy again."""
+    xb, xq = syn.normal_unit(20_000, 96, 3, 0), syn.normal_unit(20, 96, 3, 1)
+    Dr, Ir = oracle.flat_search(xb, xq, 10, 0, NT)
+    a, c = _copied(vs, xb, xq, 10), _copied(vs, xb, xq, 10)
+    b = vs.GpuIndexFlat.l2(96, storage="f32")
+    b.set_option("full_alloc", 1)
+    b.add(xb[:100])  # (its storage is the first allocation)
+    b.set_option("full_alloc", 0)
+    assert a.prof_get("copy_taken")[0] == 1 and c.prof_get("copy_taken")[0] == 1
+    for idx in (a, c):
+        for _ in range(3):
+            r = idx.search(xq, 10)
+            assert_knn_parity(r.distances, r.ids, Dr, Ir, 0, rtol=0.0, atol=0.0)
+    b.set_option("full_alloc", 1)
+    b.reserve(5000)
+    b.set_option("full_alloc", 0)
+    assert a.prof_get("copy_taken")[0] == 2  # (it had copied again)
+    a.close()
+    c.close()
+    b.set_option("full_alloc", 1)  # no copy left to take
+    _oom(vs, lambda: b.reserve(50_000))
+    b.set_option("full_alloc", 0)
+    b.close()
+
+
+def test_copies_taken_by_another_thread(vs):
+    """One thread searches on row copies, changes its rows and searches again
+    while another allocates on a full device: every result is exact, whether
+    the copy was idle (taken) or in use (left alone)."""
+    import threading
+
+    xb, xq = syn.normal_unit(30_000, 96, 3, 0), syn.normal_unit(40, 96, 3, 1)
+    Dr, Ir = oracle.flat_search(xb, xq, 10, 0, NT)
+    Dh, Ih = oracle.flat_search(xb[:20_000], xq, 10, 0, NT)
+    errors, done = [], threading.Event()
+
+    def searches():
+        try:
+            idx = vs.GpuIndexFlat.l2(96, storage="f32")
+            idx.set_option("direct", 0)
+            for _ in range(6):
+                idx.reset()
+                for rows, D, I in ((xb[:20_000], Dh, Ih), (xb[20_000:], Dr, Ir)):
+                    idx.add(rows)
+                    for _ in range(4):
+                        r = idx.search(xq, 10)
+                        assert_knn_parity(r.distances, r.ids, D, I, 0, rtol=0.0, atol=0.0)
+            idx.close()
+        except BaseException as e:  # noqa: BLE001 - reported by the main thread
+            errors.append(e)
+        finally:
+            done.set()
+
+    t = threading.Thread(target=searches)
+    t.start()
+    turns = 0
+    while not done.wait(0.002) and turns < 2000:
+        turns += 1
+        b = vs.GpuIndexFlat.l2(96, storage="f32")
+        b.set_option("full_alloc", 1)
+        try:
+            b.reserve(1000)
+        except vs.VsError as e:  # no idle copy at that moment
+            assert e.code == vs._native.VS_ERR_OOM
+        b.set_option("full_alloc", 0)
+        b.close()
+    t.join()
+    assert not errors, errors
+    assert turns > 0
