@@ -2366,7 +2366,7 @@ __global__ __launch_bounds__(512) void kmeans_update_kernel(const float *__restr
     __shared__ __align__(16) float sh[B][DC];
     const int64_t c = blockIdx.x, j0 = (int64_t)blockIdx.y * DC;
     const int cnt = counts[c];
-    if (cnt < min_points || cnt <= 0) return;
+    if (cnt < min_points) return;  // (min_points <= 0: an empty cluster is 0 times 1 / 0)
     const int32_t *ord = order + offsets[c];
     const int tid = threadIdx.x, pr = tid / TPR, pc = (tid % TPR) * 4;
     int row[NP];

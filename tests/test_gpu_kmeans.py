@@ -242,3 +242,19 @@ def test_assign_any_dimension(vs, n, d, K, kind):
         assert np.array_equal(a, ar) and obj == objr
         cen = newc
     pts.close()
+
+
+@pytest.mark.parametrize("min_points", [0, -3])
+def test_empty_clusters_without_a_minimum(vs, min_points):
+    """With min_points <= 0 an empty cluster's centroid is its sum scaled by
+    1 / 0, as kmeans.dart:110-114 computes it: not a number."""
+    x = syn.normal_unit(900, 64, 1, 0)
+    cen = np.concatenate([x[:5], np.full((2, 64), 30.0, np.float32)])
+    pts = vs.GpuIndexFlat.l2(64, storage="f32")
+    pts.add(x)
+    a, newc, cnt, obj = vs.kmeans_step(pts, cen, min_points)
+    pts.close()
+    ar, _, objr = oracle.kmeans_assign(x, cen, oracle.default_threads())
+    cr, cntr, _ = oracle.kmeans_update(x, ar, cen, min_points)
+    assert np.array_equal(a, ar) and obj == objr and np.array_equal(cnt, cntr)
+    assert np.all(np.isnan(cr[5:])) and np.array_equal(newc, cr, equal_nan=True)
