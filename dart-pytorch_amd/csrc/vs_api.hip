@@ -446,8 +446,28 @@ int ensure_capacity(vs_index *x, int64_t need) {
     return VS_OK;
 }
 
+// The bf16 rows that widen_storage replaced, until its add has succeeded.
+struct NarrowRows {
+    void *xb = nullptr;
+    float *xn = nullptr;
+    int64_t cap = 0, ld = 0;
+    ~NarrowRows() {
+        if (xb) (void)hipFree(xb);
+        if (xn) (void)hipFree(xn);
+    }
+    // the index holds them again (an add that failed after it widened them)
+    void restore(vs_index *x) {
+        std::swap(xb, x->xb);
+        std::swap(xn, x->xn);
+        x->cap = cap;
+        x->ld = ld;
+        x->storage = 1;
+        ++x->version;
+    }
+};
+
 // Switch bf16 storage to fp32 (AUTO storage meeting a non-bf16 value).
-int widen_storage(vs_index *x) {
+int widen_storage(vs_index *x, NarrowRows *old) {
     const int64_t new_ld = vs::storage_ld(x->d, 0);
     const int64_t nc = std::max<int64_t>(x->cap, 1024);
     void *nxb = nullptr;
@@ -468,8 +488,10 @@ int widen_storage(vs_index *x) {
                                      x->flags.as<uint32_t>(), x->st),
                "widening storage");
     VS_HIP(hipStreamSynchronize(x->st), "widening storage");
-    if (x->xb) (void)hipFree(x->xb);
-    if (x->xn) (void)hipFree(x->xn);
+    old->xb = x->xb;
+    old->xn = x->xn;
+    old->cap = x->cap;
+    old->ld = x->ld;
     x->xb = nxb;
     x->xn = nxn;
     x->cap = nc;
@@ -514,6 +536,8 @@ int clear_rows(vs_index *x, int64_t end) {
 template <typename Fetch>
 int add_rows(vs_index *x, int dtype, int64_t n, int64_t chunk, Fetch &&fetch) {
     if (int rc = ensure_capacity(x, x->ntotal + n)) return rc;
+    NarrowRows narrow;
+    bool widened = false;
     for (int64_t r = 0; r < n;) {
         const int64_t m = std::min(chunk, n - r);
         const void *src = nullptr;
@@ -523,14 +547,16 @@ int add_rows(vs_index *x, int dtype, int64_t n, int64_t chunk, Fetch &&fetch) {
         if (!rc && (f & vs::kFlagNonFinite))
             rc = set_err(VS_ERR_NONFINITE, "vectors contain NaN or infinity");
         if (rc) {
-            (void)clear_rows(x, x->ntotal + r + m);
+            if (widened) narrow.restore(x);  // (its rows past ntotal are clear)
+            else (void)clear_rows(x, x->ntotal + r + m);
             return rc;
         }
         if (x->mode == VS_STORAGE_AUTO && x->storage == 1 && (f & vs::kFlagNotBf16)) {
             // fp32 from here on: the rows so far are stored again
             rc = clear_rows(x, x->ntotal + r + m);
-            if (!rc) rc = widen_storage(x);
+            if (!rc) rc = widen_storage(x, &narrow);
             if (rc) return rc;
+            widened = true;
             r = 0;
             continue;
         }

@@ -302,3 +302,29 @@ def test_copies_taken_by_another_thread(vs):
     t.join()
     assert not errors, errors
     assert turns > 0
+
+
+def test_failed_add_keeps_the_storage(vs):
+    """A host add of more than one upload chunk (256 MiB) whose first rows bf16
+    does not hold and whose last row is not finite: the storage stays bf16."""
+    d, n = 4096, 16_500
+    xb, xq = syn.int_grid(300, d, 3, 0), syn.int_grid(5, d, 3, 1)
+    idx = vs.GpuIndexFlat.l2(d)
+    idx.add(xb)
+    bad = np.zeros((n, d), np.float32)
+    bad[0, 0] = 0.3
+    bad[-1, -1] = np.inf
+    with pytest.raises(vs.VsError) as e:
+        idx.add(bad)
+    assert e.value.code == vs._native.VS_ERR_NONFINITE
+    assert idx.ntotal == 300 and idx.storage == "bf16"
+    idx.set_option("direct", 0)
+    r = idx.search(xq, 12)
+    Dr, Ir = oracle.flat_search(xb, xq, 12, 0, NT)
+    assert_knn_parity(r.distances, r.ids, Dr, Ir, 0, rtol=0.0, atol=0.0, xb=xb, xq=xq)
+    bad[-1, -1] = 1.0  # and one that widens it
+    idx.add(bad)
+    assert idx.storage == "f32" and idx.ntotal == 300 + n
+    assert np.array_equal(idx.reconstruct_n(299, 2), np.concatenate([xb[299:], bad[:1]]))
+    assert np.array_equal(idx.reconstruct(300 + n - 1), bad[-1])
+    idx.close()
