@@ -925,6 +925,10 @@ struct Arena {
         *p = b.p;
         return VS_OK;
     }
+    // the same, but a buffer of this call only past `most` bytes
+    int get_upto(DevBuf &b, size_t bytes, size_t most, void **p, const char *what) {
+        return bytes <= most ? get(b, bytes, p, what) : tmp(bytes, p, what);
+    }
     // a buffer of this call only
     int tmp(size_t bytes, void **p, const char *what) {
         if (base) return carve(bytes, p, what);
@@ -940,6 +944,10 @@ struct Arena {
     size_t mark() const { return used; }
     void reset(size_t m) { used = m; }
 };
+
+// Keys (8 bytes each; range hits take 16 with their sort) up to this size
+// stay with the index, larger ones go with their call.
+constexpr size_t kKeptKeyBytes = (size_t)1 << 28;
 
 #define VS_TAKE(arena_call)          \
     do {                             \
@@ -1384,8 +1392,7 @@ int exact_topk(vs_index *x, Arena &A, const void *q, int q_dtype, int64_t stride
     const size_t kbytes = (size_t)(select ? qc : qc + 1) * n * 8;
     void *p_qd, *p_keys, *p_part = nullptr, *p_rf = nullptr, *p_tmp = nullptr;
     VS_TAKE(A.get(x->ex_qd, (size_t)qc * ldd * 8, &p_qd, "query rows"));
-    if (kbytes <= (size_t)1 << 28) VS_TAKE(A.get(x->ex_keys, kbytes, &p_keys, "keys"));
-    else VS_TAKE(A.tmp(kbytes, &p_keys, "keys"));
+    VS_TAKE(A.get_upto(x->ex_keys, kbytes, kKeptKeyBytes, &p_keys, "keys"));
     if (nseg > 1) VS_TAKE(A.get(x->ex_part, (size_t)qc * nseg * k * 8, &p_part, "segment keys"));
     if (hflags) VS_TAKE(A.get(x->flags, (size_t)nq * 4, &p_rf, "query flags"));
     if (!select) VS_TAKE(A.tmp(tmp_bytes + 256, &p_tmp, "sort scratch"));
@@ -1622,8 +1629,7 @@ int bounded_research(vs_index *x, Arena &A, const vs::PreparedQueries &pq, int p
     if (ok) {
         void *keys;
         const size_t kb = (size_t)std::max<int64_t>(found, 1) * 8;
-        if (kb <= (size_t)1 << 28) VS_TAKE(A.get(x->ex_keys, kb, &keys, "re-search keys"));
-        else VS_TAKE(A.tmp(kb, &keys, "re-search keys"));
+        VS_TAKE(A.get_upto(x->ex_keys, kb, kKeptKeyBytes, &keys, "re-search keys"));
         VS_HIP(vs::launch_count_pairs((const int32_t *)cq, found, m, qcnt, x->st),
                "re-search counts");
         VS_HIP(vs::launch_exclusive_scan_i32(qcnt, m, qoff, x->st), "re-search offsets");
@@ -1993,12 +1999,14 @@ int range_pass(vs_index *x, const void *q_dev, int q_dtype, int64_t stride, int6
     size_t tmp_bytes = 0;
     VS_HIP(vs::sort_pairs_u64(nullptr, tmp_bytes, nullptr, nullptr, nullptr, nullptr, m, bits, x->st),
            "sort size");
-    VS_HIP(x->ex_keys.ensure((size_t)m * 16), "range keys");
-    VS_HIP(x->rs.ensure((size_t)m * 8), "range scores");
-    VS_HIP(x->rtmp.ensure(tmp_bytes + (size_t)nlims * 8 + 256), "range sort");
-    uint64_t *keys = x->ex_keys.as<uint64_t>(), *sorted = keys + m;
-    float *score = x->rs.as<float>(), *sscore = score + m;
-    int64_t *lims = x->rtmp.as<int64_t>();
+    void *p_keys, *p_score, *p_tmp;
+    VS_TAKE(A.get_upto(x->ex_keys, (size_t)m * 16, kKeptKeyBytes, &p_keys, "range keys"));
+    VS_TAKE(A.get_upto(x->rs, (size_t)m * 8, kKeptKeyBytes / 2, &p_score, "range scores"));
+    VS_TAKE(A.get_upto(x->rtmp, tmp_bytes + (size_t)nlims * 8 + 256, kKeptKeyBytes / 2, &p_tmp,
+                       "range sort"));
+    uint64_t *keys = (uint64_t *)p_keys, *sorted = keys + m;
+    float *score = (float *)p_score, *sscore = score + m;
+    int64_t *lims = (int64_t *)p_tmp;
     {
         ProfScope ps(x, "refine");
         VS_HIP(vs::launch_fill32(x->flags.p, 1, 0u, x->st), "clearing flags");
@@ -2665,8 +2673,7 @@ int vs_index_search_subsets(vs_index *x, const void *q, int q_dtype, int64_t nq,
         }
         void *keys;
         const size_t kb = (size_t)std::max<int64_t>(total, 1) * 8;
-        if (kb <= (size_t)1 << 28) VS_TAKE(A.get(x->ex_keys, kb, &keys, "keys"));
-        else VS_TAKE(A.tmp(kb, &keys, "keys"));
+        VS_TAKE(A.get_upto(x->ex_keys, kb, kKeptKeyBytes, &keys, "keys"));
         {
             ProfScope ps(x, "scan");
             VS_HIP(vs::launch_subset_keys(x->xb, x->storage, x->ld, x->d, x->metric, qd + q0 * ldd,

@@ -328,3 +328,25 @@ def test_failed_add_keeps_the_storage(vs):
     assert np.array_equal(idx.reconstruct_n(299, 2), np.concatenate([xb[299:], bad[:1]]))
     assert np.array_equal(idx.reconstruct(300 + n - 1), bad[-1])
     idx.close()
+
+
+def test_range_gives_its_sort_space_back(vs):
+    """2e7 hits take 880 MB while they are scored and sorted; the index keeps
+    the candidates' 160 MB."""
+    import ctypes
+
+    def free():
+        f, t = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert vs.load().hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    xb, xq = syn.normal_unit(5000, 8, 3, 0), syn.normal_unit(4000, 8, 3, 1)
+    idx = vs.GpuIndexFlat.l2(8, storage="f32")
+    idx.add(xb)
+    idx.range_search(xq[:10], 1e9)
+    before = free()
+    rr = idx.range_search(xq, 1e9)
+    kept = before - free()
+    idx.close()
+    assert rr.limits[-1] == 20_000_000
+    assert kept <= 400e6, f"{kept / 1e6:.0f} MB kept"
