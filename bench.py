@@ -1,16 +1,16 @@
 """Benchmark of the MI355X flat k-NN path (one JSON line on stdout).
 
-Default run (no flags): every BASELINE.json configuration, in one process.
-The headline line is configs[1] (C2): exact L2 top-100 over a 1,000,000 x 128
+Default run (no flags): every benchmark configuration, in one process.
+The headline line is C2: exact L2 top-100 over a 1,000,000 x 128
 database of integers 0..255 stored as fp32, 10,000 queries of the same
 distribution; one step = one search of the whole query batch with the
 database, the queries and the result buffers resident in HBM.  The other
 configurations sit under "workloads":
 
   c1  10k x 384 fp32 unit rows, IP, 100 queries, k = 10 (the CPU-runnable case);
-  c2f configs[1]'s shape on fp32 unit N(0,1) rows, which bf16 does not hold
-      exactly: the rows stay fp32 and every product takes three MFMA passes
-      over split-bf16 planes (the path of general fp32 embeddings);
+  c2f the C2 shape on fp32 unit N(0,1) rows, which bf16 does not hold
+      exactly: the rows stay fp32, candidates are selected on their bf16 copy
+      and scored exactly (the path of general fp32 embeddings);
   c3  20M x 768 bf16 unit rows (device-generated), IP, k = 10, batches
       1 / 64 / 1024 / 8192;
   c4  k-means step, 2M x 256 fp32 mixture points, K = 4096;
@@ -23,13 +23,13 @@ Every workload reports:
                         repeated timed passes, best and median);
   roofline              the dominant kernel timed with HIP events on the
                         index's stream over the timed region: algorithmic
-                        bytes (HBM-bound: batch <= 64) or flops (MFMA-bound)
-                        per launch over its mean duration, against the spec
+                        bytes (HBM-bound: batch <= 64) or flops (MFMA-bound, or
+                        fp64 vector sums: c1) per launch over its mean duration, against the spec
                         peak and against the measured peaks (vs_dev_probe);
   cpu_baseline          the CPU oracle (oracle/oracle.c, a restatement of
                         IndexFlat.search / rangeSearch / Kmeans, index_flat.dart,
                         kmeans.dart) timed on this host: all cores (threads
-                        over queries, at most the box's 16-core share) and one
+                        over queries, at most one GPU's 16-core share) and one
                         core (the reference's own parallelism: one Dart isolate);
   parity                GPU results against the oracle on the same inputs:
                         tie-aware top-k comparison (distances bit-identical,
@@ -61,8 +61,9 @@ for _p in (ROOT, os.path.join(ROOT, "dart-pytorch_amd")):
         sys.path.insert(0, _p)
 
 METRIC = "QPS, flat top-k k-NN (1M×128 fp32, 20M×768 bf16); % HBM / MFMA roofline"
-PEAK = {"bf16_mfma_tflops": 2500.0, "fp32_mfma_tflops": 157.3, "hbm_gbs": 8000.0}
-CPU_SHARE = 16  # host cores of one GPU's share on the measurement boxes
+PEAK = {"bf16_mfma_tflops": 2500.0, "fp32_mfma_tflops": 157.3, "hbm_gbs": 8000.0,
+        "fp64_tflops": 78.6}
+CPU_SHARE = 16  # host cores that go with one GPU
 
 # HBM bytes per launch of the dominant kernel, from two rocprofv3 --pmc runs
 # (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0: the factors a plain 16-byte copy of
@@ -155,10 +156,14 @@ def time_steps(fn, steps, warmup, label):
 
 def roofline(kind, work, avg_s, peaks, kernel, launches, traffic=None, traffic_src=None,
              peak_div=1, extra=None):
-    """kind 'hbm': work = algorithmic bytes per launch; 'mfma': flops per launch."""
+    """kind 'hbm': work = algorithmic bytes per launch; 'mfma': flops per launch, on the
+    bf16 matrix cores; 'fp64': flops per launch, on the vector units."""
     if kind == "hbm":
         ach = work / avg_s / 1e9
         peak, meas, unit = PEAK["hbm_gbs"], peaks.get("hbm_read_gbs"), "GB/s"
+    elif kind == "fp64":
+        ach = work / avg_s / 1e12
+        peak, meas, unit = PEAK["fp64_tflops"], None, "TFLOP/s"
     else:
         ach = work / avg_s / 1e12
         peak = PEAK["bf16_mfma_tflops"] / peak_div
@@ -170,7 +175,7 @@ def roofline(kind, work, avg_s, peaks, kernel, launches, traffic=None, traffic_s
          "frac": round(ach / peak, 4), "traffic": traffic,
          "measured_peak": round(meas, 1) if meas else None,
          "frac_of_measured": round(ach / meas, 4) if meas else None,
-         **({} if kind == "hbm" else {
+         **({} if kind != "mfma" else {
              "measured_peak_random": round(mr, 1) if mr else None,
              "frac_of_measured_random": round(ach / mr, 4) if mr else None}),
          "kernel": kernel, "launches": launches, "avg_ms": round(avg_s * 1e3, 4),
@@ -242,13 +247,13 @@ def search_setup(vs, NN, workload, args):
         storage = "auto"
         desc = f"c2: exact L2 top-{k}, {n} x {d} fp32 integers 0..255, {nq} queries"
     elif workload == "c2f":
-        # configs[1]'s shape on general fp32 values (not exact in bf16): the rows stay fp32
-        # and the scan multiplies their split-bf16 planes, three MFMA passes per product
+        # the C2 shape on general fp32 values (not exact in bf16): the rows stay fp32 and
+        # the scan multiplies their bf16 copy, one MFMA pass per product
         n, d, nq, k, metric = args.n or 1_000_000, 128, args.nq or 10_000, args.k or 100, 0
         xb, xq = syn.normal_unit(n, d, args.seed, 0), syn.normal_unit(nq, d, args.seed, 1)
         storage = "auto"
         desc = (f"c2 shape on fp32 data: exact L2 top-{k}, {n} x {d} fp32 unit N(0,1), "
-                f"{nq} queries (split-bf16 planes, three MFMA passes)")
+                f"{nq} queries (one MFMA pass over the rows' bf16 copy)")
     else:
         n, d, nq, k, metric = args.n or 10_000, 384, args.nq or 100, args.k or 10, 1
         xb, xq = syn.normal_unit(n, d, args.seed, 0), syn.normal_unit(nq, d, args.seed, 1)
@@ -286,7 +291,10 @@ def run_search(vs, NN, workload, args, ctx, full=False):
     Ibuf.download(I)
     bf16 = idx.storage == "bf16"
     traffic, tsrc = MEASURED_TRAFFIC.get((workload, n, nq, k), (None, None))
-    roof = roofline("mfma", 2.0 * nq * n * d, scan_s, ctx["peaks"], "scan", nscan, traffic, tsrc,
+    # (a direct search's scores are fp64 sums on the vector units)
+    direct = idx.prof_get("direct")[0] > 0
+    roof = roofline("fp64" if direct else "mfma", 2.0 * nq * n * d, scan_s, ctx["peaks"],
+                    "exact keys" if direct else "scan", nscan, traffic, tsrc,
                     extra={"scan_kinds": {f: idx.prof_get(f)[0] for f in
                                           ("shared", "gemm", "streamed", "direct")
                                           if idx.prof_get(f)[0]},
@@ -479,7 +487,7 @@ def run_c3(vs, NN, args, ctx, batches):
 # C4: k-means step
 # --------------------------------------------------------------------------
 def run_kmeans(vs, NN, args, ctx):
-    """one Lloyd iteration (assign + update) per step over 2M x 256
+    """C4: one Lloyd iteration (assign + update) per step over 2M x 256
     fp32 points from a 1,024-component mixture, 4,096 centroids from a seeded
     subset; the centroids of step i feed step i + 1 (kmeans.dart:91-140)."""
     import oracle
@@ -659,7 +667,7 @@ def join_full_parity(x, pi, pj, ps, thr, planted):
 
 
 def run_join(vs, NN, args, ctx):
-    """near-duplicate cosine self-join of 500k x 512 fp32 unit
+    """C5: near-duplicate cosine self-join of 500k x 512 fp32 unit
     vectors (5% planted copies), all pairs i < j with dot >= 0.95 sorted by
     (i, j) (vector_dedup_demo.dart:115-128).  One step = one self-join."""
     import oracle
@@ -759,7 +767,7 @@ def run_copy_calibration(args):
 
 def run_library_gemm(args):
     """For scale only (not the product path): the vendor library's bf16 GEMM
-    through torch (hipBLASLt on ROCm) on the K = 768 shapes of configs[2] at
+    through torch (hipBLASLt on ROCm) on the K = 768 shapes of C3 at
     batch 1024 and 8192, output written in bf16, no selection."""
     import torch
 

@@ -809,7 +809,7 @@ __global__ __launch_bounds__(64 * WR * WQ) void gemm_scan_kernel(ScanKArgs a) {
 
 // ---------------------------------------------------------------------------
 // Four-wave pipelined GEMM-tiled scan (option gemm4): bf16 rows, one query
-// plane (configs[2] at large batches; the self-join's bf16 copy of the rows).
+// plane (C3, 20M x 768, at large batches; the self-join's bf16 copy of the rows).
 //
 // 256 rows x 256 queries per tile.  Wave (wr, wq) multiplies rows
 // wr*128 .. +128 by queries wq*128 .. +128 with sixteen 32 x 32 accumulator

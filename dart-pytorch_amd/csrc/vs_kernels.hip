@@ -2581,6 +2581,9 @@ hipError_t launch_kmeans_bound(const float *cmax, double pmax, double r, double 
     return hipGetLastError();
 }
 
+// Exclusive prefix sums of 32-bit counts (the first point of every cluster in
+// the grouped order, the first key of every query): one workgroup walks the
+// counts in tiles of 1024, carrying the running total.
 __global__ __launch_bounds__(1024) void exclusive_scan_i32_kernel(const int32_t *in, int64_t n,
                                                                   int32_t *out) {
     __shared__ int32_t part[1024];

@@ -1,4 +1,4 @@
-"""Seeded synthetic inputs for the benchmark configurations (BASELINE.json configs).
+"""Seeded synthetic inputs for the benchmark configurations.
 
 Host generation uses numpy's Philox bit generator; one host buffer is fed to
 both the GPU library and the CPU checker in the same run, so the two sides

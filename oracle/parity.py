@@ -5,8 +5,8 @@ TEST INFRASTRUCTURE ONLY (used by tests/ and by bench.py's parity fields).
 Distances: the GPU re-ranks its survivors with the reference's exact fp64
 arithmetic, so a neighbour present on both sides must carry a bit-identical
 fp32 distance.  Ids: identical except inside tie groups -- neighbours whose
-oracle distances lie within `rtol` (+ `atol`) of each other (BASELINE
-north_star: rel 1e-5 for fp32 data, 1e-3 for bf16 data fed identically to
+oracle distances lie within `rtol` (+ `atol`) of each other (the bar:
+rel 1e-5 for fp32 data, 1e-3 for bf16 data fed identically to
 both sides).
 """
 import numpy as np

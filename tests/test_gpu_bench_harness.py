@@ -39,7 +39,7 @@ def _rows(vs, metric, storage, xb, xq, k):
 
 @pytest.mark.parametrize("metric,storage", [(0, "f32"), (1, "bf16"), (0, "auto")])
 def test_bench_faiss_flat_rows(vs, metric, storage):
-    if storage == "auto":  # configs[1] arithmetic: integers 0..255, kept losslessly as bf16
+    if storage == "auto":  # C2 arithmetic: integers 0..255, kept losslessly as bf16
         xb, xq = syn.int_grid(20_000, 128, 7, 0), syn.int_grid(48, 128, 7, 1)
     else:
         xb, xq = syn.normal_unit(20_000, 96, 7, 0), syn.normal_unit(48, 96, 7, 1)

@@ -100,7 +100,7 @@ def test_gemm_shape_parity(vs, opts, shape, metric, k, d):
 @pytest.mark.parametrize("kc", [64, 32])
 @pytest.mark.parametrize("wq,qb", [(4, 2), (2, 2)])
 def test_gemm_config2_exact(vs, opts, wq, qb, kc):
-    """configs[1] arithmetic on a 100k slice with 1,000 queries: integer
+    """C2 arithmetic on a 100k slice with 1,000 queries: integer
     distances, bit-exact, k = 100, with K-chunks of 64 and 32."""
     opts(gemm_wq=wq, gemm_qb=qb, gemm_kc=kc)
     xb = syn.int_grid(100_000, 128, 1234, 0)
@@ -287,7 +287,7 @@ def _one_pass_runs(g):
 
 @pytest.mark.parametrize("coarse", [1, 0])
 def test_coarse_self_join(vs, opts, coarse):
-    """configs[4] shape at 4,000 rows (d = 512, 5% planted copies, cos >=
+    """C5 shape at 4,000 rows (d = 512, 5% planted copies, cos >=
     0.95): the one-pass selection (bf16 hi planes, widened margins, exact
     fp64 re-test) and the three-pass one give the oracle's pair list."""
     opts(gemm=-1, coarse=coarse)  # the default planner rule
@@ -307,7 +307,7 @@ def test_coarse_self_join(vs, opts, coarse):
 
 @pytest.mark.parametrize("coarse", [1, 0])
 def test_coarse_kmeans(vs, opts, coarse):
-    """configs[3] arithmetic at 30,000 points (d = 256, 1,024 mixture
+    """C4 arithmetic at 30,000 points (d = 256, 1,024 mixture
     components, 4,096 centroids): assignments, objective and centroids equal
     the oracle's with and without the one-pass selection."""
     opts(gemm=-1, coarse=coarse)

@@ -72,7 +72,7 @@ def test_range_empty_and_bf16(vs):
 
 @pytest.mark.parametrize("copy16,gemm4", [(1, 0), (0, 0), (1, 1)])
 def test_self_join_dedup(vs, opts, copy16, gemm4):
-    """configs[4] arithmetic on 30k x 512: 5 % planted near-duplicates,
+    """C5 arithmetic on 30k x 512: 5 % planted near-duplicates,
     pairs i<j with cos >= 0.95, sorted by (i, j).  The one-pass selection
     reads a bf16 copy of the fp32 rows (copy16 1, the default) or rounds
     the fp32 rows in the kernel (0); on the copy, the eight-wave or the

@@ -61,7 +61,7 @@ def test_gpu_threshold_size(vs, metric):
 
 
 def test_config1_full(vs):
-    """10k x 384 unit N(0,1) IP, 100 queries, k=10."""
+    """C1: 10k x 384 unit N(0,1) IP, 100 queries, k=10."""
     xb = syn.normal_unit(10_000, 384, 1234, 0)
     xq = syn.normal_unit(100, 384, 1234, 1)
     D, I = run(vs, xb, xq, 10, 1)
@@ -71,7 +71,7 @@ def test_config1_full(vs):
 
 @pytest.mark.parametrize("nq", [1, 64, 200])
 def test_config2_slice_exact(vs, nq):
-    """configs[1] shape on a 100k-row slice: integers 0..255, L2, k=100.
+    """C2 shape on a 100k-row slice: integers 0..255, L2, k=100.
     Integer sums stay below 2^24, so distances are exact integers and equal
     bit for bit; ids are compared per tie group (ties are frequent)."""
     xb = syn.int_grid(100_000, 128, 1234, 0)
@@ -87,7 +87,7 @@ def test_config2_slice_exact(vs, nq):
 
 @pytest.mark.parametrize("nq", [1, 7, 64, 300])
 def test_bf16_storage_ip(vs, nq):
-    """configs[2] arithmetic on a 60k x 768 slice: bf16 unit vectors, IP, k=10;
+    """C3 arithmetic on a 60k x 768 slice: bf16 unit vectors, IP, k=10;
     the oracle is fed the same bf16 values upcast to fp32."""
     xb16 = syn.to_bf16_bits(syn.normal_unit(60_000, 768, 99, 0))
     xq16 = syn.to_bf16_bits(syn.normal_unit(nq, 768, 99, 1))

@@ -67,7 +67,7 @@ def test_bf16_unit_vectors(vs, metric):
 
 
 def test_matches_streaming_scan_large(vs, opts):
-    """configs[1] shape on a 300k-row slice (estimated thresholds active):
+    """C2 shape on a 300k-row slice (estimated thresholds active):
     the row-shared scan returns the same distances as the streaming scan,
     and the oracle's on a query sample."""
     xb = syn.int_grid(300_000, 128, 4, 0)

@@ -52,7 +52,7 @@ def _check(idx, q, k, metric, dtype, xb32, q32, rtol):
 
 
 def test_noalloc_matches_search_device_bf16_ip():
-    """bf16 unit rows (configs[2] arithmetic), 300k x 768, IP: batch 64 with
+    """bf16 unit rows (C3 arithmetic), 300k x 768, IP: batch 64 with
     k = 100 (threshold seeding runs), then batch 7 with k = 10."""
     xb16 = syn.to_bf16_bits(syn.normal_unit(300_000, 768, 31, 0))
     xq16 = syn.to_bf16_bits(syn.normal_unit(64, 768, 31, 1))
