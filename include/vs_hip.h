@@ -58,7 +58,8 @@ enum { VS_DTYPE_F32 = 0, VS_DTYPE_BF16 = 1 };
  *   F32  -- fp32, as IndexFlat's Float32List storage (index_flat.dart:20);
  *           searches and joins also keep a bf16 copy of the rows to select
  *           candidates from, where it takes at most a quarter of the free
- *           device memory (given back when an allocation needs it);
+ *           device memory (given back when an allocation of this library
+ *           needs it);
  *   BF16 -- bf16; fp32 input rows are rounded to nearest-even once at add;
  *   AUTO -- bf16 while every stored value is exactly a bf16 value (then
  *           results are those of fp32 storage), fp32 otherwise; the switch
@@ -167,8 +168,10 @@ VS_API int vs_index_search_device_noalloc(vs_index *idx, const void *q_dev, int 
  * the fine scan of IndexIVFFlat.search over its probed inverted lists
  * (index_ivf_flat.dart:131-170): fp64 scores in dimension order, the k best
  * by (fp32 score, id), sentinels when fewer rows were scanned.  Host
- * buffers; any k (beyond 409 each query's subset rows are sorted on the
- * device).  An id outside [0, ntotal) gives VS_ERR_INVALID. */
+ * buffers; any k (beyond 8,192 each query's subset rows are sorted on the
+ * device, up to that their keys are selected, of fewer than 2^31 rows a
+ * query: VS_ERR_UNSUPPORTED beyond).  An id outside [0, ntotal) gives
+ * VS_ERR_INVALID. */
 VS_API int vs_index_search_subsets(vs_index *idx, const void *q, int q_dtype, int64_t nq,
                                    int64_t k, const int32_t *ids, int64_t nids,
                                    const int64_t *seg_off, const int64_t *seg_len, int64_t nseg,
