@@ -82,6 +82,11 @@ hipError_t launch_store_rows(const void *src, int src_dtype, int64_t src_stride,
 hipError_t launch_copy_rows16(const void *src, int64_t ld, int64_t n, int64_t ld16, void *dst,
                               float *res, hipStream_t st);
 
+// Rows 0, step, 2 step, ... (modulo n; m of them) of src and their norms xn,
+// one after another in dst and dxn.
+hipError_t launch_sample_rows(const void *src, int64_t row_bytes, int64_t n, int64_t step,
+                              const float *xn, int64_t m, void *dst, float *dxn, hipStream_t st);
+
 // Build PreparedQueries from n query rows (src dtype / stride).
 hipError_t launch_prepare_queries(const void *src, int src_dtype, int64_t src_stride, int64_t nq,
                                   int64_t d, int64_t ld, int metric, const PreparedQueries &pq,

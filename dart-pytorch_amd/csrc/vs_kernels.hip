@@ -154,6 +154,33 @@ hipError_t launch_copy_rows16(const void *src, int64_t ld, int64_t n, int64_t ld
 }
 
 // ---------------------------------------------------------------------------
+// Rows 0, step, 2 step, ... (modulo n) of src, and their norms, one after
+// another: a thread per 16 bytes.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void sample_rows_kernel(const u32x4_t *__restrict__ src, uint32_t w,
+                                                          int64_t n, int64_t step,
+                                                          const float *__restrict__ xn, uint32_t m,
+                                                          u32x4_t *__restrict__ dst,
+                                                          float *__restrict__ dxn) {
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (t >= m * w) return;
+    const uint32_t r = t / w, c = t - r * w;
+    const int64_t row = (int64_t)r * step % n;
+    dst[t] = src[row * w + c];
+    if (c == 0) dxn[r] = xn[row];
+}
+
+hipError_t launch_sample_rows(const void *src, int64_t row_bytes, int64_t n, int64_t step,
+                              const float *xn, int64_t m, void *dst, float *dxn, hipStream_t st) {
+    const int64_t w = row_bytes / 16;
+    if (m <= 0) return hipSuccess;
+    if (n <= 0 || step <= 0 || row_bytes % 16 || m * w > INT32_MAX) return hipErrorInvalidValue;
+    sample_rows_kernel<<<dim3((unsigned)((m * w + 255) / 256)), dim3(256), 0, st>>>(
+        (const u32x4_t *)src, (uint32_t)w, n, step, xn, (uint32_t)m, (u32x4_t *)dst, dxn);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // Query preparation.  One wave per (padded) query row.
 // ---------------------------------------------------------------------------
 template <typename TS>

@@ -208,3 +208,29 @@ def test_range_hit_buffers(vs, nq, radius):
         lims, D, I = oracle.flat_range_search(rows, xq, radius, 0, NT)
         assert np.array_equal(rr.limits, lims) and np.array_equal(rr.ids, I)
         assert np.array_equal(rr.distances, D)
+
+
+# streaming, row-shared and GEMM-tiled scans, the smallest sample and larger ones
+@pytest.mark.parametrize("n,d,nq,k", [(20_000, 384, 600, 10), (17_000, 768, 100, 10), (40_000, 64, 32, 10),
+                                      (30_000, 128, 300, 30), (60_000, 256, 520, 100)])
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+def test_estimates_on_sorted_rows(vs, n, d, nq, k, storage):
+    """Rows grouped by topic, and queries about the first topics: the sample
+    behind the thresholds is spread over the rows, so no query is misled by it
+    and searched again with full lists."""
+    g = syn.rng(n, 4)
+    cen = g.standard_normal((n // 50, d)).astype(np.float32)
+    xb = (np.repeat(cen, 50, axis=0)[:n] + np.float32(0.3) * g.standard_normal((n, d))).astype(np.float32)
+    xq = (xb[:nq] + np.float32(0.01) * g.standard_normal((nq, d))).astype(np.float32)
+    if storage == "bf16":
+        xb, xq = (syn.bf16_bits_to_f32(syn.to_bf16_bits(a)) for a in (xb, xq))
+    idx = vs.GpuIndexFlat.l2(d, storage=storage)
+    idx.set_option("direct", 0)
+    idx.add(xb)
+    for _ in range(2):
+        idx.prof_reset()
+        r = idx.search(xq, k)
+        assert idx.prof_get("guess_scans")[0] == 1 and idx.prof_get("fallback")[0] <= nq // 50
+    idx.close()
+    Dr, Ir = oracle.flat_search(xb, xq[::9], k, 0, NT)
+    assert_knn_parity(r.distances[::9], r.ids[::9], Dr, Ir, 0, rtol=0.0, atol=0.0)
