@@ -3027,7 +3027,7 @@ int vs_kmeans_step(vs_index *x, const float *centroids_in, int64_t K, int64_t mi
         VS_HIP(hipStreamCreateWithFlags(&x->st_copy, hipStreamNonBlocking), "copy stream");
     // The objective is a sequential fp64 sum over the points in index order
     // (kmeans.dart:104): a chain of n dependent adds on the host.  Over the
-    // row-shared scan's lists the pick runs in kSumChunks launches over
+    // row-shared scan's lists of many points the pick runs in kSumChunks launches over
     // consecutive point ranges (each range's points in the previous step's
     // grouped order), and each range's distances and assignments come over
     // with the fallback count so far as soon as its pick ends: the sum of a
@@ -3049,7 +3049,13 @@ int vs_kmeans_step(vs_index *x, const float *centroids_in, int64_t K, int64_t mi
         hipStream_t s;
         ~CopyDrain() { (void)hipStreamSynchronize(s); }
     } drain{x->st_copy};
-    const bool chunked = plan.kind == 3 && plan.share_kmin;
+    // Ranges that leave CUs idle cost more than they hide (a wave takes 64
+    // points, and what bounds a pick is one wave's chain of candidates):
+    // 50,000 points x 768, K = 256: 1.73 ms a step in four ranges, 1.03 in
+    // one; 100,000 x 256, K = 512: 0.92 and 0.57; 250,000 x 256, K = 256: 1.45
+    // and 1.48.
+    const bool chunked = plan.kind == 3 && plan.share_kmin &&
+                         n >= (int64_t)kSumChunks * 64 * 2 * std::max(1, x->num_cu);
     const int32_t *order = x->km_order_version == x->version && x->km_order_n == n &&
                                    x->opt.pick_order
                                ? x->km_order.as<int32_t>()

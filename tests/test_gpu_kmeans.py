@@ -258,3 +258,26 @@ def test_empty_clusters_without_a_minimum(vs, min_points):
     cr, cntr, _ = oracle.kmeans_update(x, ar, cen, min_points)
     assert np.array_equal(a, ar) and obj == objr and np.array_equal(cnt, cntr)
     assert np.all(np.isnan(cr[5:])) and np.array_equal(newc, cr, equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [131_071, 131_072, 150_001])
+@pytest.mark.parametrize("copies", [False, True])
+def test_pick_ranges(vs, n, copies):
+    """The pick in one launch below 131,072 points and in four ranges from
+    there on, in index order and by the last step's clusters, with every point
+    or none left to the exhaustive pass."""
+    x, _ = syn.gaussian_mixture(n, 20, 9, 0.05, 7)
+    cen = x[syn.seeded_subset(n, 40, 5)].copy()
+    if copies:
+        cen[:] = cen[0]
+    pts = vs.GpuIndexFlat.l2(20, storage="f32")
+    pts.add(x)
+    u = syn.rng(6, 0).random(40 * 20)
+    for _ in range(2):
+        a, newc, cnt, obj = vs.kmeans_step(pts, cen, 1, u)
+        ar, _, objr = oracle.kmeans_assign(x, cen, oracle.default_threads())
+        cr, cntr, _ = oracle.kmeans_update(x, ar, cen, 1, u)
+        assert np.array_equal(a, ar) and obj == objr and np.array_equal(cnt, cntr)
+        assert np.array_equal(newc.view(np.uint32), cr.view(np.uint32))
+        cen = newc
+    pts.close()
