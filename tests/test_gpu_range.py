@@ -110,3 +110,39 @@ def test_range_l2_one_pass_rows(vs, opts, copy16):
     lims, D, I = oracle.flat_range_search(xb, xq, radius, 0, NT)
     assert rr.total_matches > 0
     assert_range_parity(rr.limits, rr.distances, rr.ids, lims, D, I)
+
+
+# 512 candidates and fewer are sorted on the host, more on the device
+@pytest.mark.parametrize("nq,each", [(1, 1), (3, 0), (1, 511), (64, 8), (57, 9), (5, 300)])
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+def test_few_hits(vs, nq, each, storage):
+    g = syn.rng(nq, each)
+    xq = syn.normal_unit(nq, 64, 5, 1)
+    near = np.repeat(xq, each, axis=0) + 0.002 * g.standard_normal((nq * each, 64))
+    xb = np.concatenate([near, syn.normal_unit(3000, 64, 5, 0)]).astype(np.float32)
+    xb = xb[g.permutation(len(xb))]
+    if storage == "bf16":
+        xb, xq = (syn.bf16_bits_to_f32(syn.to_bf16_bits(a)) for a in (xb, xq))
+    idx = vs.GpuIndexFlat(64, vs.Metric(0), storage=storage)
+    idx.add(xb)
+    lims, D, I = oracle.flat_range_search(xb, xq, 0.02, 0, NT)
+    assert lims[-1] == nq * each
+    for _ in range(2):
+        rr = idx.range_search(xq, 0.02)
+        assert_range_parity(rr.limits, rr.distances, rr.ids, lims, D, I)
+    idx.close()
+
+
+@pytest.mark.parametrize("pairs", [1, 511, 512, 513, 900])
+def test_few_pairs(vs, pairs):
+    g = syn.rng(pairs, 1)
+    x = syn.normal_unit(4000 - pairs, 64, 6, 0)
+    xb = np.concatenate([x, x[:pairs] + 0.002 * g.standard_normal((pairs, 64))]).astype(np.float32)
+    xb = xb[g.permutation(4000)]
+    idx = vs.GpuIndexFlat.ip(64, storage="f32")
+    idx.add(xb)
+    i, j, s = idx.self_join(0.95)
+    idx.close()
+    io, jo, so = oracle.self_join(xb, 0.95, nthreads=NT)
+    assert len(io) == pairs
+    assert np.array_equal(i, io) and np.array_equal(j, jo) and np.array_equal(s, so)
