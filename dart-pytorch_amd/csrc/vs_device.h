@@ -273,30 +273,32 @@ __device__ __forceinline__ void sink_pairs(const ScanKArgs &a, int c, int *fill,
         flush_pairs(a, fill, bq, bi, lane);
         f = 0;
     }
-    int *dq = bq + f, *di = bi + f;
-    long long room = cap;
-    const bool direct = total > cap;
-    if (direct) {
+    int pos = inc - c;
+    // (two loops: one pointer to either memory would make them flat stores,
+    // after which every wait for the main loop's loads is one for all of
+    // them -- 200 queries of 100,000 x 768 fp32 rows, in two planes: 381 us
+    // instead of 292)
+    if (total > cap) {
         unsigned long long base = 0;
         if (lane == 0) base = atomicAdd(a.count, (unsigned long long)total);
         base = __shfl(base, 0);
-        dq = a.out_q + base;
-        di = a.out_i + base;
-        room = (long long)a.out_cap - (long long)base;
+        emit([&](int q, int row) {
+            const unsigned long long at = base + (unsigned)pos++;
+            if (at < (unsigned long long)a.out_cap) {
+                a.out_q[at] = q;
+                a.out_i[at] = row;
+            }
+        });
+        return;
     }
-    int pos = inc - c;
+    pos += f;
     emit([&](int q, int row) {
-        if (pos < room) {
-            dq[pos] = q;
-            di[pos] = row;
-        }
-        ++pos;
+        bq[pos] = q;
+        bi[pos++] = row;
     });
-    if (!direct) {
-        lds_wave_sync();
-        if (lane == 0) *fill = f + total;
-        lds_wave_sync();
-    }
+    lds_wave_sync();
+    if (lane == 0) *fill = f + total;
+    lds_wave_sync();
 }
 
 // Word 3 of a raw buffer resource (gfx9: 32-bit data format, no swizzle).
