@@ -470,10 +470,47 @@ struct NarrowRows {
     }
 };
 
-// Switch bf16 storage to fp32 (AUTO storage meeting a non-bf16 value).
-int widen_storage(vs_index *x, NarrowRows *old) {
+int clear_rows(vs_index *x, int64_t end);
+
+// Storage for no more than the rows there are (those past them, up to `end`,
+// belong to an add that starts over), or, without the memory to move them,
+// zeros past them: a widening add then has its rows in memory once.
+int trim_storage(vs_index *x, int64_t end) {
+    const int64_t nc = round_up(x->ntotal, kRowCapAlign), rb = row_bytes(x);
+    if (nc >= x->cap) return clear_rows(x, end);
+    void *nxb = nullptr;
+    float *nxn = nullptr;
+    if (x->ntotal > 0) {
+        const size_t xbytes = (size_t)(nc + kRowSlack) * rb, nbytes = (size_t)(nc + kRowSlack) * 4;
+        if (dev_malloc(&nxb, xbytes) != hipSuccess || dev_malloc((void **)&nxn, nbytes) != hipSuccess) {
+            (void)hipGetLastError();
+            if (nxb) (void)hipFree(nxb);
+            return clear_rows(x, end);
+        }
+        VS_HIP(hipMemcpyAsync(nxb, x->xb, (size_t)x->ntotal * rb, hipMemcpyDeviceToDevice, x->st),
+               "copying storage");
+        VS_HIP(hipMemcpyAsync(nxn, x->xn, (size_t)x->ntotal * 4, hipMemcpyDeviceToDevice, x->st),
+               "copying norms");
+        VS_HIP(hipMemsetAsync((char *)nxb + (size_t)x->ntotal * rb, 0,
+                              xbytes - (size_t)x->ntotal * rb, x->st),
+               "clearing storage");
+        VS_HIP(hipMemsetAsync(nxn + x->ntotal, 0, nbytes - (size_t)x->ntotal * 4, x->st),
+               "clearing norms");
+        VS_HIP(hipStreamSynchronize(x->st), "trimming storage");
+    }
+    if (x->xb) (void)hipFree(x->xb);
+    if (x->xn) (void)hipFree(x->xn);
+    x->xb = nxb;
+    x->xn = nxn;
+    x->cap = x->ntotal > 0 ? nc : 0;
+    return VS_OK;
+}
+
+// Switch bf16 storage to fp32, with room for `need` rows (AUTO storage meeting
+// a non-bf16 value).
+int widen_storage(vs_index *x, int64_t need, NarrowRows *old) {
     const int64_t new_ld = vs::storage_ld(x->d, 0);
-    const int64_t nc = std::max<int64_t>(x->cap, 1024);
+    const int64_t nc = std::max<int64_t>(need, 1024);
     void *nxb = nullptr;
     float *nxn = nullptr;
     const size_t xbytes = (size_t)(nc + kRowSlack) * new_ld * 4;
@@ -557,8 +594,9 @@ int add_rows(vs_index *x, int dtype, int64_t n, int64_t chunk, Fetch &&fetch) {
         }
         if (x->mode == VS_STORAGE_AUTO && x->storage == 1 && (f & vs::kFlagNotBf16)) {
             // fp32 from here on: the rows so far are stored again
-            rc = clear_rows(x, x->ntotal + r + m);
-            if (!rc) rc = widen_storage(x, &narrow);
+            const int64_t cap = x->cap;
+            rc = trim_storage(x, x->ntotal + r + m);
+            if (!rc) rc = widen_storage(x, cap, &narrow);
             if (rc) return rc;
             widened = true;
             r = 0;

@@ -350,3 +350,46 @@ def test_range_gives_its_sort_space_back(vs):
     idx.close()
     assert rr.limits[-1] == 20_000_000
     assert kept <= 400e6, f"{kept / 1e6:.0f} MB kept"
+
+
+@pytest.mark.parametrize("first", [0, 3000])
+def test_widening_add_holds_its_rows_once(vs, first):
+    """An add that widens automatic storage needs room for its rows in fp32, not
+    beside their bf16 storage as well: 805 MB and the 268 MB of staging."""
+    import ctypes
+    import threading
+
+    lib = vs.load()
+    f, t = ctypes.c_size_t(0), ctypes.c_size_t(0)
+
+    def free():
+        assert lib.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    d, n = 4096, 49_152
+    xb = np.zeros((n, d), np.float32)
+    xb[0, 0] = xb[-1, -1] = 0.3
+    head = syn.int_grid(first, d, 3, 0) if first else None
+    idx = vs.GpuIndexFlat.l2(d)
+    if first:
+        idx.add(head)
+    idx.reconstruct_n(0, first)
+    before, low, done = free(), [1 << 60], threading.Event()
+
+    def poll():
+        while not done.wait(0.001):
+            low[0] = min(low[0], free())
+
+    th = threading.Thread(target=poll)
+    th.start()
+    idx.add(xb)
+    done.set()
+    th.join()
+    used = before - low[0]
+    assert idx.storage == "f32" and idx.ntotal == first + n
+    if first:
+        assert np.array_equal(idx.reconstruct_n(0, first), head)
+    assert np.array_equal(idx.reconstruct_n(first, 1)[0], xb[0])
+    assert np.array_equal(idx.reconstruct(first + n - 1), xb[-1])
+    idx.close()
+    assert used <= 1.25e9, f"{used / 1e6:.0f} MB at the most"
