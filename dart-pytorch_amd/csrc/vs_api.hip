@@ -474,10 +474,13 @@ int clear_rows(vs_index *x, int64_t end);
 
 // Storage for no more than the rows there are (those past them, up to `end`,
 // belong to an add that starts over), or, without the memory to move them,
-// zeros past them: a widening add then has its rows in memory once.
+// zeros past them: a widening add then has its rows in memory once.  Less than
+// kTrimBytes is not worth it: freeing before the fp32 storage is allocated
+// took an add of 10,000 x 384 rows from 195 us to 735.
+constexpr int64_t kTrimBytes = 256ll << 20;
 int trim_storage(vs_index *x, int64_t end) {
     const int64_t nc = round_up(x->ntotal, kRowCapAlign), rb = row_bytes(x);
-    if (nc >= x->cap) return clear_rows(x, end);
+    if ((x->cap - nc) * rb < kTrimBytes) return clear_rows(x, end);
     void *nxb = nullptr;
     float *nxn = nullptr;
     if (x->ntotal > 0) {
